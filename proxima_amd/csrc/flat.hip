@@ -19,7 +19,10 @@
 //                         flat_seed_threshold (from all of them) turns those
 //                         keys into each query's starting threshold, and the
 //                         full pass filters them instead of recomputing
-//                         that tile.
+//                         that tile. From 64 dimensions on the products
+//                         come from the f16 matrix cores instead
+//                         (flat_split_candidates, flat_split.hpp), with the
+//                         same tiles, buffers, thresholds and merge.
 //  3. flat_merge_rescore  per query: radix-select the k' best approximate
 //                         keys over all splits, rescore those k' exactly with
 //                         the reference's 8-lane arithmetic, sort by
@@ -545,6 +548,8 @@ __global__ __launch_bounds__(256, 2) void flat_mfma_candidates(
   }
 }
 
+#include "flat_split.hpp"
+
 // ---------------------------------------------------------------------------
 // 3. merge + exact rescore (approximate candidates)
 // ---------------------------------------------------------------------------
@@ -615,10 +620,11 @@ constexpr int MERGE_MAXP = 512;
 // The certificate of one query's merge. Every candidate outside the
 // selection has approx >= approx(pivot), hence exact >= approx(pivot) - eps;
 // the k-th exact distance (the high word of `kth`) must be strictly below
-// that for the selection to contain the exact top-k.
+// that for the selection to contain the exact top-k. q_add: the query's own
+// term where the candidates' scores leave it out, else 0.
 __device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric, float qnv, float maxnorm, float eps_c,
-                                       int dim) {
-  const float ak = key_float((uint32_t)(pivot >> 32));
+                                       int dim, float q_add) {
+  const float ak = key_float((uint32_t)(pivot >> 32)) + q_add;
   const float dk = key_float((uint32_t)(kth >> 32));
   float eps;
   if (metric == 0) {
@@ -634,8 +640,8 @@ __device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric,
 __global__ __launch_bounds__(256) void flat_merge_rescore(
     const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const float* __restrict__ Qp, int ld, int dim,
     int metric, const float* __restrict__ X, const uint32_t* __restrict__ rank, const uint32_t* __restrict__ rank_slot,
-    const uint64_t* __restrict__ ids, const float* __restrict__ qn, float maxnorm, float eps_c,
-    uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
+    const uint64_t* __restrict__ ids, const float* __restrict__ qn, const float* __restrict__ q_add, float maxnorm,
+    float eps_c, uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
     int* __restrict__ flag_list, int* __restrict__ flag_count, size_t ldo) {
   const int q = blockIdx.x;
   __shared__ int hist[256];
@@ -707,7 +713,8 @@ __global__ __launch_bounds__(256) void flat_merge_rescore(
   }
   if (threadIdx.x == 0) {
     out_count[q] = kout;
-    if (valid >= Kp && !merge_certified(pivot, sel[kout - 1], metric, qn[q], maxnorm, eps_c, dim)) {
+    if (valid >= Kp && !merge_certified(pivot, sel[kout - 1], metric, qn[q], maxnorm, eps_c, dim,
+                                         q_add != nullptr ? q_add[q] : 0.0f)) {
       const int p = atomicAdd(flag_count, 1);
       flag_list[p] = q;
     }
@@ -724,9 +731,9 @@ template <int NT, int PER>
 __global__ __launch_bounds__(NT) void flat_merge_rescore_reg(
     const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const float* __restrict__ Qp, int ld, int dim,
     int metric, const float* __restrict__ X, const uint32_t* __restrict__ rank, const uint64_t* __restrict__ ids,
-    const float* __restrict__ qn, float maxnorm, float eps_c, uint64_t* __restrict__ out_ids,
-    float* __restrict__ out_d, uint32_t* __restrict__ out_count, int* __restrict__ flag_list,
-    int* __restrict__ flag_count, size_t ldo) {
+    const float* __restrict__ qn, const float* __restrict__ q_add, float maxnorm, float eps_c,
+    uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
+    int* __restrict__ flag_list, int* __restrict__ flag_count, size_t ldo) {
   const int q = blockIdx.x;
   const int lane = threadIdx.x & (WAVE - 1);
   __shared__ int hist[256];
@@ -802,7 +809,8 @@ __global__ __launch_bounds__(NT) void flat_merge_rescore_reg(
   const uint32_t kth_hi = (uint32_t)__shfl((int)(uint32_t)(key >> 32), kout - 1, WAVE);
   if (lane == 0) {
     out_count[q] = kout;
-    if (valid >= Kp && !merge_certified(pivot, (uint64_t)kth_hi << 32, metric, qn[q], maxnorm, eps_c, dim)) {
+    if (valid >= Kp && !merge_certified(pivot, (uint64_t)kth_hi << 32, metric, qn[q], maxnorm, eps_c, dim,
+                                         q_add != nullptr ? q_add[q] : 0.0f)) {
       const int p = atomicAdd(flag_count, 1);
       flag_list[p] = q;
     }
@@ -839,7 +847,12 @@ void FlatIndex::ensure_capacity(size_t need, size_t keep) {
   size_t nc = std::max<size_t>(need, std::max<size_t>(cap * 2, 1024));
   const size_t hw = std::min(keep, cap);
   X.grow(nc * ld, hw * ld, stream);
-  xb.grow(nc, hw, stream);
+  // row biases of whole tiles; +inf marks a slot that holds no row
+  const size_t nb = (nc + FB_N - 1) / FB_N * FB_N;
+  xb.grow(nb, hw, stream);
+  hipLaunchKernelGGL(fill_u32, dim3((unsigned)((nb - hw + 255) / 256)), dim3(256), 0, stream, (uint32_t*)xb.p + hw,
+                     nb - hw, 0x7F800000u);
+  PXG_HIP(hipGetLastError());
   d_live.grow(nc, hw, stream);
   d_ids.grow(nc, hw, stream);
   ranks.grow(nc, hw, stream);
@@ -920,6 +933,8 @@ void FlatIndex::remove(uint64_t id) {
   live[s] = 0;
   slots.release(s);
   PXG_HIP(hipMemsetAsync(d_live.p + s, 0, 1, stream));
+  hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, stream, (uint32_t*)xb.p + s, (size_t)1, 0x7F800000u);
+  PXG_HIP(hipGetLastError());
   ranks.remove(s, stream);
   PXG_HIP(hipStreamSynchronize(stream));
 }
@@ -961,9 +976,47 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   // per query, the least threshold any split has published (MFMA path),
   // cleared by the preparation kernel
   unsigned long long* gthr = (unsigned long long*)sc.get(25, nq * 8);
+  // Manhattan has no inner-product form and k beyond FAST_KMAX exceeds the
+  // candidate buffers: both take the exact scan, as do stores under 4096
+  // rows and batches the exact scan finishes sooner.
+  const bool exact_all = mode == 2 || metric == PXG_MANHATTAN || kq > FAST_KMAX ||
+                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq)));
+  const int Kp = (int)std::min<uint64_t>(kq + MARGIN, (uint64_t)FAST_KMAX + MARGIN);
+  // a row's buffer holds its Kp keys, one tile's appends (FB_N) and at
+  // least 64 more before it must be compacted
+  const int CAP = (Kp + FB_N + 64) <= 256 ? 256 : 512;
+  const size_t per_split_bytes = (size_t)nq * CAP * 8;
+  const float scale = metric == PXG_EUCLIDEAN ? 2.0f : 1.0f;
+  const int tiles = (int)((N + FB_N - 1) / FB_N);
+  // The split candidate pass: for widths it is at least as accurate on, norms
+  // its scales can hold, and scratch for its operands beside one split of
+  // candidates and the exact scan of one query (a fixed scratch that holds
+  // those only without them takes the f32 pass).
+  const int nKs = (int)((dim + FB_K - 1) / FB_K);
+  const size_t split_bytes = nq * nKs * 128 + nq * 4 + (d_accept ? (size_t)tiles * FB_N * 4 : 0) + 4096;
+  const size_t exact_bytes = (N / 256 + 1) * std::min<size_t>(kq, EXACT_CH) * 8 + 4096;
+  const bool split = !exact_all && kq > 0 && dim >= SPLIT_MIN_DIM && split_norm_ok(maxnorm) &&
+                     sc.room() >= split_bytes + std::max(per_split_bytes, exact_bytes);
   hipLaunchKernelGGL(init_search_flags, dim3(1), dim3(64), 0, s, bad, flag_count);
-  hipLaunchKernelGGL(flat_prep_search_queries, dim3((unsigned)nq), dim3(64), 0, s, d_raw, (int)dim, (int)ld, metric,
-                     do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr);
+  _Float16* Qs = nullptr;
+  float* cq = nullptr;
+  const float* xbias = xb.p;
+  const float sx = split ? split_scale(maxnorm) : 1.0f;
+  if (split) {
+    Qs = (_Float16*)sc.get(26, nq * nKs * 128);
+    cq = (float*)sc.get(27, nq * 4);
+    hipLaunchKernelGGL(flat_prep_split_queries, dim3((unsigned)nq), dim3(64), 0, s, d_raw, (int)dim, (int)ld, metric,
+                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr, Qs, nKs, scale, sx, cq);
+    if (d_accept) {
+      float* mb = (float*)sc.get(28, (size_t)tiles * FB_N * 4);
+      hipLaunchKernelGGL(flat_mask_bias, dim3((unsigned)((tiles * FB_N + 255) / 256)), dim3(256), 0, s, xb.p, d_accept,
+                         (int)N, tiles * FB_N, mb);
+      xbias = mb;
+    }
+  } else {
+    hipLaunchKernelGGL(flat_prep_search_queries, dim3((unsigned)nq), dim3(64), 0, s, d_raw, (int)dim, (int)ld, metric,
+                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr);
+  }
   PXG_HIP(hipGetLastError());
   unsigned long long* tail = sc.host_words();
   auto read_flags = [&](int* nflag) {
@@ -986,21 +1039,13 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   }
 
   int* flag_list = (int*)sc.get(5, nq * 4);
-  // Manhattan has no inner-product form and k beyond FAST_KMAX exceeds the
-  // candidate buffers: both take the exact scan, as do stores under 4096
-  // rows and batches the exact scan finishes sooner.
-  const bool exact_all = mode == 2 || metric == PXG_MANHATTAN || kq > FAST_KMAX ||
-                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq)));
   if (!exact_all) {
-    const int Kp = (int)std::min<uint64_t>(kq + MARGIN, (uint64_t)FAST_KMAX + MARGIN);
-    // a row's buffer holds its Kp keys, one tile's appends (FB_N) and at
-    // least 64 more before it must be compacted
-    const int CAP = (Kp + FB_N + 64) <= 256 ? 256 : 512;
-    const int QB = (int)((nq + FB_M - 1) / FB_M);
-    const int tiles = (int)((N + FB_N - 1) / FB_N);
+    // queries per workgroup: FB_M, or 32 or 64 for a smaller batch on the
+    // split pass
+    const int QT = !split || nq > 64 ? 4 : nq > 32 ? 2 : 1;
+    const int QB = (int)((nq + 32 * QT - 1) / (32 * QT));
     int S = std::max(1, std::min(512 / QB, std::max(1, tiles / 4)));
     // a fixed scratch may hold fewer splits (the results do not depend on S)
-    const size_t per_split_bytes = (size_t)nq * CAP * 8;
     const size_t fit = sc.room() / per_split_bytes;
     if (fit == 0) (void)sc.get(6, per_split_bytes);  // raises the capacity error
     S = (int)std::min<size_t>((size_t)S, fit);
@@ -1011,7 +1056,6 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     const int total = QB * S;
     tm.mark(1);
     const int grid = ((total + 7) / 8) * 8;
-    const float scale = metric == PXG_EUCLIDEAN ? 2.0f : 1.0f;
     // A first pass over the first tile of each split (spread over the whole
     // store) seeds each query's threshold with the Kp-th best of those rows,
     // so the full pass appends and compacts little from its first tile on
@@ -1022,12 +1066,22 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     const int seeded = (size_t)S * FB_N >= (size_t)Kp ? 1 : 0;
     auto candidates = [&](auto seed) {
       constexpr bool SD = decltype(seed)::value;
-      if (CAP == 256)
+#define PXG_SPLIT(CAPV, QTV)                                                                                       \
+  hipLaunchKernelGGL((flat_split_candidates<CAPV, QTV, SD>), dim3(grid), dim3(256), 0, s, Qs, (int)nq, nKs, X.p, (int)N, \
+                     (int)ld, cq, xbias, sx, S, QB, per_split, Kp, cand, gthr, seeded)
+      if (split) {
+        if (CAP == 256) {
+          if (QT == 4) PXG_SPLIT(256, 4); else if (QT == 2) PXG_SPLIT(256, 2); else PXG_SPLIT(256, 1);
+        } else {
+          if (QT == 4) PXG_SPLIT(512, 4); else if (QT == 2) PXG_SPLIT(512, 2); else PXG_SPLIT(512, 1);
+        }
+      } else if (CAP == 256)
         hipLaunchKernelGGL((flat_mfma_candidates<256, SD>), dim3(grid), dim3(256), 0, s, Qp, (int)nq, X.p, (int)N,
                            (int)ld, qb, xb.p, scale, d_live.p, d_accept, S, QB, per_split, Kp, cand, gthr, seeded);
       else
         hipLaunchKernelGGL((flat_mfma_candidates<512, SD>), dim3(grid), dim3(256), 0, s, Qp, (int)nq, X.p, (int)N,
                            (int)ld, qb, xb.p, scale, d_live.p, d_accept, S, QB, per_split, Kp, cand, gthr, seeded);
+#undef PXG_SPLIT
       PXG_HIP(hipGetLastError());
     };
     if (seeded) {
@@ -1048,17 +1102,19 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     candidates(std::false_type{});
     tm.mark(2);
     const size_t nkeys = (size_t)S * Kp;
+    const float* q_add = split ? qb : nullptr;
+    const float eps_c = split ? SPLIT_EPS_C : 4.0f;
     if (nkeys <= 8 * 256 && Kp <= WAVE)
       hipLaunchKernelGGL((flat_merge_rescore_reg<256, 8>), dim3((unsigned)nq), dim3(256), 0, s, cand, S, CAP, Kp,
-                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, maxnorm, 4.0f, d_oid,
+                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, q_add, maxnorm, eps_c, d_oid,
                          d_od, d_oc, flag_list, flag_count, ldo);
     else if (nkeys <= 16 * 1024 && Kp <= WAVE)
       hipLaunchKernelGGL((flat_merge_rescore_reg<1024, 16>), dim3((unsigned)nq), dim3(1024), 0, s, cand, S, CAP, Kp,
-                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, maxnorm, 4.0f, d_oid,
+                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, q_add, maxnorm, eps_c, d_oid,
                          d_od, d_oc, flag_list, flag_count, ldo);
     else
       hipLaunchKernelGGL(flat_merge_rescore, dim3((unsigned)nq), dim3(256), 0, s, cand, S, CAP, Kp, (int)kq, Qp,
-                         (int)ld, (int)dim, metric, X.p, ranks.rank.p, ranks.rank_slot.p, d_ids.p, qn, maxnorm, 4.0f,
+                         (int)ld, (int)dim, metric, X.p, ranks.rank.p, ranks.rank_slot.p, d_ids.p, qn, q_add, maxnorm, eps_c,
                          d_oid, d_od, d_oc, flag_list, flag_count, ldo);
     PXG_HIP(hipGetLastError());
   } else {
