@@ -56,6 +56,7 @@
 #include "device.hpp"
 #include "exact_scan.hpp"
 #include "flat.hpp"
+#include "split.hpp"
 #include "wide.hpp"
 
 namespace pxg {

@@ -40,6 +40,7 @@
 
 #include "common.hpp"
 #include "device.hpp"
+#include "split.hpp"
 #include "train.hpp"
 
 namespace pxg {
@@ -238,17 +239,22 @@ static void launch_assign(const float* P, int ldp, const uint32_t* rows, size_t 
 constexpr int KA_M = 128, KA_N = 128, KA_K = 32;
 
 // |row|^2 in fp32 (any order; it only feeds the approximation): eight lanes
-// per row, float4 loads (rows 16-byte aligned, dim a multiple of 4).
+// per row, float4 loads (vec4: rows 16-byte aligned, dim a multiple of 4) or
+// single ones.
 __device__ __forceinline__ void km_row_norms_body(const float* __restrict__ P, int ldp,
                                                   const uint32_t* __restrict__ rows, int n, int dim,
-                                                  float* __restrict__ out, int bx) {
+                                                  float* __restrict__ out, int bx, bool vec4 = true) {
   const int i = bx * 32 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
   float s = 0.0f;
   if (i < n) {
     const float* pr = P + (size_t)(rows ? rows[i] : (uint32_t)i) * ldp;
-    for (int j = sub * 4; j < dim; j += 32) {
-      const float4 x = *reinterpret_cast<const float4*>(pr + j);
-      s += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+    if (vec4) {
+      for (int j = sub * 4; j < dim; j += 32) {
+        const float4 x = *reinterpret_cast<const float4*>(pr + j);
+        s += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+      }
+    } else {
+      for (int j = sub; j < dim; j += 8) s += pr[j] * pr[j];
     }
   }
   s += __shfl_xor(s, 4, WAVE);
@@ -258,8 +264,8 @@ __device__ __forceinline__ void km_row_norms_body(const float* __restrict__ P, i
 }
 __global__ __launch_bounds__(256) void km_row_norms(const float* __restrict__ P, int ldp,
                                                     const uint32_t* __restrict__ rows, int n, int dim,
-                                                    float* __restrict__ out) {
-  km_row_norms_body(P, ldp, rows, n, dim, out, blockIdx.x);
+                                                    float* __restrict__ out, int vec4) {
+  km_row_norms_body(P, ldp, rows, n, dim, out, blockIdx.x, vec4 != 0);
 }
 
 // The largest of v[0..n), or NaN if any is NaN.
@@ -555,8 +561,7 @@ __global__ __launch_bounds__(256, 2) void km_mfma_small(const float* __restrict_
                          blockIdx.x);
 }
 
-// km_mfma_reg: km_mfma_small's form for rows of 32 to 128 floats (dim a
-// multiple of 32): each wave holds its 32 points' rows in VGPRs (lane half h
+// km_mfma_reg: km_mfma_small's form for rows of 32 floats: each wave holds its 32 points' rows in VGPRs (lane half h
 // the dims [h dim/2, (h+1) dim/2)) for the whole pass, and the centroids
 // stream through LDS 32 rows at a time (a block of the MFMA), copied
 // straight from memory (km_lds_copy16), double-buffered, one barrier per
@@ -677,6 +682,177 @@ __global__ __launch_bounds__(256, 3) void km_mfma_reg(const float* __restrict__ 
   }
 }
 
+// km_split: the assignment's approximate distances on the f16 matrix cores
+// (split.hpp), for rows of 64 to 32 NS floats (any alignment).
+//
+// km_split_cents writes the centroids' parts once per pass: per centroid and
+// 32 dimensions a record of 32 hi and 32 lo halves (zeros past dim and past
+// k), scaled by the largest centroid norm, and the norms padded with +inf to
+// whole blocks of 32.
+//
+// km_split: each wave takes 32 points, splits their rows once into VGPRs
+// (scaled by each point's own norm) and keeps them for the whole pass; the
+// records stream through LDS 32 centroids at a time (km_lds_copy16,
+// double-buffered, one barrier per block, chunk c of a row at c ^ (row & 7)).
+// Centroids are the MFMA's A operand and points B, so a lane ends each block
+// with its point's values for centroids 8 (v / 4) + 4 h + v % 4 and keeps the
+// top-2 in registers as km_mfma_small does.
+// What bounds it: per block and wave 6 NS MFMAs (192 NS cycles of the matrix
+// pipe) beside 80 VALU instructions of the top-2, which other waves' MFMAs
+// cover. A full pass over 2M x 128 points and 4096 centroids: 16.3 ms on the
+// f32 MFMA (km_mfma_reg's form, 129 TFLOP/s) -> 5.6 ms here (375 TFLOP/s of
+// f32 products, 1125 of f16 ones; the card's large f16 matrix product reaches
+// 1140); 300k x 96 and 1024 centroids 264 -> 85 us; 60k x 100 and 300
+// centroids 64 us (km_mfma_top) -> 20 us.
+// From 64 dimensions because of the error (split.hpp), to 256 because a
+// lane's 16 registers per 32 dimensions of its point would not leave two
+// waves per SIMD beyond; 32 and 33-63 dimensions keep km_mfma_reg and
+// km_mfma_top, wider rows km_mfma_top.
+//
+// A centroid or point norm that the scales cannot hold gets best = second, so
+// that the certificate sends it to the exact scan.
+constexpr int KM_SPLIT_MAX_DIM = 256;
+
+// km_mfma_verify's eps is 2 (eps_d d + 6) 2^-24 s^2 with s = |p| + max |c|.
+// In units of 2^-24 s^2 (4 |p||c| <= s^2) the split product's error counts
+// (7.13 d + 6) / 2, the exact sequential sum's d + 3, the centroid's norm
+// d / 8 + 3 and the last rounding 2: below 4.7 d + 11.
+constexpr float KM_SPLIT_EPS_D = 2.5f;
+
+// Centroid norms the split pass takes: a point whose own squared norm
+// underflows to 0 goes in as zeros, which is within eps only while the
+// centroids' norms are above about 2^-58.
+__device__ __forceinline__ bool km_split_cmax_ok(float cmax) {
+  return cmax == 0.0f || (cmax >= 0x1p-100f && cmax <= 0x1p+120f);
+}
+
+__global__ __launch_bounds__(256) void km_split_cents(const float* __restrict__ C, int ldc, int k, int dim, int ns,
+                                                      const float* __restrict__ cn, const float* __restrict__ cmax,
+                                                      _Float16* __restrict__ out, float* __restrict__ cn_pad) {
+  const int kr = (k + 31) & ~31;
+  const float cm = cmax[0];
+  const float sc = km_split_cmax_ok(cm) ? split_scale(sqrtf(cm)) : 0.0f;
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int w = 32 * ns;
+  if (t < (size_t)kr) cn_pad[t] = t < (size_t)k ? cn[t] : INFINITY;
+  if (t >= (size_t)kr * w) return;
+  const int c = (int)(t / w), j = (int)(t - (size_t)c * w);
+  _Float16 hi = (_Float16)0.0f, lo = (_Float16)0.0f;
+  if (c < k && j < dim) split_f16(C[(size_t)c * ldc + j], sc, hi, lo);
+  _Float16* rec = out + ((size_t)c * ns + (j >> 5)) * 64 + (j & 31);
+  rec[0] = hi;
+  rec[32] = lo;
+}
+
+template <int NS>
+__global__ __launch_bounds__(256, (NS <= 4 ? 3 : 2)) void km_split(
+    const float* __restrict__ P, int ldp, const uint32_t* __restrict__ rows, int n, int dim, int vec4,
+    const _Float16* __restrict__ Cs, int k, const float* __restrict__ cn_pad, const float* __restrict__ pn,
+    const float* __restrict__ cmax, uint32_t* __restrict__ best_idx, float* __restrict__ best,
+    float* __restrict__ second) {
+  constexpr int CPR = 8 * NS;        // 16-byte chunks per centroid
+  constexpr int TILE = 32 * 32 * NS;  // words per centroid block
+  __shared__ __align__(16) float sc[2 * TILE];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, r = lane & 31;
+  const int wid_s = __builtin_amdgcn_readfirstlane(w);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) float*)sc;
+  // the copy of block b into buffer buf: instruction u of wave w covers chunk
+  // positions 64 (w NS + u) + lane of the block's 32 CPR
+  auto gload = [&](int b, int buf) __attribute__((always_inline)) {
+    const char* cb = reinterpret_cast<const char*>(Cs) + (size_t)b * (TILE * 4);
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      const int g = wid_s * NS + u;
+      const int idx = 64 * g + lane, row = idx / CPR, pos = idx - row * CPR;
+      km_lds_copy16(cb + (row * CPR + (pos ^ (row & 7))) * 16, lds0 + (uint32_t)((buf * TILE + 64 * 4 * g) * 4));
+    }
+  };
+  gload(0, 0);
+  const int p0 = (blockIdx.x * 4 + w) * 32;
+  const int pi = min(p0 + r, n - 1);
+  const float* prow = P + (size_t)(rows ? rows[pi] : (uint32_t)pi) * ldp;
+  const float cm = cmax[0], pnorm = sqrtf(pn[pi]);
+  const bool ok = km_split_cmax_ok(cm) && (pnorm == 0.0f || split_norm_ok(pnorm));
+  const float sp = ok ? split_scale(pnorm) : 0.0f;
+  // a block's value is cn - 2 p.c = fma(f, acc, cn); the factor is exact
+  const float f = ok ? -2.0f / split_scale(sqrtf(cm)) / sp : 0.0f;
+  h8v ph[2 * NS], pl[2 * NS];
+#pragma unroll
+  for (int t = 0; t < 2 * NS; ++t) {
+    float x[8];
+    const int j0 = 16 * t + 8 * h;
+    if (vec4) {
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+      if (j0 < dim) a = *reinterpret_cast<const float4*>(prow + j0);
+      if (j0 + 4 < dim) b = *reinterpret_cast<const float4*>(prow + j0 + 4);
+      x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = j0 + e < dim ? prow[j0 + e] : 0.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      _Float16 hi, lo;
+      split_f16(x[e], sp, hi, lo);
+      ph[t][e] = hi;
+      pl[t][e] = lo;
+    }
+  }
+  const int nblk = (k + 31) / 32;
+  float b1 = INFINITY, b2 = INFINITY;
+  int i1 = 0, t1 = 0;
+  auto take = [&](float x, int v) {
+    i1 = x < b1 ? v : i1;
+    b2 = __builtin_amdgcn_fmed3f(b1, b2, x);
+    b1 = fminf(b1, x);
+  };
+  const int r7 = r & 7;
+  for (int blk = 0; blk < nblk; ++blk) {
+    const int cur = blk & 1;
+    // this block's norms (rows 8 (v / 4) + 4 h + v % 4), loaded before the wait
+    float cv[16];
+#pragma unroll
+    for (int vb = 0; vb < 4; ++vb) {
+      const float4 c4 = *reinterpret_cast<const float4*>(cn_pad + blk * 32 + 4 * h + 8 * vb);
+      cv[4 * vb] = c4.x;
+      cv[4 * vb + 1] = c4.y;
+      cv[4 * vb + 2] = c4.z;
+      cv[4 * vb + 3] = c4.w;
+    }
+    km_vm_wait0();    // this wave's copies of block blk (and the norms) have landed
+    __syncthreads();  // everyone's copies of blk are in; everyone is done with blk - 1
+    if (blk + 1 < nblk) gload(blk + 1, cur ^ 1);
+    const float* ca = &sc[cur * TILE + r * (CPR * 4)];
+    f16v acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 2 * NS; ++t) {
+      // chunk 8 (t / 2) + 2 (t % 2) + h holds the hi parts, four on the lo
+      const int c = 8 * (t >> 1) + 2 * (t & 1) + h;
+      const h8v ah = *reinterpret_cast<const h8v*>(ca + ((c ^ r7) << 2));
+      const h8v al = *reinterpret_cast<const h8v*>(ca + (((c + 4) ^ r7) << 2));
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph[t], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, pl[t], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ph[t], acc, 0, 0, 0);
+    }
+    const float b1_in = b1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) take(__builtin_fmaf(f, acc[v], cv[v]), v);
+    t1 = b1 < b1_in ? blk : t1;
+  }
+  const int ix = t1 * 32 + 8 * (i1 >> 2) + 4 * h + (i1 & 3);
+  const float y1 = __shfl_xor(b1, 32, WAVE), y2 = __shfl_xor(b2, 32, WAVE);
+  const int yi = __shfl_xor(ix, 32, WAVE);
+  if (h == 0 && p0 + r < n) {
+    const bool tk = y1 < b1 || (y1 == b1 && yi < ix);
+    const float bst = tk ? y1 : b1;
+    best[p0 + r] = bst;
+    best_idx[p0 + r] = (uint32_t)min(tk ? yi : ix, k - 1);
+    second[p0 + r] = ok ? fminf(tk ? b1 : y1, fminf(b2, y2)) : bst;
+  }
+}
+
 constexpr int KV_PB = 128;  // points per km_mfma_verify block (256 threads)
 template <bool UNR>
 __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P, int ldp,
@@ -686,7 +862,8 @@ __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P,
                                                     const uint32_t* __restrict__ best_idx,
                                                     const float* __restrict__ best, const float* __restrict__ second,
                                                     uint32_t* __restrict__ assign, float* __restrict__ dist,
-                                                    uint32_t* __restrict__ redo, int* __restrict__ nredo, int bx) {
+                                                    uint32_t* __restrict__ redo, int* __restrict__ nredo, int bx,
+                                                    float eps_d = 2.0f, bool vec4 = true) {
   // the block's KV_PB points and their winning centroids, staged through LDS
   // 32 coordinates at a time (eight lanes per 128-byte row slice); 34 KB of
   // LDS, so four blocks per CU keep the row loads in flight
@@ -697,7 +874,7 @@ __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P,
   if (t < KV_PB) {  // threads KV_PB.. only help with the loads
     if (i < n) {
       const float s = (sqrtf(pn[i]) + sqrtf(cmax[0])) * 1.0001f;
-      const float eps = 2.0f * (2.0f * (float)dim + 6.0f) * 5.9604645e-08f * s * s;
+      const float eps = 2.0f * (eps_d * (float)dim + 6.0f) * 5.9604645e-08f * s * s;
       ok = second[i] > best[i] + 2.0f * eps;
       if (!ok) redo[atomicAdd(nredo, 1)] = (uint32_t)i;
       sr[t] = rows ? rows[i] : (uint32_t)i;
@@ -715,10 +892,19 @@ __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P,
     for (int f = t; f < KV_PB * 8; f += 256) {
       const int r = f >> 3, c4 = (f & 7) * 4;
       if (c4 < w && i0 + r < n) {
-        const float4 x = *reinterpret_cast<const float4*>(P + (size_t)sr[r] * ldp + j0 + c4);
-        const float4 y = *reinterpret_cast<const float4*>(C + (size_t)sc[r] * ldc + j0 + c4);
+        const float* pr = P + (size_t)sr[r] * ldp + j0 + c4;
+        const float* cr = C + (size_t)sc[r] * ldc + j0 + c4;
         float* dp = tp + r * 33 + c4;
         float* dc = tc + r * 33 + c4;
+        if (!vec4) {
+          for (int e = 0; e < 4 && c4 + e < w; ++e) {
+            dp[e] = pr[e];
+            dc[e] = cr[e];
+          }
+          continue;
+        }
+        const float4 x = *reinterpret_cast<const float4*>(pr);
+        const float4 y = *reinterpret_cast<const float4*>(cr);
         dp[0] = x.x; dp[1] = x.y; dp[2] = x.z; dp[3] = x.w;
         dc[0] = y.x; dc[1] = y.y; dc[2] = y.z; dc[3] = y.w;
       }
@@ -762,9 +948,10 @@ __global__ __launch_bounds__(256) void km_mfma_verify(const float* __restrict__ 
                                                       const uint32_t* __restrict__ best_idx,
                                                       const float* __restrict__ best, const float* __restrict__ second,
                                                       uint32_t* __restrict__ assign, float* __restrict__ dist,
-                                                      uint32_t* __restrict__ redo, int* __restrict__ nredo) {
+                                                      uint32_t* __restrict__ redo, int* __restrict__ nredo,
+                                                      float eps_d, int vec4) {
   km_mfma_verify_body<UNR>(P, ldp, rows, n, dim, C, ldc, pn, cmax, best_idx, best, second, assign, dist, redo, nredo,
-                           blockIdx.x);
+                           blockIdx.x, eps_d, vec4 != 0);
 }
 
 constexpr int KW_DMAX = 2048;  // largest dim of the MFMA assignment path
@@ -775,10 +962,11 @@ constexpr int KW_DMAX = 2048;  // largest dim of the MFMA assignment path
 // stream once per KX_PB points. Per point the distance is the reference's
 // sequential `squared` (or, UNR, the 8-lane kernel); the lanes' and waves'
 // bests merge lexicographically in (distance, centroid), which keeps the
-// lowest index among equal distances. Centroid rows are read as float4 (rows
-// 16-byte aligned, dim a multiple of 4, dim <= KW_DMAX).
+// lowest index among equal distances. V4: centroid rows are read as float4
+// (rows 16-byte aligned, dim a multiple of 4), else one float at a time;
+// dim <= KW_DMAX.
 constexpr int KX_PB = 8;
-template <bool UNR>
+template <bool UNR, bool V4 = true>
 __global__ __launch_bounds__(256) void km_exact_multi(const float* __restrict__ P, int ldp,
                                                       const uint32_t* __restrict__ rows, int m, int dim,
                                                       const float* __restrict__ C, int ldc, int k,
@@ -812,14 +1000,28 @@ __global__ __launch_bounds__(256) void km_exact_multi(const float* __restrict__ 
 #pragma unroll
         for (int u = 0; u < 8; ++u) acc[i][u] = 0.0f;
       for (int j = 0; j < ch8; j += 8) {
-        const float4 c0 = *reinterpret_cast<const float4*>(cr + j);
-        const float4 c1 = *reinterpret_cast<const float4*>(cr + j + 4);
-        const float cv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        float cv[8];
+        if constexpr (V4) {
+          const float4 c0 = *reinterpret_cast<const float4*>(cr + j);
+          const float4 c1 = *reinterpret_cast<const float4*>(cr + j + 4);
+          cv[0] = c0.x, cv[1] = c0.y, cv[2] = c0.z, cv[3] = c0.w, cv[4] = c1.x, cv[5] = c1.y, cv[6] = c1.z,
+          cv[7] = c1.w;
+        } else {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) cv[u] = cr[j + u];
+        }
 #pragma unroll
         for (int i = 0; i < KX_PB; ++i) {
-          const float4 x0 = *reinterpret_cast<const float4*>(sp + i * dim + j);
-          const float4 x1 = *reinterpret_cast<const float4*>(sp + i * dim + j + 4);
-          const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+          float xv[8];
+          if constexpr (V4) {
+            const float4 x0 = *reinterpret_cast<const float4*>(sp + i * dim + j);
+            const float4 x1 = *reinterpret_cast<const float4*>(sp + i * dim + j + 4);
+            xv[0] = x0.x, xv[1] = x0.y, xv[2] = x0.z, xv[3] = x0.w, xv[4] = x1.x, xv[5] = x1.y, xv[6] = x1.z,
+            xv[7] = x1.w;
+          } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) xv[u] = sp[i * dim + j + u];
+          }
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
             const float d = xv[u] - cv[u];
@@ -840,6 +1042,17 @@ __global__ __launch_bounds__(256) void km_exact_multi(const float* __restrict__ 
     } else {
 #pragma unroll
       for (int i = 0; i < KX_PB; ++i) sum[i] = 0.0f;
+      if constexpr (!V4) {
+#pragma unroll 4
+        for (int j = 0; j < dim; ++j) {
+          const float cj = cr[j];
+#pragma unroll
+          for (int i = 0; i < KX_PB; ++i) {
+            const float d = sp[i * dim + j] - cj;
+            sum[i] += d * d;
+          }
+        }
+      } else
       for (int j = 0; j < dim; j += 4) {
         const float4 cv = *reinterpret_cast<const float4*>(cr + j);
 #pragma unroll
@@ -907,7 +1120,7 @@ __global__ void km_compose_rows(const uint32_t* __restrict__ redo, int m, const 
   if (t < m) out[t] = rows ? rows[redo[t]] : redo[t];
 }
 
-// Points with enough work for the matrix cores (and float4-aligned rows)
+// Points with enough work for the matrix cores
 // take the MFMA pass; the exact VALU scan serves the rest and the points the
 // MFMA pass cannot certify.
 void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int dim, const float* C, int ldc,
@@ -923,7 +1136,9 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
                        ((uintptr_t)C & 15) == 0;
   // narrow rows (product-quantizer subspaces) with their centroids in LDS
   const bool small = aligned && (dim == 8 || dim == 16 || dim == 24) && k >= 64 && k * dim <= KS_MAXF && n >= 4096;
-  if (!small && !(aligned && dim >= 32 && dim <= KW_DMAX && k >= 64 && n >= 4096)) {
+  // rows of 64 to 256 floats, of any alignment, on the f16 matrix cores
+  const bool split = dim >= (int)SPLIT_MIN_DIM && dim <= KM_SPLIT_MAX_DIM && k >= 64 && n >= 4096;
+  if (!small && !split && !(aligned && dim >= 32 && dim <= KW_DMAX && k >= 64 && n >= 4096)) {
     if (unrolled)
       launch_assign<true>(P, ldp, rows, n, dim, C, ldc, k, assign, dist, s);
     else
@@ -947,14 +1162,14 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
   const bool keyed = rows == nullptr;
   if (!(keyed && w.pn_of == P && w.pn_ld == ldp && w.pn_dim == dim && w.pn_n == n)) {
     hipLaunchKernelGGL(km_row_norms, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, s, P, ldp, rows, (int)n, dim,
-                       pn);
+                       pn, (int)aligned);
     w.pn_of = keyed ? P : nullptr;
     w.pn_ld = ldp;
     w.pn_dim = dim;
     w.pn_n = n;
   }
   hipLaunchKernelGGL(km_row_norms, dim3((unsigned)((k + 31) / 32)), dim3(256), 0, s, C, ldc,
-                     (const uint32_t*)nullptr, (int)k, dim, cn);
+                     (const uint32_t*)nullptr, (int)k, dim, cn, (int)aligned);
   hipLaunchKernelGGL(km_max_of, dim3(1), dim3(1024), 0, s, cn, (int)k, cmax);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (small) {
@@ -974,15 +1189,30 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
     PXG_HIP(hipEventCreate(&e1));
     PXG_HIP(hipEventRecord(e0, s));
     const dim3 g128((unsigned)((n + 127) / 128));
-    if (dim == 128)
-      hipLaunchKernelGGL(km_mfma_reg<64>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
-                         (const float*)cn, bidx, best, second);
-    else if (dim == 96)
-      hipLaunchKernelGGL(km_mfma_reg<48>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
-                         (const float*)cn, bidx, best, second);
-    else if (dim == 64)
-      hipLaunchKernelGGL(km_mfma_reg<32>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
-                         (const float*)cn, bidx, best, second);
+    if (split) {
+      const int ns = (dim + 31) / 32, kr = ((int)k + 31) & ~31;
+      w.cs.reserve((size_t)kr * ns * 32);
+      w.cn_pad.reserve(kr);
+      _Float16* cs = reinterpret_cast<_Float16*>(w.cs.p);
+      hipLaunchKernelGGL(km_split_cents, dim3((unsigned)(((size_t)kr * ns * 32 + 255) / 256)), dim3(256), 0, s, C, ldc,
+                         (int)k, dim, ns, (const float*)cn, (const float*)cmax, cs, w.cn_pad.p);
+#define PXG_KM_SPLIT(NSV)                                                                                            \
+  case NSV:                                                                                                          \
+    hipLaunchKernelGGL(km_split<NSV>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, dim, (int)aligned,                \
+                       (const _Float16*)cs, (int)k, (const float*)w.cn_pad.p, (const float*)pn, (const float*)cmax,  \
+                       bidx, best, second);                                                                          \
+    break
+      switch (ns) {
+        PXG_KM_SPLIT(2);
+        PXG_KM_SPLIT(3);
+        PXG_KM_SPLIT(4);
+        PXG_KM_SPLIT(5);
+        PXG_KM_SPLIT(6);
+        PXG_KM_SPLIT(7);
+        PXG_KM_SPLIT(8);
+      }
+#undef PXG_KM_SPLIT
+    }
     else if (dim == 32)
       hipLaunchKernelGGL(km_mfma_reg<16>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
                          (const float*)cn, bidx, best, second);
@@ -993,14 +1223,15 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
   }
   PXG_HIP(hipMemsetAsync(nredo, 0, 4, s));
   const dim3 g((unsigned)((n + KV_PB - 1) / KV_PB));
+  const float eps_d = split ? KM_SPLIT_EPS_D : 2.0f;
   if (unrolled)
     hipLaunchKernelGGL(km_mfma_verify<true>, g, dim3(256), 0, s, P, ldp, rows, (int)n, dim, C, ldc, (const float*)pn,
                        (const float*)cmax, (const uint32_t*)bidx, (const float*)best, (const float*)second, assign,
-                       dist, redo, nredo);
+                       dist, redo, nredo, eps_d, (int)aligned);
   else
     hipLaunchKernelGGL(km_mfma_verify<false>, g, dim3(256), 0, s, P, ldp, rows, (int)n, dim, C, ldc, (const float*)pn,
                        (const float*)cmax, (const uint32_t*)bidx, (const float*)best, (const float*)second, assign,
-                       dist, redo, nredo);
+                       dist, redo, nredo, eps_d, (int)aligned);
   PXG_HIP(hipGetLastError());
   int m = 0;
   PXG_HIP(hipMemcpyAsync(&m, nredo, 4, hipMemcpyDeviceToHost, s));
@@ -1027,12 +1258,15 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
                      rows, rrows);
   const dim3 gx((unsigned)((m + KX_PB - 1) / KX_PB));
   const size_t lx = (size_t)KX_PB * dim * 4;
-  if (unrolled)
-    hipLaunchKernelGGL(km_exact_multi<true>, gx, dim3(256), lx, s, P, ldp, (const uint32_t*)rrows, m, dim, C, ldc,
-                       (int)k, ra, rd);
-  else
-    hipLaunchKernelGGL(km_exact_multi<false>, gx, dim3(256), lx, s, P, ldp, (const uint32_t*)rrows, m, dim, C, ldc,
-                       (int)k, ra, rd);
+#define PXG_EXACT(UNRV, V4V)                                                                                       \
+  hipLaunchKernelGGL((km_exact_multi<UNRV, V4V>), gx, dim3(256), lx, s, P, ldp, (const uint32_t*)rrows, m, dim, C, \
+                     ldc, (int)k, ra, rd)
+  if (unrolled) {
+    if (aligned) PXG_EXACT(true, true); else PXG_EXACT(true, false);
+  } else {
+    if (aligned) PXG_EXACT(false, true); else PXG_EXACT(false, false);
+  }
+#undef PXG_EXACT
   hipLaunchKernelGGL(km_scatter_redo, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, (const uint32_t*)redo, m,
                      (const uint32_t*)ra, (const float*)rd, assign, dist);
   PXG_HIP(hipGetLastError());

@@ -55,7 +55,8 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
 // them, the point norms are reused: the caller promises the points did not
 // change in between.
 struct NearestWork {
-  DevBuf<float> pn, cn, cmax, best, second, rd;
+  DevBuf<float> pn, cn, cmax, best, second, rd, cn_pad;
+  DevBuf<uint32_t> cs;  // the centroids' f16 parts
   DevBuf<uint32_t> bidx, redo, rrows, ra;
   DevBuf<int> nredo;
   const float* pn_of = nullptr;

@@ -388,3 +388,37 @@ def test_kmeans_pp_certified_int8_rounds(gpu, case):
     w = orc.kmeans(pts, k, 4, 3)
     assert np.array_equal(bits(g.centroids.reshape(-1)), bits(w[0].reshape(-1)))
     assert g.inertia == w[1] and g.iterations == w[2]
+
+
+@pytest.mark.parametrize("n,dim,k", [(4096, 64, 64), (4099, 65, 65), (5003, 95, 97), (4100, 100, 300), (4127, 127, 64),
+                                     (4128, 129, 31 + 64), (4500, 160, 70), (4096, 190, 64), (4700, 222, 80),
+                                     (4097, 256, 129)])
+@pytest.mark.parametrize("scale", [1.0, 1e-13, 1e-17, 3e16, 1e19])
+def test_assign_split_widths(gpu, n, dim, k, scale):
+    """The f16 split pass at the edges of its tiles (32 points, 32 centroids,
+    32 dimensions), for rows of any alignment, and at both ends of the norms
+    its scales hold (beyond them every point takes the exact scan): the
+    assignment and the distances are the oracle's bits."""
+    rng = np.random.default_rng(dim + k)
+    cents = rng.standard_normal((k, dim))
+    pts = cents[rng.integers(0, k, n)] + 0.4 * rng.standard_normal((n, dim))
+    pts[5] = 0.0
+    pts[7] *= 1e-6
+    cents[k - 1] = cents[3]  # a tie: the lower index wins
+    pts, cents = (pts * scale).astype(np.float32), (cents * scale).astype(np.float32)
+    a, d = gpu.kmeans_assign(pts, cents)
+    with np.errstate(all="ignore"):
+        wa, wd = orc.kmeans_assign(pts, cents)
+    assert np.array_equal(a, wa)
+    assert np.array_equal(d.view(np.uint32), wd.view(np.uint32))
+
+
+@pytest.mark.parametrize("dim", [66, 100])
+def test_lloyd_split_any_alignment(gpu, dim):
+    rng = np.random.default_rng(dim)
+    pts = (rng.standard_normal((40, dim))[rng.integers(0, 40, 4800)] + 0.3 * rng.standard_normal((4800, dim))).astype(np.float32)
+    init = pts[:70].copy()
+    cents, assign, inertia, its = gpu.kmeans_lloyd(pts, init, 6)
+    want = orc.kmeans_lloyd(pts, init, 6)
+    assert np.array_equal(np.asarray(want[0], np.float32).reshape(cents.shape).view(np.uint32), cents.view(np.uint32))
+    assert np.array_equal(want[1], assign) and want[2] == inertia and want[3] == its
