@@ -1526,27 +1526,54 @@ __global__ __launch_bounds__(256) void km_pp_round(const float* __restrict__ P, 
 }
 
 // ---------------------------------------------------------------------------
-// k-means++ rounds over an int8 copy of the points, certified
+// k-means++ rounds over 4-bit and int8 copies of the points, certified
 // ---------------------------------------------------------------------------
 // A round only lowers ns[i] when the new centre c is strictly nearer than the
-// current one. Each point also has an int8 copy q_i (scale s_i = max|p_i| /
-// 127, q = rint(p / s_i)) and the exact distance delta_i = |p_i - s_i q_i|.
-// The centre is itself a point (kmeans.rs:169-186 picks rows), so it has q_c,
-// s_c and delta_c. With e = |s_i q_i - s_c q_c| from the exact integer dot
-// product, the triangle inequality gives |p_i - c| >= e - delta_i - delta_c
-// = L. The reference's sequential f32 sum (kmeans.rs:234-241) of dim
-// squares is >= |p_i - c|^2 (1 - (dim + 2) 2^-24) for non-negative terms, so
-// when L^2 (1 - gamma) >= ns[i] (with margins for the f64 rounding of e and
-// for subnormal terms) the exact distance cannot be below ns[i] and the
-// point keeps its value without its f32 row being read. The other points
-// (those the centre may capture) are scored exactly as km_pp_round does.
-// Per point the round then reads 4 + 16 bytes plus dim bytes, not 4 dim.
-constexpr int Q8_ROWS = 256;  // points per km_pp_round_q8 block
+// current one, so a point keeps its value without its f32 row being read when
+// a lower bound L on |p_i - c| has L^2 (1 - gamma) >= ns[i]: the reference's
+// sequential f32 sum (kmeans.rs:234-241) of dim squares is
+// >= |p_i - c|^2 (1 - (dim + 2) 2^-24) for non-negative terms (with margins
+// for the f64 rounding and for subnormal terms). Three bounds are tried, each
+// reading more of the point than the one before:
+//
+//  1. near[i] is the chosen centre a whose distance ns[i] holds.
+//     |p - c| >= |a - c| - |p - a|, with |p - a|^2 <= (ns + 1e-35) /
+//     (1 - gamma) from ns being the reference's sum for a. km_pp_cdist leaves
+//     T[a] <= |a - c|^2 (1 - gamma) / 4; ns + 1e-35 <= T[a] gives
+//     |p - a| <= |a - c| / 2 <= |p - c|, hence the test. Reads 8 bytes.
+//  2. A 4-bit copy q_i (scale s_i = max|p_i| / 7 rounded up to bf16, q =
+//     rint(p / s_i)) with delta_i >= |p_i - s_i q_i|. The centre is itself a
+//     point (kmeans.rs:169-186 picks rows) with an int8 copy: from the exact
+//     integer dot product, e = |s_i q_i - s_c q_c| and |p_i - c| >= e -
+//     delta_i - delta_c. Reads dim / 2 + 4 bytes.
+//  3. The same with the point's own int8 copy (scale max|p_i| / 119, so that
+//     a code is 16 a + b with a and b in [-8, 7], the two 4-bit words that
+//     step 2 multiplies). Reads dim + 12 bytes.
+//
+// The points none of them settles (those the centre may capture) are scored
+// exactly as km_pp_round does. Blocks none of whose distances changed keep
+// their sums.
+//
+// What bounds a round: memory while many points' clusters hold no centre yet
+// (those stop at step 2; four lanes read one point's 64 bytes at 128
+// dimensions together, one lane per point having cost one cache line per lane
+// and instruction), and later, when almost every point stops at step 1, the
+// chain of dependent loads. Mean over 4096 centres of 2M x 128: 39.2 us a
+// round with the int8 copy alone -> 28.3 (181 -> 208 in the first, 43.8 ->
+// 32.9 at the 800th, 22.5 -> 16.2 at the 4000th); 1024 centres of 100k x 96:
+// 7.9 -> 7.0 us. km_pp_pick, its partials loaded together: 14.7 -> 11.1 us.
+constexpr int Q8_MAX = 119;
 
-// int8 copy, scale, delta and squared norm of the copy: one wave per point.
+// Smallest bf16 at or above x >= 0, as its 16 bits (infinity where none is).
+__device__ __forceinline__ uint32_t bf16_up(float x) { return (__float_as_uint(x) + 0xFFFFu) >> 16; }
+
+// The copies, scales, deltas and the int8 copy's squared norm: one wave per
+// point. Q4: 16-byte chunks of 32 dimensions, dimension j the nibble j % 8 of
+// word j / 8; meta4: bf16 scale << 16 | bf16 delta.
 __global__ __launch_bounds__(256) void km_q8_prep(const float* __restrict__ P, int ldp, int n, int dim, int kq,
                                                   int8_t* __restrict__ Q, float* __restrict__ scale,
-                                                  float* __restrict__ delta, int* __restrict__ qnorm) {
+                                                  float* __restrict__ delta, int* __restrict__ qnorm, int words4,
+                                                  uint32_t* __restrict__ Q4, uint32_t* __restrict__ meta4) {
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= n) return;
@@ -1554,97 +1581,262 @@ __global__ __launch_bounds__(256) void km_q8_prep(const float* __restrict__ P, i
   float mx = 0.0f;
   for (int j = lane; j < dim; j += 64) mx = fmaxf(mx, fabsf(p[j]));
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  const float sc = mx / 127.0f;
-  double d2 = 0.0;
+  const float sc = mx / (float)Q8_MAX;
+  const float s4u = __uint_as_float(bf16_up(mx / 7.0f) << 16);
+  const float s4 = isfinite(s4u) ? s4u : 0.0f;
+  double d2 = 0.0, d42 = 0.0;
   int qn = 0;
-  for (int j = lane; j < kq; j += 64) {
-    int q = 0;
-    if (j < dim && sc > 0.0f) q = max(-127, min(127, (int)rintf(p[j] / sc)));
-    if (j < dim) {
-      const double r = (double)p[j] - (double)q * (double)sc;
-      d2 += r * r;
-    }
+  for (int j0 = 0; j0 < words4 * 8; j0 += 64) {
+    const int j = j0 + lane;
+    const float x = j < dim ? p[j] : 0.0f;
+    int q = 0, q4 = 0;
+    if (sc > 0.0f) q = max(-Q8_MAX, min(Q8_MAX, (int)rintf(x / sc)));
+    if (s4 > 0.0f) q4 = max(-7, min(7, (int)rintf(x / s4)));
+    const double r = (double)x - (double)q * (double)sc, r4 = (double)x - (double)q4 * (double)s4;
+    d2 += r * r;
+    d42 += r4 * r4;
     qn += q * q;
-    Q[(size_t)i * kq + j] = (int8_t)q;
+    if (j < kq) Q[(size_t)i * kq + j] = (int8_t)q;
+    // eight lanes' nibbles to one word
+    uint32_t w = (uint32_t)(q4 & 15) << (4 * (lane & 7));
+    w |= xor_lane<1>(w);
+    w |= xor_lane<2>(w);
+    w |= xor_lane<4>(w);
+    if (Q4 != nullptr && (lane & 7) == 0 && j < words4 * 8) Q4[(size_t)i * words4 + (j >> 3)] = w;
   }
   for (int o = 32; o > 0; o >>= 1) {
     d2 += __shfl_xor(d2, o, 64);
+    d42 += __shfl_xor(d42, o, 64);
     qn += __shfl_xor(qn, o, 64);
   }
   if (lane == 0) {
     scale[i] = sc;
-    // an upper bound in f32 (the f64 sum's own rounding is far below one ulp)
-    const double d = sqrt(d2) * (1.0 + 1e-12);
-    float df = (float)d;
-    if ((double)df < d) df = nextafterf(df, INFINITY);
-    delta[i] = isfinite(mx) ? df : INFINITY;
+    // upper bounds in f32 (the f64 sum's own rounding is far below one ulp)
+    auto up = [&](double v) {
+      const double d = sqrt(v) * (1.0 + 1e-12);
+      float df = (float)d;
+      if ((double)df < d) df = nextafterf(df, INFINITY);
+      return isfinite(mx) ? df : INFINITY;
+    };
+    delta[i] = up(d2);
+    meta4[i] = (__float_as_uint(s4) & 0xFFFF0000u) | bf16_up(up(d42));
     qnorm[i] = qn;
   }
 }
 
-// Lower bounds on the distances from the chosen centres 0 .. chosen-1 to
-// centre `chosen` (all rows of the points): f64 sums of the f32 coordinates'
-// squared differences, four lanes per centre, rounded down to f32 after a
-// relative margin far above the f64 rounding.
-__global__ __launch_bounds__(256) void km_pp_cdist(const float* __restrict__ cents, int dim, int chosen,
-                                                   float* __restrict__ dcc) {
-  const int j = blockIdx.x * 64 + (threadIdx.x >> 2), part = threadIdx.x & 3;
+// T[j] for the chosen centres 0 .. chosen-1 (step 1 above) against centre
+// `chosen` (all rows of the points): f64 sums of the f32 coordinates' squared
+// differences, sixteen lanes per centre, rounded down after a relative margin
+// far above the f64 rounding and the f32 addition of the test.
+__global__ __launch_bounds__(256) void km_pp_cdist(const float* __restrict__ cents, int dim, int chosen, double gamma,
+                                                   float* __restrict__ T) {
+  const int j = blockIdx.x * 16 + (threadIdx.x >> 4), part = threadIdx.x & 15;
   const bool on = j < chosen;
   const float* a = cents + (size_t)(on ? j : 0) * dim;
   const float* b = cents + (size_t)chosen * dim;
   double d = 0.0;
-  for (int u = part; u < dim; u += 4) {
+#pragma unroll 4
+  for (int u = part; u < dim; u += 16) {
     const double x = (double)a[u] - (double)b[u];
     d += x * x;
   }
-  d += __shfl_xor(d, 1, 64);
-  d += __shfl_xor(d, 2, 64);
-  if (on && part == 0) dcc[j] = __double2float_rd(sqrt(d) * (1.0 - 1e-12));
+  d += shfl_xor_f64(d, 1);
+  d += shfl_xor_f64(d, 2);
+  d += shfl_xor_f64(d, 4);
+  d += shfl_xor_f64(d, 8);
+  if (on && part == 0) T[j] = __double2float_rd(0.25 * d * (1.0 - gamma) * (1.0 - 1e-6));
 }
 
-// near[i] is the chosen centre whose distance ns[i] holds. Before the
-// int8 test, a point whose nearest centre a lies far from the new centre c
-// keeps its distance without reading its codes: |p - c| >= |a - c| - |p - a|,
-// with |p - a|^2 <= (ns + 1e-35) / (1 - gamma) from ns being the reference's
-// sequential sum for a, and dcc[a] a lower bound on |a - c|; the same
-// L^2 (1 - gamma) >= ns + 1e-35 test as the int8 bound then follows.
-__global__ __launch_bounds__(256) void km_pp_round_q8(const float* __restrict__ P, int ldp, int n, int dim,
-                                                      const int8_t* __restrict__ Q, int kq,
-                                                      const float* __restrict__ scale,
-                                                      const float* __restrict__ delta, const int* __restrict__ qnorm,
-                                                      const int* __restrict__ picked, float* __restrict__ ns,
-                                                      double* __restrict__ ps, int* __restrict__ pe,
-                                                      double gamma, uint32_t* __restrict__ near,
-                                                      const float* __restrict__ dcc, int chosen) {
-  __shared__ int qc[KW_DMAX / 4];
-  __shared__ float cs[KW_DMAX];
-  __shared__ int list[Q8_ROWS];
-  __shared__ int nlist;
+// |s q - s_c q_c| lower bound against ns: the test of steps 2 and 3, from the
+// exact integers qn = |q|^2, qnc = |q_c|^2 and dot.
+__device__ __forceinline__ bool km_pp_keeps(float cur, double sp, double qn, double dp, double sc, double qnc,
+                                            double dc, double dot, double gamma) {
+  const double A = sp * sp * qn, B = sc * sc * qnc, C = sp * sc * dot;
+  const double e2 = A + B - 2.0 * C;
+  const double err = 1e-13 * (A + B + 2.0 * fabs(C));
+  const double e = sqrt(fmax(e2 - err, 0.0)) * (1.0 - 1e-13);
+  const double L = e - dp - dc;
+  return isfinite(cur) && L > 0.0 && L * L * (1.0 - gamma) >= (double)cur + 1e-35;
+}
+
+// One round. SUB blocks of PP_ROWS points per workgroup: four for stores whose
+// copies are read from memory (half a million points on), with LP lanes per
+// 4-bit row; one for smaller ones, which leave out step 2 (their round is a
+// chain of dependent loads and not bytes: with it 100k x 96 takes 8.6 us
+// instead of 7.9). Eight workgroups fit a CU (64 VGPRs, 15 KB of LDS up to 256
+// dimensions), so a round's workgroups are all resident at once and their
+// chains of dependent loads overlap.
+template <int LP, int SUB>
+__global__ __launch_bounds__(256, 8) void km_pp_round_q8(const float* __restrict__ P, int ldp, int n, int dim,
+                                                         const int8_t* __restrict__ Q, int kq,
+                                                         const float* __restrict__ scale,
+                                                         const float* __restrict__ delta,
+                                                         const int* __restrict__ qnorm,
+                                                         const uint32_t* __restrict__ Q4,
+                                                         const uint32_t* __restrict__ meta4, int words4,
+                                                         const int* __restrict__ picked, float* __restrict__ ns,
+                                                         double* __restrict__ ps, int* __restrict__ pe, double gamma,
+                                                         uint32_t* __restrict__ near, const float* __restrict__ T,
+                                                         int chosen) {
+  static_assert(PP_ROWS == 256, "one point per thread and sub-block");
+  constexpr int PTS = SUB * PP_ROWS;
+  constexpr bool FOUR = SUB > 1;
+  constexpr int WMAX = (LP < 16 ? 32 * LP : KW_DMAX) / 8;  // words of 8 nibbles
+  __shared__ __align__(16) uint32_t ch4[FOUR ? WMAX : 4], cl4[FOUR ? WMAX : 4];  // the centre's 4-bit words
+  __shared__ int qc[2 * WMAX];                             // its int8 codes
+  __shared__ float nv_s[PTS];
+  __shared__ uint16_t act[PTS], act8[FOUR ? PTS : 1], actx[PTS];
+  __shared__ __align__(16) float sq[8][132];
+  __shared__ int n_act, n_act8, n_actx, changed[SUB];
   __shared__ SumCert sh[4];
-  const int t = threadIdx.x;
-  const int c = *picked;
-  const int words = kq / 4;
-  for (int j = t; j < words; j += 256) qc[j] = reinterpret_cast<const int*>(Q + (size_t)c * kq)[j];
-  for (int j = t; j < dim; j += 256) cs[j] = P[(size_t)c * ldp + j];
-  if (t == 0) nlist = 0;
-  __syncthreads();
-  const double sc = scale[c], dc = delta[c], qnc = (double)qnorm[c];
-  const int i = blockIdx.x * Q8_ROWS + t;
-  float cur = 0.0f;
-  bool exact = false;
-  bool far = false;
-  if (i < n) {
-    cur = ns[i];
-    const double r = sqrt(((double)cur + 1e-35) / (1.0 - gamma)) * (1.0 + 1e-12);
-    const double L0 = (double)dcc[near[i]] - r;
-    far = isfinite(cur) && L0 > 0.0 && L0 * L0 * (1.0 - gamma) >= (double)cur + 1e-35;
+  const int t = threadIdx.x, lane = t & 63;
+  const size_t base = (size_t)blockIdx.x * PTS;
+  // the distances, nearest centres and the picked row together, then what
+  // hangs on them
+  float cur[SUB];
+  uint32_t nr[SUB];
+#pragma unroll
+  for (int b = 0; b < SUB; ++b) {
+    const size_t i = min(base + b * PP_ROWS + t, (size_t)n - 1);  // unconditional loads
+    cur[b] = ns[i];
+    nr[b] = near[i];
   }
-  if (i < n && !far) {
+  const int c = *picked;
+  if (t == 0) n_act = n_act8 = n_actx = 0;
+  if (t < SUB) changed[t] = 0;
+  float tn[SUB];
+#pragma unroll
+  for (int b = 0; b < SUB; ++b) tn[b] = T[nr[b]];
+  for (int j = t; j < (FOUR ? words4 : 0); j += 256) {
+    // eight int8 codes q = 16 a + b as two words of nibbles
+    uint32_t wa = 0, wb = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int q = 8 * j + e < dim ? Q[(size_t)c * kq + 8 * j + e] : 0;
+      const int a = (q + 8) >> 4;
+      wa |= (uint32_t)(a & 15) << (4 * e);
+      wb |= (uint32_t)((q - 16 * a) & 15) << (4 * e);
+    }
+    ch4[j] = wa;
+    cl4[j] = wb;
+  }
+  for (int j = t; j < kq / 4; j += 256) qc[j] = reinterpret_cast<const int*>(Q + (size_t)c * kq)[j];
+  const double sc = scale[c], dc = delta[c], qnc = (double)qnorm[c];
+  __syncthreads();
+  // 1. by the nearest centre's distance to the new one
+#pragma unroll
+  for (int b = 0; b < SUB; ++b) {
+    const bool in = base + b * PP_ROWS + t < (size_t)n;
+    const bool active = in && !(cur[b] + 1e-35f <= tn[b]);
+    nv_s[b * PP_ROWS + t] = in ? cur[b] : 0.0f;
+    const uint64_t m = __ballot(active);
+    if (m != 0) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&n_act, __popcll(m));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (active) act[at + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)(b * PP_ROWS + t);
+    }
+  }
+  __syncthreads();
+  const int m1 = n_act;
+  if (m1 == 0) return;  // no distance changes: the blocks keep their sums
+  // 2. the 4-bit copies: LP lanes multiply a point's row, four points of a
+  // group at once, and then each test one or more of the four
+  if constexpr (FOUR) {
+    const int chunks = words4 / 4, sub = t & (LP - 1), g = t / LP;
+    constexpr int G = 256 / LP, PER = (4 + LP - 1) / LP;
+    for (int u0 = 0; u0 < m1; u0 += 4 * G) {
+      int dot[4], qn[4];
+      uint32_t mt[PER];
+#pragma unroll
+      for (int x = 0; x < PER; ++x) mt[x] = meta4[base + act[min(u0 + ((sub + x * LP) & 3) * G + g, m1 - 1)]];
+      if constexpr (LP < 16) {
+        // at most LP chunks: one load per point and lane
+        uint4 v[4];
+        const bool on = sub < chunks;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const size_t i = base + act[min(u0 + e * G + g, m1 - 1)];
+          v[e] = *reinterpret_cast<const uint4*>(Q4 + i * words4 + 4 * (on ? sub : 0));
+        }
+        uint4 ca = make_uint4(0, 0, 0, 0), cb = ca;
+        if (on) {
+          ca = *reinterpret_cast<const uint4*>(ch4 + 4 * sub);
+          cb = *reinterpret_cast<const uint4*>(cl4 + 4 * sub);
+        }
+        const int cav[4] = {(int)ca.x, (int)ca.y, (int)ca.z, (int)ca.w};
+        const int cbv[4] = {(int)cb.x, (int)cb.y, (int)cb.z, (int)cb.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int w[4] = {(int)v[e].x, (int)v[e].y, (int)v[e].z, (int)v[e].w};
+          int da = 0, db = 0, q = 0;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            da = __builtin_amdgcn_sdot8(w[x], cav[x], da, false);
+            db = __builtin_amdgcn_sdot8(w[x], cbv[x], db, false);
+            q = __builtin_amdgcn_sdot8(w[x], w[x], q, false);
+          }
+          dot[e] = 16 * da + db;
+          qn[e] = on ? q : 0;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const size_t i = base + act[min(u0 + e * G + g, m1 - 1)];
+          int da = 0, db = 0, q = 0;
+          for (int ck = sub; ck < chunks; ck += LP) {
+            const uint4 v = *reinterpret_cast<const uint4*>(Q4 + i * words4 + 4 * ck);
+            const int w[4] = {(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              da = __builtin_amdgcn_sdot8(w[x], (int)ch4[4 * ck + x], da, false);
+              db = __builtin_amdgcn_sdot8(w[x], (int)cl4[4 * ck + x], db, false);
+              q = __builtin_amdgcn_sdot8(w[x], w[x], q, false);
+            }
+          }
+          dot[e] = 16 * da + db;
+          qn[e] = q;
+        }
+      }
+      auto sum = [](int x) {
+        if constexpr (LP >= 2) x += (int)xor_lane<1>((uint32_t)x);
+        if constexpr (LP >= 4) x += (int)xor_lane<2>((uint32_t)x);
+        if constexpr (LP >= 8) x += (int)xor_lane<4>((uint32_t)x);
+        if constexpr (LP >= 16) x += (int)xor_lane<8>((uint32_t)x);
+        return x;
+      };
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        dot[e] = sum(dot[e]);
+        qn[e] = sum(qn[e]);
+      }
+#pragma unroll
+      for (int x = 0; x < PER; ++x) {
+        const int e = sub + x * LP;
+        const int d = e == 0 ? dot[0] : e == 1 ? dot[1] : e == 2 ? dot[2] : dot[3];
+        const int q = e == 0 ? qn[0] : e == 1 ? qn[1] : e == 2 ? qn[2] : qn[3];
+        const int u = u0 + e * G + g;
+        if (e < 4 && u < m1) {
+          const int pt = act[u];
+          const double sp = (double)__uint_as_float(mt[x] & 0xFFFF0000u), dp = (double)__uint_as_float(mt[x] << 16);
+          if (!km_pp_keeps(nv_s[pt], sp, (double)q, dp, sc, qnc, dc, (double)d, gamma))
+            act8[atomicAdd(&n_act8, 1)] = (uint16_t)pt;
+        }
+      }
+    }
+  }
+  if constexpr (FOUR) __syncthreads();
+  // 3. the int8 copies of what is left
+  const int m2 = FOUR ? n_act8 : m1;
+  if (m2 == 0) return;
+  for (int u = t; u < m2; u += 256) {
+    const int pt = FOUR ? act8[u] : act[u];
+    const size_t i = base + pt;
     int dot = 0;  // exact in any order: |dot| < 2^31 for kq <= KW_DMAX
     if ((kq & 15) == 0) {
-      // 16-byte loads: the row's bytes in kq/16 loads instead of kq/4
-      const int4* qv = reinterpret_cast<const int4*>(Q + (size_t)i * kq);
-      for (int j = 0; j < words / 4; ++j) {
+      const int4* qv = reinterpret_cast<const int4*>(Q + i * kq);
+#pragma unroll 4
+      for (int j = 0; j < kq / 16; ++j) {
         const int4 v = qv[j];
         dot = __builtin_amdgcn_sdot4(v.x, qc[4 * j], dot, false);
         dot = __builtin_amdgcn_sdot4(v.y, qc[4 * j + 1], dot, false);
@@ -1652,45 +1844,63 @@ __global__ __launch_bounds__(256) void km_pp_round_q8(const float* __restrict__ 
         dot = __builtin_amdgcn_sdot4(v.w, qc[4 * j + 3], dot, false);
       }
     } else {
-      const int* qv = reinterpret_cast<const int*>(Q + (size_t)i * kq);
-      for (int j = 0; j < words; ++j) dot = __builtin_amdgcn_sdot4(qv[j], qc[j], dot, false);
+      const int* qv = reinterpret_cast<const int*>(Q + i * kq);
+      for (int j = 0; j < kq / 4; ++j) dot = __builtin_amdgcn_sdot4(qv[j], qc[j], dot, false);
     }
-    const double sp = scale[i];
-    const double A = sp * sp * (double)qnorm[i], B = sc * sc * qnc, C = sp * sc * (double)dot;
-    const double e2 = A + B - 2.0 * C;
-    const double err = 1e-13 * (A + B + 2.0 * fabs(C));
-    const double e = sqrt(fmax(e2 - err, 0.0)) * (1.0 - 1e-13);
-    const double L = e - (double)delta[i] - dc;
-    const bool keep = isfinite(cur) && L > 0.0 && L * L * (1.0 - gamma) >= (double)cur + 1e-35;
-    exact = !keep;
+    if (!km_pp_keeps(nv_s[pt], (double)scale[i], (double)qnorm[i], (double)delta[i], sc, qnc, dc, (double)dot, gamma))
+      actx[atomicAdd(&n_actx, 1)] = (uint16_t)pt;
   }
-  if (exact) list[atomicAdd(&nlist, 1)] = t;
   __syncthreads();
-  __shared__ float nv_s[Q8_ROWS];
-  nv_s[t] = cur;
-  __syncthreads();
-  const int m = nlist;
-  for (int u = t; u < m; u += 256) {
-    const int tt = list[u];
-    const int ii = blockIdx.x * Q8_ROWS + tt;
-    const float* row = P + (size_t)ii * ldp;
+  // the reference's own sum for the points the centre may capture, eight at a
+  // time: 32 threads square a point's differences (128 coordinates at a time),
+  // one adds them in order
+  const int m3 = n_actx;
+  if (m3 == 0) return;
+  for (int u0 = 0; u0 < m3; u0 += 8) {
+    const int xu = min(u0 + (t >> 5), m3 - 1);
+    const float* row = P + (base + actx[xu]) * ldp;
+    const float* cr = P + (size_t)c * ldp;
     float sum = 0.0f;
-    for (int j = 0; j < dim; ++j) {
-      const float d = row[j] - cs[j];
-      sum += d * d;
+    for (int j0 = 0; j0 < dim; j0 += 128) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = j0 + 32 * e + (t & 31), jc = min(j, dim - 1);
+        const float d = row[jc] - cr[jc];
+        sq[t >> 5][32 * e + (t & 31)] = d * d;
+      }
+      __syncthreads();
+      if (t < 8) {
+        const int w = min(128, dim - j0);
+        int j = 0;
+        for (; j + 4 <= w; j += 4) {
+          const float4 x = *reinterpret_cast<const float4*>(&sq[t][j]);
+          sum += x.x;
+          sum += x.y;
+          sum += x.z;
+          sum += x.w;
+        }
+        for (; j < w; ++j) sum += sq[t][j];
+      }
+      __syncthreads();
     }
-    if (sum < nv_s[tt]) nv_s[tt] = sum;
+    if (t < 8 && u0 + t < m3) {
+      const int pt = actx[u0 + t];
+      if (sum < nv_s[pt]) {
+        nv_s[pt] = sum;
+        ns[base + pt] = sum;
+        near[base + pt] = (uint32_t)chosen;
+        changed[pt / PP_ROWS] = 1;
+      }
+    }
   }
   __syncthreads();
-  const float nv = i < n ? nv_s[t] : 0.0f;
-  if (i < n && nv != cur) {
-    ns[i] = nv;
-    near[i] = (uint32_t)chosen;
-  }
-  const SumCert r = block_cert_256(cert_of(nv), sh);
-  if (t == 0) {
-    ps[blockIdx.x] = r.s;
-    pe[blockIdx.x] = r.e;
+  for (int b = 0; b < SUB; ++b) {
+    if (changed[b] == 0) continue;  // block-uniform
+    const SumCert r = block_cert_256(cert_of(nv_s[b * PP_ROWS + t]), sh);
+    if (t == 0) {
+      ps[blockIdx.x * SUB + b] = r.s;
+      pe[blockIdx.x * SUB + b] = r.e;
+    }
   }
 }
 
@@ -1723,17 +1933,60 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
   __shared__ double s_target;
   __shared__ int s_mode, s_pick, s_block;
   const int t = threadIdx.x;
-  if (*status != 0) return;
-  if (t == 0) rng = *grng;
-  // each thread sums a contiguous run of block partials
+  // the status, the generator and the partials are loaded together: each is a
+  // round trip to memory that other XCDs wrote
+  const int stat = *status;
+  constexpr int RNG_WORDS = sizeof(ChaCha8) / 4;
+  static_assert(sizeof(ChaCha8) % 4 == 0, "copied by words");
+  if (t < RNG_WORDS) reinterpret_cast<uint32_t*>(rng_mem)[t] = reinterpret_cast<const uint32_t*>(grng)[t];
+  // each thread sums a contiguous run of block partials; up to PB of them
+  // come through LDS (coalesced loads, all in flight together; a run starts
+  // one place further on per thread, so that the threads' reads spread over
+  // the banks) and are held for the search below
+  constexpr int PB = 8;
+  __shared__ double sps[1024 * (PB + 1)];
   const int per = (nb + 1023) / 1024;
   const int b0 = min(nb, t * per), b1 = min(nb, (t + 1) * per);
-  double ls = 0.0;
+  double ls = 0.0, pv[PB];
   int le = NO_TERMS;
-  for (int b = b0; b < b1; ++b) {
-    ls += ps[b];
-    le = min(le, pe[b]);
+  if (per == 1) {
+    const int b = min(t, nb - 1);
+    pv[0] = ps[b];
+    const int e = pe[b];
+    if (t < nb) {
+      ls = pv[0];
+      le = e;
+    }
+  } else if (per <= PB) {
+    double lv[PB];
+    int ev[PB];
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+      const int b = min(u * 1024 + t, nb - 1);  // unconditional loads
+      lv[u] = ps[b];
+      ev[u] = pe[b];
+    }
+#pragma unroll
+    for (int u = 0; u < PB; ++u)
+      if (u * 1024 + t < nb) {
+        const int b = u * 1024 + t;
+        sps[b + b / per] = lv[u];
+        le = min(le, ev[u]);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PB; ++u)
+      if (b0 + u < b1) {
+        pv[u] = sps[b0 + t + u];
+        ls += pv[u];
+      }
+  } else {
+    for (int b = b0; b < b1; ++b) {
+      ls += ps[b];
+      le = min(le, pe[b]);
+    }
   }
+  if (stat != 0) return;
   // inclusive scan over the threads: wave scans, then the earlier waves'
   // totals in wave order
   const int lane = t & 63, wv = t >> 6;
@@ -1799,22 +2052,32 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
     // first block whose inclusive prefix reaches the target, then the first
     // point inside it
     double run = before;
-    for (int b = b0; b < b1; ++b) {
-      if (run + ps[b] >= target) {
-        atomicMin(&s_block, b);
-        break;
+    if (per <= PB) {
+      bool found = false;
+#pragma unroll
+      for (int u = 0; u < PB; ++u)
+        if (!found && b0 + u < b1) {
+          if (run + pv[u] >= target) {
+            atomicMin(&s_block, b0 + u);
+            found = true;
+          } else {
+            run += pv[u];
+          }
+        }
+    } else {
+      for (int b = b0; b < b1; ++b) {
+        if (run + ps[b] >= target) {
+          atomicMin(&s_block, b);
+          break;
+        }
+        run += ps[b];
       }
-      run += ps[b];
     }
     __syncthreads();
     const int bb = s_block;
     if (bb < nb) {
-      // prefix before block bb: recomputed by the owning thread's run
-      if (b0 <= bb && bb < b1) {
-        double pre = before;
-        for (int b = b0; b < bb; ++b) pre += ps[b];
-        s_pre = pre;
-      }
+      // prefix before block bb: where the owning thread's run stopped
+      if (b0 <= bb && bb < b1) s_pre = run;
       // the block's PP_ROWS points (the first PP_ROWS / 64 waves): wave
       // scans, then the earlier waves' totals; wtot is free after the scan
       // above (every thread read it before s_block was settled)
@@ -1831,10 +2094,8 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
   __syncthreads();
   const int picked = s_pick;
   for (int j = t; j < dim; j += 1024) row_out[j] = P[(size_t)picked * ldp + j];
-  if (t == 0) {
-    *grng = rng;
-    if (picked_out) *picked_out = picked;
-  }
+  if (t < RNG_WORDS) reinterpret_cast<uint32_t*>(grng)[t] = reinterpret_cast<const uint32_t*>(rng_mem)[t];
+  if (t == 0 && picked_out) *picked_out = picked;
 }
 
 __global__ __launch_bounds__(1024) void km_pp_pick(const float* __restrict__ P, int ldp, int n, int dim,
@@ -1889,19 +2150,22 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   const int vec4 = (ldp % 4 == 0 && dim % 4 == 0 && ((uintptr_t)P & 15) == 0) ? 1 : 0;
   hipLaunchKernelGGL(km_pp_round, dim3(nb), dim3(256), 0, s, P, ldp, (int)n, dim, cents, ns.p, 1, ps.p, pe.p, vec4);
   PXG_HIP(hipGetLastError());
-  // rounds after the first over the certified int8 copy (dim >= 32; for
-  // narrower points the copy saves little of each row's bytes)
-  const bool q8 = dim >= 32 && dim <= KW_DMAX && k > 1 && Q8_ROWS == PP_ROWS;
-  const int kq = (dim + 3) / 4 * 4;
+  // rounds after the first over the certified 4-bit and int8 copies (dim >=
+  // 32; for narrower points the copies save little of each row's bytes)
+  const bool q8 = dim >= 32 && dim <= KW_DMAX && k > 1;
+  const int kq = (dim + 3) / 4 * 4, words4 = (dim + 31) / 32 * 4;
   DevBuf<int8_t> Q(q8 ? n * kq : 0);
   DevBuf<float> qscale(q8 ? n : 0), qdelta(q8 ? n : 0);
   DevBuf<int> qnorm(q8 ? n : 0), picked(1);
+  // four blocks of points per workgroup once that still gives every CU two
+  const bool wide = nb >= 4 * 512;
+  DevBuf<uint32_t> q4(q8 && wide ? n * words4 : 0), qmeta4(q8 ? n : 0);
   DevBuf<uint32_t> near(q8 ? n : 0);  // every distance is to centre 0 so far
-  DevBuf<float> dcc(q8 ? k : 0);
+  DevBuf<float> tnear(q8 ? k : 0);
   if (q8) {
     PXG_HIP(hipMemsetAsync(near.p, 0, n * 4, s));
     hipLaunchKernelGGL(km_q8_prep, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, P, ldp, (int)n, dim, kq, Q.p,
-                       qscale.p, qdelta.p, qnorm.p);
+                       qscale.p, qdelta.p, qnorm.p, words4, wide ? q4.p : nullptr, qmeta4.p);
     PXG_HIP(hipGetLastError());
   }
   const double gamma = (double)(dim + 4) * 0x1p-24 * 1.01;
@@ -1911,11 +2175,27 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
                        flags.p, flags.p + 1, picked.p);
     if (chosen + 1 < k) {
       if (q8) {
-        hipLaunchKernelGGL(km_pp_cdist, dim3((unsigned)((chosen + 63) / 64)), dim3(256), 0, s, (const float*)cents,
-                           dim, (int)chosen, dcc.p);
-        hipLaunchKernelGGL(km_pp_round_q8, dim3(nb), dim3(256), 0, s, P, ldp, (int)n, dim, (const int8_t*)Q.p, kq,
-                           (const float*)qscale.p, (const float*)qdelta.p, (const int*)qnorm.p, (const int*)picked.p,
-                           ns.p, ps.p, pe.p, gamma, near.p, (const float*)dcc.p, (int)chosen);
+        hipLaunchKernelGGL(km_pp_cdist, dim3((unsigned)((chosen + 15) / 16)), dim3(256), 0, s, (const float*)cents,
+                           dim, (int)chosen, gamma, tnear.p);
+#define PXG_PP(LPV, SUBV)                                                                                            \
+  hipLaunchKernelGGL((km_pp_round_q8<LPV, SUBV>), dim3((nb + SUBV - 1) / SUBV), dim3(256), 0, s, P, ldp, (int)n, dim, \
+                     (const int8_t*)Q.p, kq, (const float*)qscale.p, (const float*)qdelta.p, (const int*)qnorm.p,    \
+                     (const uint32_t*)q4.p, (const uint32_t*)qmeta4.p, words4, (const int*)picked.p, ns.p, ps.p,     \
+                     pe.p, gamma, near.p, (const float*)tnear.p, (int)chosen)
+        if (!wide) {
+          if (dim <= 256) PXG_PP(8, 1); else PXG_PP(16, 1);
+        } else if (dim <= 32) {
+          PXG_PP(1, 4);
+        } else if (dim <= 64) {
+          PXG_PP(2, 4);
+        } else if (dim <= 128) {
+          PXG_PP(4, 4);
+        } else if (dim <= 256) {
+          PXG_PP(8, 4);
+        } else {
+          PXG_PP(16, 4);
+        }
+#undef PXG_PP
       } else
         hipLaunchKernelGGL(km_pp_round, dim3(nb), dim3(256), 0, s, P, ldp, (int)n, dim, c, ns.p, 0, ps.p, pe.p,
                            vec4);

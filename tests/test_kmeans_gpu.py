@@ -422,3 +422,20 @@ def test_lloyd_split_any_alignment(gpu, dim):
     want = orc.kmeans_lloyd(pts, init, 6)
     assert np.array_equal(np.asarray(want[0], np.float32).reshape(cents.shape).view(np.uint32), cents.view(np.uint32))
     assert np.array_equal(want[1], assign) and want[2] == inertia and want[3] == its
+
+
+@pytest.mark.parametrize("dim,k", [(32, 24), (60, 24), (100, 20), (200, 10), (270, 8)])
+def test_kmeans_pp_four_bit_rounds(gpu, dim, k):
+    """Enough points (2048 blocks of 256) for the rounds over the 4-bit copy, at
+    each of its lane counts: tight clusters, coarse copies (one large
+    coordinate), duplicates and far outliers; the seeds are the oracle's bits."""
+    rng = np.random.default_rng(dim)
+    n = 524_288 + 77
+    pts = rng.standard_normal((15, dim)).astype(np.float32)[rng.integers(0, 15, n)]
+    pts += 0.05 * rng.standard_normal((n, dim)).astype(np.float32)
+    pts[::9, 3] += np.float32(300.0)
+    pts[1::9] = pts[4]
+    pts[2::5001] *= np.float32(1e3)
+    got = gpu.kmeans_pp(pts, k, 11)
+    want = orc.kmeans_pp(pts, k, 11)
+    assert np.array_equal(bits(got), bits(want))
