@@ -412,6 +412,87 @@ __device__ inline uint64_t block_radix_select_each(Each each, int K, int* hist, 
   return prefix;
 }
 
+// block_radix_select_each for 64-bit keys whose smallest and largest (lo and
+// hi: each thread's own, KEY_MAX and 0 where it has none) are combined first:
+// the digits start at the highest bit in which the keys differ, so that keys
+// that share their leading bits (distances of one neighbourhood) need one or
+// two passes instead of four or five. sh: 4 u64, hist: 256 ints.
+template <int NT, class Each>
+__device__ inline uint64_t block_radix_select_range(Each each, uint64_t lo, uint64_t hi, int K, int* hist,
+                                                    uint64_t* sh) {
+  __shared__ uint64_t wlo[NT / WAVE], whi[NT / WAVE];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t a = shfl_xor64(lo, o), b = shfl_xor64(hi, o);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  const int lane = threadIdx.x & (WAVE - 1);
+  if (lane == 0) {
+    wlo[threadIdx.x >> 6] = lo;
+    whi[threadIdx.x >> 6] = hi;
+  }
+  if (threadIdx.x == 0) sh[3] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / WAVE; ++w) {
+    lo = wlo[w] < lo ? wlo[w] : lo;
+    hi = whi[w] > hi ? whi[w] : hi;
+  }
+  if (lo >= hi) return hi;  // one key
+  int top = 64 - __builtin_clzll(lo ^ hi);  // bits above are shared
+  uint64_t mask = top == 64 ? 0 : ~0ull << top, prefix = lo & mask;
+  int remaining = K;
+  while (top > 0) {
+    const int shift = top > 8 ? top - 8 : 0, width = top - shift;
+    for (int i = threadIdx.x; i < 256; i += NT) hist[i] = 0;
+    __syncthreads();
+    each([&](uint64_t x) {
+      if ((x & mask) == prefix) atomicAdd(&hist[(int)((x >> shift) & 255) & ((1 << width) - 1)], 1);
+    });
+    __syncthreads();
+    if (threadIdx.x < WAVE) {
+      // the digit whose bins' running sum reaches `remaining`: 4 bins per lane
+      const int c0 = hist[lane * 4], c1 = hist[lane * 4 + 1], c2 = hist[lane * 4 + 2], c3 = hist[lane * 4 + 3];
+      const int s = c0 + c1 + c2 + c3;
+      int incl = s;
+      for (int o = 1; o < WAVE; o <<= 1) {
+        const int u = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += u;
+      }
+      const int e0 = incl - s, e1 = e0 + c0, e2 = e1 + c1, e3 = e2 + c2;
+      int d = -1, before = 0, cnt = 0;
+      if (remaining > e0 && remaining <= e1) { d = lane * 4; before = e0; cnt = c0; }
+      else if (remaining > e1 && remaining <= e2) { d = lane * 4 + 1; before = e1; cnt = c1; }
+      else if (remaining > e2 && remaining <= e3) { d = lane * 4 + 2; before = e2; cnt = c2; }
+      else if (remaining > e3 && remaining <= e3 + c3) { d = lane * 4 + 3; before = e3; cnt = c3; }
+      if (d >= 0) {
+        sh[0] = (uint64_t)d;
+        sh[1] = (uint64_t)before;
+        sh[2] = (uint64_t)cnt;
+      }
+    }
+    __syncthreads();
+    remaining -= (int)sh[1];
+    const int cnt = (int)sh[2];
+    prefix |= sh[0] << shift;
+    mask = shift == 0 ? ~0ull : ~0ull << shift;
+    __syncthreads();
+    if (cnt == remaining && shift > 0) {
+      // all keys of the bin are wanted: the K-th smallest is their largest
+      uint64_t m = 0;
+      each([&](uint64_t x) {
+        if ((x & mask) == prefix && x > m) m = x;
+      });
+      if (m) atomicMax((unsigned long long*)&sh[3], (unsigned long long)m);
+      __syncthreads();
+      return sh[3];
+    }
+    top = shift;
+  }
+  return prefix;
+}
+
 template <class Get, int BITS = 64, int PER = 0>
 __device__ inline uint64_t block_radix_select(Get get, int n, int K, int* hist, uint64_t* sh) {
   static_assert(BITS % 8 == 0 && BITS <= 64, "whole-byte digits");

@@ -71,6 +71,7 @@ constexpr int FB_K = 32;    // k-slice staged in LDS
 // consecutive rows touch 8 different groups of banks.
 constexpr int MARGIN = 16;  // k' = k + MARGIN
 constexpr int FAST_KMAX = 256;
+constexpr int FLAT_MAX_SPLITS = 512;
 
 // ---------------------------------------------------------------------------
 // 2. MFMA distance GEMM fused with a per-query top-k' filter
@@ -109,7 +110,7 @@ __device__ __forceinline__ void vm_wait0() { asm volatile("s_waitcnt vmcnt(0)" :
 
 template <int CAP>
 __device__ inline void compact_row_w(uint64_t* __restrict__ base, int c, int Kp, int lane, uint64_t* thr_row,
-                                     float* thrf_row, int* cnt_row, unsigned long long* gthr_row, bool final_pass) {
+                                     float* thrf_row, int* cnt_row, unsigned long long* gthr_row) {
   constexpr int E = CAP / WAVE;
   uint64_t kk[E];
 #pragma unroll
@@ -122,7 +123,7 @@ __device__ inline void compact_row_w(uint64_t* __restrict__ base, int c, int Kp,
   for (int e = 0; e < E; ++e) {
     const int idx = lane * E + e;
     if (idx < Kp) base[idx] = kk[e];
-    if (idx == Kp - 1 && !final_pass) {
+    if (idx == Kp - 1) {
       *thr_row = kk[e];
       *thrf_row = key_float((uint32_t)(kk[e] >> 32));
       // this split keeps Kp candidates at or below kk[e] to the end, so no
@@ -130,7 +131,7 @@ __device__ inline void compact_row_w(uint64_t* __restrict__ base, int c, int Kp,
       if (kk[e] != KEY_MAX) atomicMin(gthr_row, (unsigned long long)kk[e]);
     }
   }
-  if (lane == 0 && !final_pass) *cnt_row = Kp;
+  if (lane == 0) *cnt_row = Kp;
 }
 
 // Keep the Kp smallest of a row's c buffered keys, sorted, KEY_MAX padded to
@@ -138,16 +139,16 @@ __device__ inline void compact_row_w(uint64_t* __restrict__ base, int c, int Kp,
 // holds max(c, Kp), up to the buffer's CAP.
 template <int CAP>
 __device__ __attribute__((noinline)) void compact_row(uint64_t* __restrict__ base, int c, int Kp, int lane, uint64_t* thr_row,
-                                   float* thrf_row, int* cnt_row, unsigned long long* gthr_row, bool final_pass) {
+                                   float* thrf_row, int* cnt_row, unsigned long long* gthr_row) {
   const int need = c > Kp ? c : Kp;
   if (need <= 64)
-    compact_row_w<64>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row, final_pass);
+    compact_row_w<64>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row);
   else if (need <= 128 && CAP >= 128)
-    compact_row_w<(CAP >= 128 ? 128 : CAP)>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row, final_pass);
+    compact_row_w<(CAP >= 128 ? 128 : CAP)>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row);
   else if (need <= 256 && CAP >= 256)
-    compact_row_w<(CAP >= 256 ? 256 : CAP)>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row, final_pass);
+    compact_row_w<(CAP >= 256 ? 256 : CAP)>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row);
   else
-    compact_row_w<CAP>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row, final_pass);
+    compact_row_w<CAP>(base, c, Kp, lane, thr_row, thrf_row, cnt_row, gthr_row);
 }
 
 // The first tile of a seeded split in the full pass: the keys the seeding
@@ -527,26 +528,16 @@ __global__ __launch_bounds__(256, 2) void flat_mfma_candidates(
         full &= full - 1;
         const int row = wid + 4 * l;
         compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP, __builtin_amdgcn_readlane(c_l, l), Kp,
-                         lane, &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row, false);
+                         lane, &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row);
       }
       __syncthreads();
     }
   }
   // Seeding pass: each row has left its one tile's FB_N distance parts.
   if constexpr (SEED) return;
-  // Final: every row leaves Kp keys, its Kp smallest (KEY_MAX padded). The
-  // merge reads them as a set, so a row with at most Kp keys is only padded;
-  // a fuller one is sorted down to Kp.
-  for (int row = wid; row < FB_M; row += 4) {
-    if (q0 + row >= nq) continue;
-    uint64_t* base = cand + ((size_t)(q0 + row) * S + split) * CAP;
-    const int c = cnt[row];
-    if (c <= Kp) {
-      for (int i = c + lane; i < Kp; i += WAVE) base[i] = KEY_MAX;
-    } else {
-      compact_row<CAP>(base, c, Kp, lane, &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row, true);
-    }
-  }
+  // Final: every row leaves its keys (at most CAP - FB_N after the last
+  // tile's compaction) and their number in the buffer's last entry.
+  if (tid < FB_M && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP + CAP - 1] = (uint64_t)cnt[tid];
 }
 
 #include "flat_split.hpp"
@@ -616,202 +607,206 @@ __global__ __launch_bounds__(64) void flat_seed_threshold2_wave(const uint64_t* 
   if (lane == 0 && hi != 0xFFFFFFFFull) atomicMin(gthr + q, (unsigned long long)((hi << 32) | 0xFFFFFFFFull));
 }
 
-constexpr int MERGE_MAXP = 512;
+constexpr int MERGE_MAXP = 512;  // k' at most, as a power of two
 
 // The certificate of one query's merge. Every candidate outside the
 // selection has approx >= approx(pivot), hence exact >= approx(pivot) - eps;
 // the k-th exact distance (the high word of `kth`) must be strictly below
-// that for the selection to contain the exact top-k. q_add: the query's own
-// term where the candidates' scores leave it out, else 0.
-__device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric, float qnv, float maxnorm, float eps_c,
-                                       int dim, float q_add) {
+// that for the selection to contain the exact top-k. SPLIT: the scores are
+// the split pass's, which leave out the query's own term q_add.
+//
+// eps, in units of 2^-24, with q and x the query's and the largest row norm
+// and s = q + x:
+//   f32 pass: 4 d s^2 (Euclidean), 4 d q x (else), generous for both the MFMA
+//     sum and the reference's.
+//   split pass: the products' 3.75 d + 6 (split.hpp) times 2 q x or q x; the
+//     reference's own sum, d / 8 + 5 of the distance (at most s^2, or q x);
+//     for Euclidean also the two squared norms' d / 8 + 3 each and two
+//     roundings of at most s^2. The norms are themselves within d / 8 + 3,
+//     covered by the factor 1.01.
+// 2.4e-7 covers the roundings of 1 - dot.
+__device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric, float qnv, float maxnorm, int dim,
+                                       bool split, float q_add) {
   const float ak = key_float((uint32_t)(pivot >> 32)) + q_add;
   const float dk = key_float((uint32_t)(kth >> 32));
+  constexpr float U = 5.9604645e-08f;
+  const float d = (float)dim, qx = qnv * maxnorm, s = qnv + maxnorm;
   float eps;
-  if (metric == 0) {
-    const float s = qnv + maxnorm;
-    eps = eps_c * (float)dim * 5.9604645e-08f * s * s;
+  if (split) {
+    const float d8 = 0.125f * d;
+    eps = metric == 0 ? 1.01f * U * ((7.5f * d + 12.0f) * qx + (d8 + 3.0f) * (qnv * qnv + maxnorm * maxnorm) +
+                                     (d8 + 7.0f) * s * s)
+                      : 1.01f * U * (3.75f * d + 6.0f + d8 + 6.0f) * qx + 2.4e-7f;
   } else {
-    eps = eps_c * (float)dim * 5.9604645e-08f * qnv * maxnorm + 2.4e-7f;
+    eps = metric == 0 ? 4.0f * d * U * s * s : 4.0f * d * U * qx + 2.4e-7f;
   }
   eps += 1e-30f;
   return dk < ak - eps;
 }
 
-__global__ __launch_bounds__(256) void flat_merge_rescore(
-    const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const float* __restrict__ Qp, int ld, int dim,
-    int metric, const float* __restrict__ X, const uint32_t* __restrict__ rank, const uint32_t* __restrict__ rank_slot,
-    const uint64_t* __restrict__ ids, const float* __restrict__ qn, const float* __restrict__ q_add, float maxnorm,
-    float eps_c, uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
+// Per query: the k' smallest approximate keys of its S candidate lists
+// (list s: the first cand[s * CAP + CAP - 1] entries of its buffer, unsorted),
+// rescored exactly and sorted; see the file's head.
+//
+// At least k' keys of the lists are at or below the query's shared threshold
+// (its seed, or the k'-th key some split published), so only those can be
+// among the k' smallest: they are gathered into LDS (16 threads per list, the
+// first 16 entries of four lists loaded together) and selected there. More
+// than LM of them are selected from memory instead.
+// What bounds it: round trips to memory (counts, keys, rows, ids), five to
+// seven of them; 313 queries of 170 lists and k' = 116 (about 1600 gathered
+// keys): 225 us when every list was padded to k' keys and all 19,720 were
+// selected over, 31 us here; 1000 queries of 61 lists, k' = 26: 14.6 -> 11.8
+// us; 48 queries of 195 lists, k' = 26: 16.2 -> 10.6 us.
+template <int NT, int LM>
+__global__ __launch_bounds__(NT) void flat_merge(
+    const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const unsigned long long* __restrict__ gthr,
+    const float* __restrict__ Qp, int ld, int dim, int metric, const float* __restrict__ X,
+    const uint32_t* __restrict__ rank, const uint32_t* __restrict__ rank_slot, const uint64_t* __restrict__ ids,
+    const float* __restrict__ qn, const float* __restrict__ q_add, float maxnorm,
+    uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
     int* __restrict__ flag_list, int* __restrict__ flag_count, size_t ldo) {
-  const int q = blockIdx.x;
+  constexpr int NG = NT / 16;  // groups of 16 threads
+  constexpr int PER = LM / NT;
+  __shared__ uint64_t lst[LM];
+  __shared__ uint16_t scnt[FLAT_MAX_SPLITS];
   __shared__ int hist[256];
   __shared__ uint64_t sh[4];
   __shared__ uint64_t sel[MERGE_MAXP];
-  __shared__ int n_sel;
-  __shared__ int n_valid;
+  __shared__ uint32_t rslot[WAVE];
+  __shared__ int n_list, n_valid, n_sel;
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & (WAVE - 1);
   const uint64_t* base = cand + (size_t)q * S * CAP;
-  const int n = S * Kp;
-  auto get = [&](int i) -> uint64_t { return base[(size_t)(i / Kp) * CAP + (i % Kp)]; };
-
-  if (threadIdx.x == 0) {
-    n_valid = 0;
-    n_sel = 0;
-  }
+  const uint64_t g = gthr[q];
+  if (tid == 0) n_list = n_valid = n_sel = 0;
   __syncthreads();
   int local = 0;
-  // eight keys per thread per step, loaded together before any is used
-  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * blockDim.x) {
-    uint64_t x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = get(min(i0 + u * (int)blockDim.x, n - 1));  // unconditional loads
-#pragma unroll
-    for (int u = 0; u < 8; ++u) local += (i0 + u * (int)blockDim.x < n && x[u] != KEY_MAX) ? 1 : 0;
+  for (int s = tid; s < S; s += NT) {
+    const int c = (int)(uint32_t)base[(size_t)s * CAP + CAP - 1];
+    scnt[s] = (uint16_t)c;
+    local += c;
   }
-  atomicAdd(&n_valid, local);
+  if (local) atomicAdd(&n_valid, local);
   __syncthreads();
   const int valid = n_valid;
   const int ksel = min(Kp, valid);
   if (ksel == 0) {
-    if (threadIdx.x == 0) out_count[q] = 0;
+    if (tid == 0) out_count[q] = 0;
     return;
   }
-  const uint64_t pivot = n <= 16 * (int)blockDim.x ? block_radix_select<decltype(get), 64, 16>(get, n, ksel, hist, sh)
-                         : n <= 40 * (int)blockDim.x ? block_radix_select<decltype(get), 64, 40>(get, n, ksel, hist, sh)
-                                         : block_radix_select(get, n, ksel, hist, sh);
-  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * blockDim.x) {
-    uint64_t x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = get(min(i0 + u * (int)blockDim.x, n - 1));  // unconditional loads
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (i0 + u * (int)blockDim.x < n && x[u] <= pivot && x[u] != KEY_MAX) {
-        const int p = atomicAdd(&n_sel, 1);
-        sel[p] = x[u];
-      }
-  }
-  __syncthreads();
-  // rescore: 8 threads per candidate
-  const int g = threadIdx.x & 7, grp = threadIdx.x >> 3;
-  const float* qv = Qp + (size_t)q * ld;
-  for (int c = grp; c < ksel; c += 32) {
-    const uint32_t slot = (uint32_t)sel[c];
-    const float d = dist_group8_rt(metric, qv, X + (size_t)slot * ld, dim, g);
-    if (g == 0) sel[c] = ((uint64_t)ord_key(d) << 32) | rank[slot];
-  }
-  __syncthreads();
-  int P = 1;
-  while (P < ksel) P <<= 1;
-  for (int i = ksel + threadIdx.x; i < P; i += blockDim.x) sel[i] = KEY_MAX;
-  __syncthreads();
-  block_bitonic_sort(sel, P);
-  const int kout = min(k, ksel);
-  for (int i = threadIdx.x; i < kout; i += blockDim.x) {
-    const uint64_t key = sel[i];
-    const uint32_t slot = rank_slot[(uint32_t)key];
-    out_ids[(size_t)q * ldo + i] = ids[slot];
-    out_d[(size_t)q * ldo + i] = key_float((uint32_t)(key >> 32));
-  }
-  if (threadIdx.x == 0) {
-    out_count[q] = kout;
-    if (valid >= Kp && !merge_certified(pivot, sel[kout - 1], metric, qn[q], maxnorm, eps_c, dim,
-                                         q_add != nullptr ? q_add[q] : 0.0f)) {
-      const int p = atomicAdd(flag_count, 1);
-      flag_list[p] = q;
-    }
-  }
-}
-
-// flat_merge_rescore for a query whose S * Kp keys fit PER per thread of an
-// NT-thread block and whose Kp fits one wavefront. Each key is read once into
-// registers, and the count, the select and the gather use that copy; one
-// wavefront sorts the rescored keys with their slots in registers. Same
-// results as the general kernel: the same selection, rescore arithmetic and
-// (distance, rank) order.
-template <int NT, int PER>
-__global__ __launch_bounds__(NT) void flat_merge_rescore_reg(
-    const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const float* __restrict__ Qp, int ld, int dim,
-    int metric, const float* __restrict__ X, const uint32_t* __restrict__ rank, const uint64_t* __restrict__ ids,
-    const float* __restrict__ qn, const float* __restrict__ q_add, float maxnorm, float eps_c,
-    uint64_t* __restrict__ out_ids, float* __restrict__ out_d, uint32_t* __restrict__ out_count,
-    int* __restrict__ flag_list, int* __restrict__ flag_count, size_t ldo) {
-  const int q = blockIdx.x;
-  const int lane = threadIdx.x & (WAVE - 1);
-  __shared__ int hist[256];
-  __shared__ uint64_t sh[4];
-  __shared__ uint64_t sel[WAVE];
-  __shared__ uint64_t rkey[WAVE];
-  __shared__ uint32_t rslot[WAVE];
-  __shared__ int n_sel;
-  __shared__ int n_valid;
-  const uint64_t* base = cand + (size_t)q * S * CAP;
-  const int n = S * Kp;
-  if (threadIdx.x == 0) {
-    n_valid = 0;
-    n_sel = 0;
-  }
-  uint64_t x[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = min((int)threadIdx.x + u * NT, n - 1);  // unconditional loads
-    x[u] = base[(size_t)(i / Kp) * CAP + i % Kp];
-  }
-  int wcount = 0;
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    if ((int)threadIdx.x + u * NT >= n) x[u] = KEY_MAX;
-    wcount += __popcll(__ballot(x[u] != KEY_MAX));
-  }
-  __syncthreads();  // the counters are set
-  if (lane == 0) atomicAdd(&n_valid, wcount);
-  __syncthreads();
-  const int valid = n_valid;
-  const int ksel = min(Kp, valid);
-  if (ksel == 0) {
-    if (threadIdx.x == 0) out_count[q] = 0;
-    return;
-  }
-  auto each = [&](auto f) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u)
-      if (x[u] != KEY_MAX) f(x[u]);
+  // appends the calling lanes' keys at or below the threshold, one counter
+  // update per wave
+  auto push = [&](uint64_t x) {
+    const uint64_t m = __ballot(x <= g && x != KEY_MAX);
+    if (m == 0) return;
+    const int leader = __builtin_ctzll(m);
+    int at = 0;
+    if (lane == leader) at = atomicAdd(&n_list, __popcll(m));
+    at = __builtin_amdgcn_readlane(at, leader) + __popcll(m & ((1ull << lane) - 1));
+    if (((m >> lane) & 1) != 0 && at < LM) lst[at] = x;
   };
-  const uint64_t pivot = block_radix_select_each<64>(each, ksel, hist, sh);
-  // keys are distinct (one per row), so exactly ksel <= WAVE of them are
-  // <= pivot (the bound on the write only guards the array)
+  const int gl = tid & 15, grp = tid >> 4;
+  for (int s0 = 0; s0 < S; s0 += 4 * NG) {  // uniform, so that every lane takes part in push
+    uint64_t x[4];
+    int c[4], most = 0;
 #pragma unroll
-  for (int u = 0; u < PER; ++u)
-    if (x[u] <= pivot && x[u] != KEY_MAX) {
-      const int p = atomicAdd(&n_sel, 1);
-      if (p < WAVE) sel[p] = x[u];
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + u * NG + grp;
+      c[u] = s < S ? scnt[s] : 0;
+      x[u] = base[(size_t)min(s, S - 1) * CAP + min(gl, CAP - 1)];  // unconditional loads
+      most = max(most, c[u]);
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) push(gl < c[u] ? x[u] : KEY_MAX);
+    for (int j0 = 16; __ballot(j0 < most) != 0; j0 += 16) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = min(s0 + u * NG + grp, S - 1);
+        x[u] = j0 + gl < c[u] ? base[(size_t)s * CAP + j0 + gl] : KEY_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) push(x[u]);
+    }
+  }
   __syncthreads();
-  // rescore: 8 threads per candidate
-  const int g = threadIdx.x & 7, grp = threadIdx.x >> 3;
+  const int n = n_list;
+  uint64_t pivot;
+  if (n <= LM) {
+    // the digits start at the highest bit in which the keys differ
+    uint64_t v[PER], lo = KEY_MAX, hi = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      v[j] = tid + j * NT < n ? lst[tid + j * NT] : KEY_MAX;
+      if (v[j] != KEY_MAX) {
+        lo = min(lo, v[j]);
+        hi = max(hi, v[j]);
+      }
+    }
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (v[j] != KEY_MAX) f(v[j]);
+    };
+    pivot = block_radix_select_range<NT>(each, lo, hi, ksel, hist, sh);
+    each([&](uint64_t x) {
+      if (x <= pivot) sel[atomicAdd(&n_sel, 1) & (MERGE_MAXP - 1)] = x;
+    });
+  } else {
+    auto each = [&](auto f) {
+      for (int s = grp; s < S; s += NG)
+        for (int j = gl; j < (int)scnt[s]; j += 16) {
+          const uint64_t x = base[(size_t)s * CAP + j];
+          if (x <= g) f(x);
+        }
+    };
+    pivot = block_radix_select_each<64>(each, ksel, hist, sh);
+    each([&](uint64_t x) {
+      if (x <= pivot) sel[atomicAdd(&n_sel, 1) & (MERGE_MAXP - 1)] = x;
+    });
+  }
+  __syncthreads();
+  // rescore: 8 threads per candidate (keys are distinct, one per row, so
+  // exactly ksel of them are at or below the pivot)
   const float* qv = Qp + (size_t)q * ld;
-  for (int c = grp; c < ksel; c += NT / 8) {
+  for (int c = tid >> 3; c < ksel; c += NT / 8) {
     const uint32_t slot = (uint32_t)sel[c];
-    const float d = dist_group8_rt(metric, qv, X + (size_t)slot * ld, dim, g);
-    if (g == 0) {
-      rkey[c] = ((uint64_t)ord_key(d) << 32) | rank[slot];
-      rslot[c] = slot;
+    const float d = dist_group8_rt(metric, qv, X + (size_t)slot * ld, dim, tid & 7);
+    if ((tid & 7) == 0) {
+      if (Kp <= WAVE) rslot[c] = slot;
+      sel[c] = ((uint64_t)ord_key(d) << 32) | rank[slot];
     }
   }
   __syncthreads();
-  if (threadIdx.x >= WAVE) return;
-  uint64_t key = lane < ksel ? rkey[lane] : KEY_MAX;
-  uint32_t slot = lane < ksel ? rslot[lane] : 0;
-  wave_sort_kv64(key, slot, lane);
   const int kout = min(k, ksel);
-  if (lane < kout) {
-    out_ids[(size_t)q * ldo + lane] = ids[slot];
-    out_d[(size_t)q * ldo + lane] = key_float((uint32_t)(key >> 32));
+  uint64_t kth;
+  if (Kp <= WAVE) {
+    // one wavefront sorts the keys with their slots
+    if (tid >= WAVE) return;
+    uint64_t key = lane < ksel ? sel[lane] : KEY_MAX;
+    uint32_t slot = lane < ksel ? rslot[lane] : 0;
+    wave_sort_kv64(key, slot, lane);
+    if (lane < kout) {
+      out_ids[(size_t)q * ldo + lane] = ids[slot];
+      out_d[(size_t)q * ldo + lane] = key_float((uint32_t)(key >> 32));
+    }
+    kth = (uint64_t)(uint32_t)__shfl((int)(uint32_t)(key >> 32), kout - 1, WAVE) << 32;
+  } else {
+    int P = 1;
+    while (P < ksel) P <<= 1;
+    for (int i = ksel + tid; i < P; i += NT) sel[i] = KEY_MAX;
+    __syncthreads();
+    block_bitonic_sort(sel, P);
+    for (int i = tid; i < kout; i += NT) {
+      const uint64_t key = sel[i];
+      out_ids[(size_t)q * ldo + i] = ids[rank_slot[(uint32_t)key]];
+      out_d[(size_t)q * ldo + i] = key_float((uint32_t)(key >> 32));
+    }
+    kth = sel[kout - 1];
   }
-  const uint32_t kth_hi = (uint32_t)__shfl((int)(uint32_t)(key >> 32), kout - 1, WAVE);
-  if (lane == 0) {
+  if (tid == 0) {
     out_count[q] = kout;
-    if (valid >= Kp && !merge_certified(pivot, (uint64_t)kth_hi << 32, metric, qn[q], maxnorm, eps_c, dim,
-                                         q_add != nullptr ? q_add[q] : 0.0f)) {
+    if (valid >= Kp && !merge_certified(pivot, kth, metric, qn[q], maxnorm, dim, q_add != nullptr,
+                                        q_add != nullptr ? q_add[q] : 0.0f)) {
       const int p = atomicAdd(flag_count, 1);
       flag_list[p] = q;
     }
@@ -1045,7 +1040,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     // split pass
     const int QT = !split || nq > 64 ? 4 : nq > 32 ? 2 : 1;
     const int QB = (int)((nq + 32 * QT - 1) / (32 * QT));
-    int S = std::max(1, std::min(512 / QB, std::max(1, tiles / 4)));
+    int S = std::max(1, std::min(FLAT_MAX_SPLITS / QB, std::max(1, tiles / 4)));
     // a fixed scratch may hold fewer splits (the results do not depend on S)
     const size_t fit = sc.room() / per_split_bytes;
     if (fit == 0) (void)sc.get(6, per_split_bytes);  // raises the capacity error
@@ -1087,12 +1082,14 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     };
     if (seeded) {
       candidates(std::true_type{});
-      // the splits' pairs when they are many against Kp (and fit the
-      // select's 16 words per thread), else every seeding word
+      // the splits' pairs when there are at least as many splits as Kp (and
+      // they fit the select's 16 words per thread), else every seeding word.
+      // With one of the Kp best per split on average, a tenth of them lie
+      // third or later in their split, so the bound is about a tenth looser.
       if (2 * S >= 4 * Kp && S <= WAVE)
         hipLaunchKernelGGL(flat_seed_threshold2_wave, dim3((unsigned)nq), dim3(64), 0, s, (const uint64_t*)cand, S,
                            CAP, Kp, gthr);
-      else if (2 * S >= 4 * Kp && 2 * S <= 16 * 64)
+      else if (S >= Kp && 2 * S <= 16 * 64)
         hipLaunchKernelGGL(flat_seed_threshold2, dim3((unsigned)nq), dim3(64), 0, s, (const uint64_t*)cand, S, CAP,
                            Kp, gthr);
       else
@@ -1102,21 +1099,19 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     }
     candidates(std::false_type{});
     tm.mark(2);
-    const size_t nkeys = (size_t)S * Kp;
     const float* q_add = split ? qb : nullptr;
-    const float eps_c = split ? SPLIT_EPS_C : 4.0f;
-    if (nkeys <= 8 * 256 && Kp <= WAVE)
-      hipLaunchKernelGGL((flat_merge_rescore_reg<256, 8>), dim3((unsigned)nq), dim3(256), 0, s, cand, S, CAP, Kp,
-                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, q_add, maxnorm, eps_c, d_oid,
-                         d_od, d_oc, flag_list, flag_count, ldo);
-    else if (nkeys <= 16 * 1024 && Kp <= WAVE)
-      hipLaunchKernelGGL((flat_merge_rescore_reg<1024, 16>), dim3((unsigned)nq), dim3(1024), 0, s, cand, S, CAP, Kp,
-                         (int)kq, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p, d_ids.p, qn, q_add, maxnorm, eps_c, d_oid,
-                         d_od, d_oc, flag_list, flag_count, ldo);
+#define PXG_MERGE(NTV, LMV)                                                                                        \
+  hipLaunchKernelGGL((flat_merge<NTV, LMV>), dim3((unsigned)nq), dim3(NTV), 0, s, (const uint64_t*)cand, S, CAP, Kp, \
+                     (int)kq, (const unsigned long long*)gthr, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p,     \
+                     ranks.rank_slot.p, d_ids.p, qn, q_add, maxnorm, d_oid, d_od, d_oc, flag_list, flag_count, \
+                     ldo)
+    // the lists hold S * Kp keys at or below a query's threshold at most, far
+    // fewer where the seed is tight; the small form fits four blocks per CU
+    if ((size_t)S * Kp <= 8192 && Kp <= WAVE)
+      PXG_MERGE(256, 4096);
     else
-      hipLaunchKernelGGL(flat_merge_rescore, dim3((unsigned)nq), dim3(256), 0, s, cand, S, CAP, Kp, (int)kq, Qp,
-                         (int)ld, (int)dim, metric, X.p, ranks.rank.p, ranks.rank_slot.p, d_ids.p, qn, q_add, maxnorm, eps_c,
-                         d_oid, d_od, d_oc, flag_list, flag_count, ldo);
+      PXG_MERGE(512, 8192);
+#undef PXG_MERGE
     PXG_HIP(hipGetLastError());
   } else {
     hipLaunchKernelGGL(iota_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, flag_list, (int)nq,

@@ -10,11 +10,6 @@
 
 #include "split.hpp"
 
-// Certificate constant of the split pass: |approximation - exact| is below
-// SPLIT_EPS_C * d * 2^-24 * |q||x|: the product's 7.13 d + 6, and the
-// reference's 8-lane sum's d / 8 + 3, for d >= 64.
-constexpr float SPLIT_EPS_C = 8.0f;
-
 // flat_prep_search_queries for the split pass: also each query's parts, as
 // records of 32 hi then 32 lo halves per 32 dimensions (nK records per query,
 // zeros past dim), and the factor cq that takes an accumulated product back
@@ -373,20 +368,11 @@ __global__ __launch_bounds__(256, 2) void flat_split_candidates(
         full &= full - 1;
         const int row = wid + 4 * l;
         compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP, __builtin_amdgcn_readlane(c_l, l), Kp, lane,
-                         &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row, false);
+                         &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row);
       }
       __syncthreads();
     }
   }
   if constexpr (SEED) return;
-  for (int row = wid; row < R; row += 4) {
-    if (q0 + row >= nq) continue;
-    uint64_t* base = cand + ((size_t)(q0 + row) * S + split) * CAP;
-    const int c = cnt[row];
-    if (c <= Kp) {
-      for (int i = c + lane; i < Kp; i += WAVE) base[i] = KEY_MAX;
-    } else {
-      compact_row<CAP>(base, c, Kp, lane, &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row, true);
-    }
-  }
+  if (tid < R && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP + CAP - 1] = (uint64_t)cnt[tid];
 }

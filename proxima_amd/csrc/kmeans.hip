@@ -228,7 +228,10 @@ static void launch_assign(const float* P, int ldp, const uint32_t* rows, size_t 
 //
 // eps: the fp32 dot product and norms over d terms, the final rounding and
 // the exact sequential (or 8-lane) sum of squares each stay within
-// (2d + 6) * 2^-24 * (|p| + max|c|)^2; twice that is used.
+// (2d + 6) * 2^-24 * s^2, s = |p| + max|c|; twice that is used. km_split's
+// products are within (3.75 d + 6) * 2^-24 * |p||c| (split.hpp), twice that
+// in the distance and 4 |p||c| <= s^2; with the exact sum's d + 3, the
+// centroid norm's d / 8 + 3 and the last rounding: 3 d + 11 of the 4 d + 12.
 //
 // Non-finite values: with finite coordinates every partial sum of the
 // approximation is at most (|p| + |c|)^2 in magnitude, which is below s^2 in
@@ -713,12 +716,6 @@ __global__ __launch_bounds__(256, 3) void km_mfma_reg(const float* __restrict__ 
 // that the certificate sends it to the exact scan.
 constexpr int KM_SPLIT_MAX_DIM = 256;
 
-// km_mfma_verify's eps is 2 (eps_d d + 6) 2^-24 s^2 with s = |p| + max |c|.
-// In units of 2^-24 s^2 (4 |p||c| <= s^2) the split product's error counts
-// (7.13 d + 6) / 2, the exact sequential sum's d + 3, the centroid's norm
-// d / 8 + 3 and the last rounding 2: below 4.7 d + 11.
-constexpr float KM_SPLIT_EPS_D = 2.5f;
-
 // Centroid norms the split pass takes: a point whose own squared norm
 // underflows to 0 goes in as zeros, which is within eps only while the
 // centroids' norms are above about 2^-58.
@@ -863,7 +860,7 @@ __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P,
                                                     const float* __restrict__ best, const float* __restrict__ second,
                                                     uint32_t* __restrict__ assign, float* __restrict__ dist,
                                                     uint32_t* __restrict__ redo, int* __restrict__ nredo, int bx,
-                                                    float eps_d = 2.0f, bool vec4 = true) {
+                                                    bool vec4 = true) {
   // the block's KV_PB points and their winning centroids, staged through LDS
   // 32 coordinates at a time (eight lanes per 128-byte row slice); 34 KB of
   // LDS, so four blocks per CU keep the row loads in flight
@@ -874,7 +871,7 @@ __device__ __forceinline__ void km_mfma_verify_body(const float* __restrict__ P,
   if (t < KV_PB) {  // threads KV_PB.. only help with the loads
     if (i < n) {
       const float s = (sqrtf(pn[i]) + sqrtf(cmax[0])) * 1.0001f;
-      const float eps = 2.0f * (eps_d * (float)dim + 6.0f) * 5.9604645e-08f * s * s;
+      const float eps = 2.0f * (2.0f * (float)dim + 6.0f) * 5.9604645e-08f * s * s;
       ok = second[i] > best[i] + 2.0f * eps;
       if (!ok) redo[atomicAdd(nredo, 1)] = (uint32_t)i;
       sr[t] = rows ? rows[i] : (uint32_t)i;
@@ -949,9 +946,9 @@ __global__ __launch_bounds__(256) void km_mfma_verify(const float* __restrict__ 
                                                       const float* __restrict__ best, const float* __restrict__ second,
                                                       uint32_t* __restrict__ assign, float* __restrict__ dist,
                                                       uint32_t* __restrict__ redo, int* __restrict__ nredo,
-                                                      float eps_d, int vec4) {
+                                                      int vec4) {
   km_mfma_verify_body<UNR>(P, ldp, rows, n, dim, C, ldc, pn, cmax, best_idx, best, second, assign, dist, redo, nredo,
-                           blockIdx.x, eps_d, vec4 != 0);
+                           blockIdx.x, vec4 != 0);
 }
 
 constexpr int KW_DMAX = 2048;  // largest dim of the MFMA assignment path
@@ -1223,15 +1220,14 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
   }
   PXG_HIP(hipMemsetAsync(nredo, 0, 4, s));
   const dim3 g((unsigned)((n + KV_PB - 1) / KV_PB));
-  const float eps_d = split ? KM_SPLIT_EPS_D : 2.0f;
   if (unrolled)
     hipLaunchKernelGGL(km_mfma_verify<true>, g, dim3(256), 0, s, P, ldp, rows, (int)n, dim, C, ldc, (const float*)pn,
                        (const float*)cmax, (const uint32_t*)bidx, (const float*)best, (const float*)second, assign,
-                       dist, redo, nredo, eps_d, (int)aligned);
+                       dist, redo, nredo, (int)aligned);
   else
     hipLaunchKernelGGL(km_mfma_verify<false>, g, dim3(256), 0, s, P, ldp, rows, (int)n, dim, C, ldc, (const float*)pn,
                        (const float*)cmax, (const uint32_t*)bidx, (const float*)best, (const float*)second, assign,
-                       dist, redo, nredo, eps_d, (int)aligned);
+                       dist, redo, nredo, (int)aligned);
   PXG_HIP(hipGetLastError());
   int m = 0;
   PXG_HIP(hipMemcpyAsync(&m, nredo, 4, hipMemcpyDeviceToHost, s));
