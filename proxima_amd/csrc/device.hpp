@@ -420,7 +420,8 @@ __device__ inline uint64_t block_radix_select_each(Each each, int K, int* hist, 
 template <int NT, class Each>
 __device__ inline uint64_t block_radix_select_range(Each each, uint64_t lo, uint64_t hi, int K, int* hist,
                                                     uint64_t* sh) {
-  __shared__ uint64_t wlo[NT / WAVE], whi[NT / WAVE];
+  __shared__ uint64_t wlo[NT / WAVE], whi[NT / WAVE], few[WAVE];
+  __shared__ int n_few;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const uint64_t a = shfl_xor64(lo, o), b = shfl_xor64(hi, o);
@@ -432,7 +433,10 @@ __device__ inline uint64_t block_radix_select_range(Each each, uint64_t lo, uint
     wlo[threadIdx.x >> 6] = lo;
     whi[threadIdx.x >> 6] = hi;
   }
-  if (threadIdx.x == 0) sh[3] = 0;
+  if (threadIdx.x == 0) {
+    sh[3] = 0;
+    n_few = 0;
+  }
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NT / WAVE; ++w) {
@@ -485,6 +489,20 @@ __device__ inline uint64_t block_radix_select_range(Each each, uint64_t lo, uint
         if ((x & mask) == prefix && x > m) m = x;
       });
       if (m) atomicMax((unsigned long long*)&sh[3], (unsigned long long)m);
+      __syncthreads();
+      return sh[3];
+    }
+    if (cnt <= WAVE && shift > 0) {
+      // one wavefront sorts the bin
+      each([&](uint64_t x) {
+        if ((x & mask) == prefix) few[atomicAdd(&n_few, 1)] = x;
+      });
+      __syncthreads();
+      if (threadIdx.x < WAVE) {
+        uint64_t k1[1] = {lane < cnt ? few[lane] : KEY_MAX};
+        wave_bitonic_sort<1>(k1, lane);
+        if (lane == remaining - 1) sh[3] = k1[0];
+      }
       __syncthreads();
       return sh[3];
     }

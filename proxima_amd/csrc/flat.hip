@@ -195,7 +195,7 @@ __device__ __attribute__((noinline)) void flat_stored_tile(uint64_t* __restrict_
         const uint64_t key = ((uint64_t)kk[e] << 32) | (uint32_t)slot;
         if (key < t && usable[e]) {
           const int pos = atomicAdd(&cnt[row], 1);
-          cand[((size_t)(q0 + row) * S + split) * CAP + pos] = key;
+          cand[((size_t)(q0 + row) * S + split) * CAP + 1 + pos] = key;
         }
       }
     }
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256, 2) void flat_mfma_candidates(
             const uint64_t key = ((uint64_t)ord_key(a) << 32) | (uint32_t)(n0 + wn + j * 32 + r);
             if (key < thr[row]) {
               const int pos = atomicAdd(&cnt[row], 1);
-              cand[((size_t)(q0 + row) * S + split) * CAP + pos] = key;
+              cand[((size_t)(q0 + row) * S + split) * CAP + 1 + pos] = key;
             }
           }
         }
@@ -522,12 +522,12 @@ __global__ __launch_bounds__(256, 2) void flat_mfma_candidates(
       // this wave's rows wid, wid + 4, ...: one count per lane, then a
       // compaction for each row that might not take another tile's appends
       const int c_l = lane < FB_M / 4 ? cnt[wid + 4 * lane] : 0;
-      uint64_t full = __ballot(c_l > CAP - FB_N);
+      uint64_t full = __ballot(c_l > CAP - 1 - FB_N);
       while (full) {
         const int l = __builtin_ctzll(full);
         full &= full - 1;
         const int row = wid + 4 * l;
-        compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP, __builtin_amdgcn_readlane(c_l, l), Kp,
+        compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP + 1, __builtin_amdgcn_readlane(c_l, l), Kp,
                          lane, &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row);
       }
       __syncthreads();
@@ -535,9 +535,9 @@ __global__ __launch_bounds__(256, 2) void flat_mfma_candidates(
   }
   // Seeding pass: each row has left its one tile's FB_N distance parts.
   if constexpr (SEED) return;
-  // Final: every row leaves its keys (at most CAP - FB_N after the last
-  // tile's compaction) and their number in the buffer's last entry.
-  if (tid < FB_M && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP + CAP - 1] = (uint64_t)cnt[tid];
+  // Final: every row leaves its keys' number in the buffer's first entry (the
+  // keys follow it, so that the merge finds the first 15 in the same line).
+  if (tid < FB_M && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP] = (uint64_t)cnt[tid];
 }
 
 #include "flat_split.hpp"
@@ -645,19 +645,19 @@ __device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric,
 }
 
 // Per query: the k' smallest approximate keys of its S candidate lists
-// (list s: the first cand[s * CAP + CAP - 1] entries of its buffer, unsorted),
-// rescored exactly and sorted; see the file's head.
+// (list s: cand[s * CAP] keys from cand[s * CAP + 1] on, unsorted), rescored exactly and sorted; see the file's head.
 //
 // At least k' keys of the lists are at or below the query's shared threshold
 // (its seed, or the k'-th key some split published), so only those can be
 // among the k' smallest: they are gathered into LDS (16 threads per list, the
 // first 16 entries of four lists loaded together) and selected there. More
 // than LM of them are selected from memory instead.
-// What bounds it: round trips to memory (counts, keys, rows, ids), five to
-// seven of them; 313 queries of 170 lists and k' = 116 (about 1600 gathered
-// keys): 225 us when every list was padded to k' keys and all 19,720 were
-// selected over, 31 us here; 1000 queries of 61 lists, k' = 26: 14.6 -> 11.8
-// us; 48 queries of 195 lists, k' = 26: 16.2 -> 10.6 us.
+// What bounds it: round trips to memory (the lists, then rows, ranks and ids
+// together) and the select's barriers. 313 queries of 170 lists and k' = 116
+// (about 1600 gathered keys): 225 us when every list was padded to k' keys
+// and all 19,720 were selected over, 36 us here; 48 queries of 195 lists, k'
+// = 26: 16.2 -> 11.4 us; 1000 queries of 61 lists: 14.6 -> 16.6 us, for 7 us
+// less in the candidate pass, which no longer sorts and pads its lists.
 template <int NT, int LM>
 __global__ __launch_bounds__(NT) void flat_merge(
     const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const unsigned long long* __restrict__ gthr,
@@ -673,27 +673,18 @@ __global__ __launch_bounds__(NT) void flat_merge(
   __shared__ int hist[256];
   __shared__ uint64_t sh[4];
   __shared__ uint64_t sel[MERGE_MAXP];
-  __shared__ uint32_t rslot[WAVE];
+  __shared__ uint64_t rid[WAVE];
   __shared__ int n_list, n_valid, n_sel;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & (WAVE - 1);
   const uint64_t* base = cand + (size_t)q * S * CAP;
   const uint64_t g = gthr[q];
+  const int gl = tid & 15, grp = tid >> 4;
+  // the counts and first 15 keys of the first 4 NG lists, in flight together
+  uint64_t x[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) x[u] = base[(size_t)min(u * NG + grp, S - 1) * CAP + gl];
   if (tid == 0) n_list = n_valid = n_sel = 0;
   __syncthreads();
-  int local = 0;
-  for (int s = tid; s < S; s += NT) {
-    const int c = (int)(uint32_t)base[(size_t)s * CAP + CAP - 1];
-    scnt[s] = (uint16_t)c;
-    local += c;
-  }
-  if (local) atomicAdd(&n_valid, local);
-  __syncthreads();
-  const int valid = n_valid;
-  const int ksel = min(Kp, valid);
-  if (ksel == 0) {
-    if (tid == 0) out_count[q] = 0;
-    return;
-  }
   // appends the calling lanes' keys at or below the threshold, one counter
   // update per wave
   auto push = [&](uint64_t x) {
@@ -705,33 +696,67 @@ __global__ __launch_bounds__(NT) void flat_merge(
     at = __builtin_amdgcn_readlane(at, leader) + __popcll(m & ((1ull << lane) - 1));
     if (((m >> lane) & 1) != 0 && at < LM) lst[at] = x;
   };
-  const int gl = tid & 15, grp = tid >> 4;
+  int mine = 0;  // keys of this group's lists
   for (int s0 = 0; s0 < S; s0 += 4 * NG) {  // uniform, so that every lane takes part in push
-    uint64_t x[4];
     int c[4], most = 0;
+    if (s0 > 0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = base[(size_t)min(s0 + u * NG + grp, S - 1) * CAP + gl];  // unconditional loads
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int s = s0 + u * NG + grp;
-      c[u] = s < S ? scnt[s] : 0;
-      x[u] = base[(size_t)min(s, S - 1) * CAP + min(gl, CAP - 1)];  // unconditional loads
+      const int cs = __shfl((int)(uint32_t)x[u], lane & ~15, WAVE);
+      c[u] = s < S ? cs : 0;
+      if (gl == 0 && s < S) scnt[s] = (uint16_t)cs;
+      mine += c[u];
       most = max(most, c[u]);
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) push(gl < c[u] ? x[u] : KEY_MAX);
-    for (int j0 = 16; __ballot(j0 < most) != 0; j0 += 16) {
+    for (int u = 0; u < 4; ++u) push(gl > 0 && gl <= c[u] ? x[u] : KEY_MAX);
+    for (int j0 = 15; __ballot(j0 < most) != 0; j0 += 16) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int s = min(s0 + u * NG + grp, S - 1);
-        x[u] = j0 + gl < c[u] ? base[(size_t)s * CAP + j0 + gl] : KEY_MAX;
+        x[u] = j0 + gl < c[u] ? base[(size_t)s * CAP + 1 + j0 + gl] : KEY_MAX;
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) push(x[u]);
     }
   }
+  if (gl == 0 && mine) atomicAdd(&n_valid, mine);
   __syncthreads();
+  const int valid = n_valid;
+  const int ksel = min(Kp, valid);
+  if (ksel == 0) {
+    if (tid == 0) out_count[q] = 0;
+    return;
+  }
   const int n = n_list;
   uint64_t pivot;
-  if (n <= LM) {
+  if (n <= 2 * NT && gridDim.x <= 256) {
+    // few keys, and one query per CU: each thread counts the keys below its
+    // own two (a chain of LDS reads instead of the select's barriers; with
+    // several queries per CU those reads are what they wait for: 1000 queries
+    // 18.6 -> 27.5 us)
+    const uint64_t a = tid < n ? lst[tid] : KEY_MAX, b = tid + NT < n ? lst[tid + NT] : KEY_MAX;
+    int ra = 0, rb = 0;
+    if (n <= NT) {
+#pragma unroll 8
+      for (int j = 0; j < n; ++j) ra += lst[j] < a ? 1 : 0;
+    } else {
+#pragma unroll 8
+      for (int j = 0; j < n; ++j) {
+        const uint64_t y = lst[j];
+        ra += y < a ? 1 : 0;
+        rb += y < b ? 1 : 0;
+      }
+    }
+    if (a != KEY_MAX && ra < ksel) sel[ra] = a;
+    if (b != KEY_MAX && rb < ksel) sel[rb] = b;
+    __syncthreads();
+    pivot = sel[ksel - 1];
+  } else if (n <= LM) {
     // the digits start at the highest bit in which the keys differ
     uint64_t v[PER], lo = KEY_MAX, hi = 0;
 #pragma unroll
@@ -755,7 +780,7 @@ __global__ __launch_bounds__(NT) void flat_merge(
     auto each = [&](auto f) {
       for (int s = grp; s < S; s += NG)
         for (int j = gl; j < (int)scnt[s]; j += 16) {
-          const uint64_t x = base[(size_t)s * CAP + j];
+          const uint64_t x = base[(size_t)s * CAP + 1 + j];
           if (x <= g) f(x);
         }
     };
@@ -770,23 +795,25 @@ __global__ __launch_bounds__(NT) void flat_merge(
   const float* qv = Qp + (size_t)q * ld;
   for (int c = tid >> 3; c < ksel; c += NT / 8) {
     const uint32_t slot = (uint32_t)sel[c];
+    const uint32_t rk = rank[slot];
+    const uint64_t id = Kp <= WAVE ? ids[slot] : 0;
     const float d = dist_group8_rt(metric, qv, X + (size_t)slot * ld, dim, tid & 7);
     if ((tid & 7) == 0) {
-      if (Kp <= WAVE) rslot[c] = slot;
-      sel[c] = ((uint64_t)ord_key(d) << 32) | rank[slot];
+      if (Kp <= WAVE) rid[c] = id;
+      sel[c] = ((uint64_t)ord_key(d) << 32) | rk;
     }
   }
   __syncthreads();
   const int kout = min(k, ksel);
   uint64_t kth;
   if (Kp <= WAVE) {
-    // one wavefront sorts the keys with their slots
+    // one wavefront sorts the keys with their places
     if (tid >= WAVE) return;
     uint64_t key = lane < ksel ? sel[lane] : KEY_MAX;
-    uint32_t slot = lane < ksel ? rslot[lane] : 0;
-    wave_sort_kv64(key, slot, lane);
+    uint32_t at = (uint32_t)lane;
+    wave_sort_kv64(key, at, lane);
     if (lane < kout) {
-      out_ids[(size_t)q * ldo + lane] = ids[slot];
+      out_ids[(size_t)q * ldo + lane] = rid[at];
       out_d[(size_t)q * ldo + lane] = key_float((uint32_t)(key >> 32));
     }
     kth = (uint64_t)(uint32_t)__shfl((int)(uint32_t)(key >> 32), kout - 1, WAVE) << 32;

@@ -80,7 +80,7 @@ __device__ __attribute__((noinline)) void split_stored_tile(uint64_t* __restrict
         const uint64_t key = ((uint64_t)kk[e] << 32) | (uint32_t)(n0 + 4 * c + e);
         if (key < t) {
           const int pos = atomicAdd(&cnt[row], 1);
-          cand[((size_t)(q0 + row) * S + split) * CAP + pos] = key;
+          cand[((size_t)(q0 + row) * S + split) * CAP + 1 + pos] = key;
         }
       }
     }
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256, 2) void flat_split_candidates(
               const uint64_t key = ((uint64_t)ord_key(a) << 32) | (uint32_t)slot;
               if (key < thr[row]) {
                 const int pos = atomicAdd(&cnt[row], 1);
-                cand[((size_t)(q0 + row) * S + split) * CAP + pos] = key;
+                cand[((size_t)(q0 + row) * S + split) * CAP + 1 + pos] = key;
               }
             }
           }
@@ -362,17 +362,17 @@ __global__ __launch_bounds__(256, 2) void flat_split_candidates(
       // this wave's rows wid, wid + 4, ...: a compaction for each row that
       // might not take another tile's appends
       const int c_l = lane < R / 4 ? cnt[wid + 4 * lane] : 0;
-      uint64_t full = __ballot(c_l > CAP - FB_N);
+      uint64_t full = __ballot(c_l > CAP - 1 - FB_N);
       while (full) {
         const int l = __builtin_ctzll(full);
         full &= full - 1;
         const int row = wid + 4 * l;
-        compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP, __builtin_amdgcn_readlane(c_l, l), Kp, lane,
+        compact_row<CAP>(cand + ((size_t)(q0 + row) * S + split) * CAP + 1, __builtin_amdgcn_readlane(c_l, l), Kp, lane,
                          &thr[row], &thr_f[row], &cnt[row], gthr + q0 + row);
       }
       __syncthreads();
     }
   }
   if constexpr (SEED) return;
-  if (tid < R && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP + CAP - 1] = (uint64_t)cnt[tid];
+  if (tid < R && q0 + tid < nq) cand[((size_t)(q0 + tid) * S + split) * CAP] = (uint64_t)cnt[tid];
 }
