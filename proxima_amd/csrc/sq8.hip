@@ -58,6 +58,10 @@ constexpr uint32_t SQ_MAX_DIM = 65536;  // |S| < 2^31
 // Buffer resource word 3 for raw (untyped, stride 0) gfx9 buffer accesses.
 [[maybe_unused]] constexpr int SQ_RSRC_WORD3 = 0x00020000;
 constexpr int SQ_LCAP = 1024;         // per-workgroup candidate list in LDS
+// Ints between the queries' candidate counters: 256 bytes, since atomics to
+// one line from many workgroups go one after another (33 adjacent counters,
+// about 1200 adds each: stage 2 took 108 us, 51 us with the counters apart).
+constexpr int SQ_CSTRIDE = 64;
 
 __host__ __device__ constexpr int sq_rows(int kb) { return kb <= 4 ? 256 : 128; }
 
@@ -291,13 +295,24 @@ __device__ __forceinline__ uint32_t lds_addr(const T* p) {
 // QTT: query tiles per wave (0 = sq_qt(KB)). A smaller batch takes fewer,
 // so that its queries spread over all the waves (and SIMDs) of a workgroup
 // rather than a few waves multiplying code tiles of absent queries.
-template <int KB, bool STAGE1, int QTT = 0>
+//
+// RS: row groups. A batch too small for the waves (up to 128 queries) has the
+// waves share a tile's row blocks instead: SQ_NW / RS waves along the queries,
+// RS along the rows, each wave with its own stage-1 maxima (so the thresholds
+// are tighter too). Such a scan is bound by reading the codes; a wave then
+// takes passing scores straight from its accumulators, without the second
+// product. 33 queries, 1M x 128-byte codes, rescoring 100: the two scans 123
+// -> 42 us (stage 2 alone without a passing score: 22 us, 5.8 TB/s).
+template <int KB, bool STAGE1, int QTT = 0, int RS = 1>
 __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
     const int8_t* __restrict__ Qc, int nq, const int8_t* __restrict__ C, int N, const uint8_t* __restrict__ live,
     const uint8_t* __restrict__ accept, const uint32_t* __restrict__ rank, int nchunks, int qgroups,
     int tiles_per_chunk, int sample, const int* __restrict__ thr_in, int* __restrict__ tmax,
     int* __restrict__ ccount, uint64_t* __restrict__ cand, int cap) {
-  constexpr int KP = KB * 32, SR = KP + 16, R = sq_rows(KB), RT = R / 32, QT = QTT > 0 ? QTT : sq_qt(KB);
+  constexpr int KP = KB * 32, SR = KP + 16, R = sq_rows(KB), QT = QTT > 0 ? QTT : sq_qt(KB);
+  constexpr int RT = R / 32 / RS;      // row blocks of a tile per wave
+  constexpr int WQ = SQ_NW / RS;       // waves along the queries
+  static_assert(RT >= 1 && R / 32 % RS == 0 && SQ_NW % RS == 0, "whole row blocks per wave");
   constexpr int PPR = KP / 16;         // 16-byte pieces per row
   constexpr int D = 3;                // LDS tiles: the next two tiles load during the current one
   __shared__ __align__(16) int8_t tile[D][R * SR];
@@ -324,7 +339,8 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = qgroup * (SQ_NW * QT * 32) + w * (QT * 32);
+  const int q0 = qgroup * (WQ * QT * 32) + w % WQ * (QT * 32);
+  const int rb0 = w / WQ * RT;  // this wave's first row block
   const bool active = q0 < nq;
 
   i4v qa[QT][KB];
@@ -388,7 +404,8 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
   // kb*32 + 16*(l/32) .. +16 of every K block.
   auto load_a = [&](i4v(&a)[KB], const int8_t* tl, int rt) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) a[kb] = *reinterpret_cast<const i4v*>(&tl[(rt * 32 + r) * SR + kb * 32 + h * 16]);
+    for (int kb = 0; kb < KB; ++kb)
+      a[kb] = *reinterpret_cast<const i4v*>(&tl[((rb0 + rt) * 32 + r) * SR + kb * 32 + h * 16]);
   };
   auto mfmas = [&](i16v(&acc)[QT], const i4v(&a)[KB]) __attribute__((always_inline)) {
 #pragma unroll
@@ -400,14 +417,37 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) acc[qt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kb], qa[qt][kb], acc[qt], 0, 0, 0);
   };
+  // stage 2: the passing scores x[0..15] of a lane's query in row block rt of
+  // tile t, to the workgroup list
+  auto collect = [&](const i16v& x, int qt, int rt, int t) __attribute__((always_inline)) {
+    const int q = q0 + qt * 32 + r;
+    const int tq = thr[qt];
+    const int rowb = t * R + (rb0 + rt) * 32 + 4 * h;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int val = x[v];
+      const int row = rowb + 8 * (v >> 2) + (v & 3);
+      if (val >= tq && row < N && q < nq) {
+        const int pos = atomicAdd(&lc_n, 1);
+        if (pos < SQ_LCAP) {
+          lc_score[pos] = val;
+          lc_row[pos] = row;
+          lc_q[pos] = q;
+        } else if (live[row] && (accept == nullptr || accept[row])) {  // list full: publish directly
+          const int gp = atomicAdd(&ccount[(size_t)q * SQ_CSTRIDE], 1);
+          if (gp < cap) cand[(size_t)q * cap + gp] = ((uint64_t)ord_key(-(float)val) << 32) | rank[row];
+        }
+      }
+    }
+  };
   uint32_t passmask = 0;  // stage 2, bit rt*QT+qt: that 32 x 32 block has a score >= the threshold
-  auto reduce = [&](const i16v(&acc)[QT], int rt, int buf) __attribute__((always_inline)) {
+  auto reduce = [&](const i16v(&acc)[QT], int rt, int buf, [[maybe_unused]] int t) __attribute__((always_inline)) {
     if constexpr (STAGE1) {
       uint32_t vw[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        vw[g] = *reinterpret_cast<const uint32_t*>(&vlive[buf][rt * 32 + 8 * g + 4 * h]) &
-                *reinterpret_cast<const uint32_t*>(&vacc[buf][rt * 32 + 8 * g + 4 * h]);
+        vw[g] = *reinterpret_cast<const uint32_t*>(&vlive[buf][(rb0 + rt) * 32 + 8 * g + 4 * h]) &
+                *reinterpret_cast<const uint32_t*>(&vacc[buf][(rb0 + rt) * 32 + 8 * g + 4 * h]);
       if (__all((vw[0] & vw[1] & vw[2] & vw[3]) == 0x01010101u)) {
         // every row of the 32 x 32 block is usable: a v_max3 chain
 #pragma unroll
@@ -445,7 +485,11 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
         m = max(max(m, x[11]), x[12]);
         m = max(max(m, x[13]), x[14]);
         m = max(m, x[15]);
-        passmask |= (__ballot(m >= thr[qt]) != 0 ? 1u : 0u) << (rt * QT + qt);
+        if constexpr (RS == 1) {
+          passmask |= (__ballot(m >= thr[qt]) != 0 ? 1u : 0u) << (rt * QT + qt);
+        } else if (__ballot(m >= thr[qt]) != 0) {
+          collect(x, qt, rt, t);
+        }
       }
     }
   };
@@ -476,13 +520,13 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
         if (rt % 2 == 0) {
           mfmas(c0, a0);
           if (rt + 1 < RT) load_a(a1, tl, rt + 1);
-          if (rt > 0) reduce(c1, rt - 1, buf);
+          if (rt > 0) reduce(c1, rt - 1, buf, t);
         } else {
           mfmas(c1, a1);
           if (rt + 1 < RT) load_a(a0, tl, rt + 1);
-          reduce(c0, rt - 1, buf);
+          reduce(c0, rt - 1, buf, t);
         }
-        if constexpr (!STAGE1) {
+        if constexpr (!STAGE1 && RS == 1) {
           // the next A operand's reads first, then each MFMA followed by
           // four of the previous block's filter instructions; nothing of
           // this block's filter moves up
@@ -495,12 +539,12 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if ((RT - 1) % 2 == 0) reduce(c0, RT - 1, buf);
-      else reduce(c1, RT - 1, buf);
+      if ((RT - 1) % 2 == 0) reduce(c0, RT - 1, buf, t);
+      else reduce(c1, RT - 1, buf, t);
       // Rare: some 32 x 32 blocks hold a score >= the threshold. Recompute
       // exactly those from the LDS tile (still valid until the barrier) and
       // append their passing scores to the workgroup list.
-      if constexpr (!STAGE1) {
+      if constexpr (!STAGE1 && RS == 1) {
         if (passmask) {
 #pragma unroll 1
           for (int rt = 0; rt < RT; ++rt) {
@@ -516,25 +560,7 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
               for (int v = 0; v < 16; ++v) x[v] = 0;
 #pragma unroll
               for (int kb = 0; kb < KB; ++kb) x = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kb], qa[qt][kb], x, 0, 0, 0);
-              const int q = q0 + qt * 32 + r;
-              const int tq = thr[qt];
-              const int rowb = t * R + rt * 32 + 4 * h;
-#pragma unroll
-              for (int v = 0; v < 16; ++v) {
-                const int val = x[v];
-                const int row = rowb + 8 * (v >> 2) + (v & 3);
-                if (val >= tq && row < N && q < nq) {
-                  const int pos = atomicAdd(&lc_n, 1);
-                  if (pos < SQ_LCAP) {
-                    lc_score[pos] = val;
-                    lc_row[pos] = row;
-                    lc_q[pos] = q;
-                  } else if (live[row] && (accept == nullptr || accept[row])) {  // list full: publish directly
-                    const int gp = atomicAdd(&ccount[q], 1);
-                    if (gp < cap) cand[(size_t)q * cap + gp] = ((uint64_t)ord_key(-(float)val) << 32) | rank[row];
-                  }
-                }
-              }
+              collect(x, qt, rt, t);
             }
           }
         }
@@ -553,7 +579,7 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const int q = q0 + qt * 32 + r;
-        if (q < nq) tmax[(size_t)q * (nchunks * 2) + chunk * 2 + h] = run[qt];
+        if (q < nq) tmax[(size_t)q * (nchunks * 2 * RS) + (chunk * RS + w / WQ) * 2 + h] = run[qt];
       }
     }
   } else {
@@ -563,7 +589,7 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
     for (int i = tid; i < n; i += SQ_NW * 64) {
       const int row = lc_row[i], q = lc_q[i];
       if (live[row] && (accept == nullptr || accept[row])) {
-        const int gp = atomicAdd(&ccount[q], 1);
+        const int gp = atomicAdd(&ccount[(size_t)q * SQ_CSTRIDE], 1);
         if (gp < cap) cand[(size_t)q * cap + gp] = ((uint64_t)ord_key(-(float)lc_score[i]) << 32) | rank[row];
       }
     }
@@ -583,20 +609,28 @@ __global__ __launch_bounds__(256) void sq8_thresholds(const int* __restrict__ tm
   // the k-th largest maximum: the k-th smallest of INT_MAX - v (in [0, 2^32))
   const int* t = tmax + (size_t)q * E;
   auto get = [&](int i) { return (uint64_t)((int64_t)INT_MAX - (int64_t)t[i]); };
-  const uint64_t v = E <= 8 * (int)blockDim.x ? block_radix_select<decltype(get), 32, 8>(get, E, k, hist, sh)
-                                  : block_radix_select<decltype(get), 32>(get, E, k, hist, sh);
+  const uint64_t v = E <= 8 * (int)blockDim.x    ? block_radix_select<decltype(get), 32, 8>(get, E, k, hist, sh)
+                     : E <= 32 * (int)blockDim.x ? block_radix_select<decltype(get), 32, 32>(get, E, k, hist, sh)
+                                                 : block_radix_select<decltype(get), 32>(get, E, k, hist, sh);
   if (threadIdx.x == 0) thr[q] = (int)((int64_t)INT_MAX - (int64_t)v);
 }
 
-// Per query: sort the appended candidates and keep the first kk; a query
-// with more than `cap` candidates is listed for the exact scan.
+// Per query: the first kk of the appended candidates, sorted; a query with
+// more than `cap` candidates is listed for the exact scan. The kk-th is
+// selected first (keys in registers, PER per thread), so that only kk keys are
+// sorted: 33 queries, kk = 100: 25.6 -> 12.8 us; 1024 queries, kk = 10: 13.7
+// -> 10.3 us.
+template <int PER>
 __global__ __launch_bounds__(256) void sq8_finish(const int* __restrict__ ccount, const uint64_t* __restrict__ cand,
                                                   int cap, int kk, uint64_t* __restrict__ okeys,
                                                   uint32_t* __restrict__ ocount, int* __restrict__ flag_list,
                                                   int* __restrict__ flag_count) {
-  extern __shared__ uint64_t sk[];
+  extern __shared__ uint64_t sk[];  // kk rounded up to a power of two
+  __shared__ int hist[256];
+  __shared__ uint64_t sh[4];
+  __shared__ int n_sel;
   const int q = blockIdx.x;
-  const int c = ccount[q];
+  const int c = ccount[(size_t)q * SQ_CSTRIDE];
   if (c > cap) {
     // listed for the exact scan; no result until then
     if (threadIdx.x == 0) {
@@ -605,14 +639,42 @@ __global__ __launch_bounds__(256) void sq8_finish(const int* __restrict__ ccount
     }
     return;
   }
+  if (threadIdx.x == 0) {
+    n_sel = 0;
+    ocount[q] = (uint32_t)min(kk, c);
+  }
+  if (c == 0) return;
+  const int ksel = min(kk, c);
+  uint64_t v[PER], lo = KEY_MAX, hi = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = threadIdx.x + j * 256;
+    v[j] = cand[(size_t)q * cap + min(i, c - 1)];  // unconditional loads
+    if (i >= c) v[j] = KEY_MAX;
+    if (v[j] != KEY_MAX) {
+      lo = min(lo, v[j]);
+      hi = max(hi, v[j]);
+    }
+  }
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (v[j] != KEY_MAX) f(v[j]);
+  };
+  const uint64_t pivot = block_radix_select_range<256>(each, lo, hi, ksel, hist, sh);
+  // keys are distinct (one per row): exactly ksel are at or below the pivot
+  each([&](uint64_t x) {
+    if (x <= pivot) {
+      const int at = atomicAdd(&n_sel, 1);
+      if (at < ksel) sk[at] = x;
+    }
+  });
   int P = 1;
-  while (P < c) P <<= 1;
-  for (int i = threadIdx.x; i < P; i += blockDim.x) sk[i] = i < c ? cand[(size_t)q * cap + i] : KEY_MAX;
+  while (P < ksel) P <<= 1;
+  for (int i = ksel + threadIdx.x; i < P; i += 256) sk[i] = KEY_MAX;
   __syncthreads();
   block_bitonic_sort(sk, P);
-  const int kout = min(kk, c);
-  for (int i = threadIdx.x; i < kout; i += blockDim.x) okeys[(size_t)q * kk + i] = sk[i];
-  if (threadIdx.x == 0) ocount[q] = (uint32_t)kout;
+  for (int i = threadIdx.x; i < ksel; i += 256) okeys[(size_t)q * kk + i] = sk[i];
 }
 
 // Exact scan of listed queries in EXACT_CH-row chunks (v_dot4_i32_i8 over
@@ -708,7 +770,12 @@ __global__ __launch_bounds__(256) void sq8_wide_rescore(const uint64_t* __restri
 }
 
 // Rescore a query's integer top kk with asymmetric_inner_product
-// (scalar.rs:313-319) and keep the best k by (distance, id).
+// (scalar.rs:313-319) and keep the best k by (distance, id). One thread per
+// candidate adds its components in order; the query, the ranges (in LDS, read
+// as broadcasts) and the code bytes (16 per load) come SQ_RC components at a
+// time, so that the chain is the additions and not the loads: 100 candidates
+// of 100 components 19.9 -> 13.9 us.
+constexpr int SQ_RC = 128;
 __global__ __launch_bounds__(256) void sq8_rescore(const uint64_t* __restrict__ okeys,
                                                    const uint32_t* __restrict__ ocount, int kk, int k,
                                                    const float* __restrict__ Qp, int ld, int dim,
@@ -718,24 +785,44 @@ __global__ __launch_bounds__(256) void sq8_rescore(const uint64_t* __restrict__ 
                                                    const uint64_t* __restrict__ ids, uint64_t* __restrict__ out_ids,
                                                    float* __restrict__ out_d, uint32_t* __restrict__ out_count) {
   extern __shared__ uint64_t sk[];
+  __shared__ __align__(16) float qs[SQ_RC], ms[SQ_RC], ss[SQ_RC];
   const int q = blockIdx.x;
   const int c = (int)ocount[q];
   int P = 1;
   while (P < c) P <<= 1;
   const float* qv = Qp + (size_t)q * ld;
-  for (int i = threadIdx.x; i < P; i += blockDim.x) {
-    uint64_t key = KEY_MAX;
-    if (i < c) {
-      const uint32_t rk = (uint32_t)okeys[(size_t)q * kk + i];
-      const uint8_t* code = reinterpret_cast<const uint8_t*>(C + (size_t)rank_slot[rk] * KP);
-      float sum = 0.0f;
-      for (int j = 0; j < dim; ++j) {
-        const int g = per_dim ? j : 0;
-        sum += qv[j] * sq_reconstruct(code[j], 1, mn[g], scale[g]);
+  for (int i0 = 0; i0 < P; i0 += 256) {  // uniform
+    const int i = i0 + threadIdx.x;
+    const bool on = i < c;
+    const uint32_t rk = on ? (uint32_t)okeys[(size_t)q * kk + i] : 0;
+    // code rows are KP bytes, a multiple of 32, 16-byte aligned
+    const uint4* code = reinterpret_cast<const uint4*>(C + (on ? (size_t)rank_slot[rk] * KP : 0));
+    float sum = 0.0f;
+    for (int j0 = 0; j0 < dim; j0 += SQ_RC) {
+      const int w = min(SQ_RC, dim - j0);
+      __syncthreads();
+      if (threadIdx.x < w) {
+        const int j = j0 + threadIdx.x, g = per_dim ? j : 0;
+        qs[threadIdx.x] = qv[j];
+        ms[threadIdx.x] = mn[g];
+        ss[threadIdx.x] = scale[g];
       }
-      key = ((uint64_t)ord_key(-arm_nan(sum)) << 32) | rk;
+      uint4 b[SQ_RC / 16];
+#pragma unroll
+      for (int u = 0; u < SQ_RC / 16; ++u) b[u] = code[min(j0 / 16 + u, KP / 16 - 1)];
+      __syncthreads();
+      if (!on) continue;
+#pragma unroll
+      for (int u = 0; u < SQ_RC / 16; ++u) {
+        const uint32_t word[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int j = 16 * u + e;
+          if (j < w) sum += qs[j] * sq_reconstruct((uint8_t)(word[e >> 2] >> (8 * (e & 3))), 1, ms[j], ss[j]);
+        }
+      }
     }
-    sk[i] = key;
+    if (i < P) sk[i] = on ? ((uint64_t)ord_key(-arm_nan(sum)) << 32) | rk : KEY_MAX;
   }
   __syncthreads();
   block_bitonic_sort(sk, P);
@@ -1195,7 +1282,10 @@ struct Sq8Index {
       // query tiles per wave: the fewest that hold the batch in one
       // workgroup's SQ_NW waves (1 up to 256 queries, 2 up to 512), at most
       // sq_qt(KB); qtt names the kernel variant (0 = sq_qt(KB))
+      // row groups: the waves that a batch of up to 128 queries leaves over
+      // (4 at most where a tile has four row blocks)
       const int R = sq_rows(KB), QT = nq <= 256 ? 1 : (nq <= 512 ? std::min(2, sq_qt(KB)) : sq_qt(KB));
+      const int RS = nq > 128 ? 1 : (nq > 64 ? 2 : (nq > 32 || R < 256 ? 4 : 8));
       const int qtt = QT == sq_qt(KB) ? 0 : QT;
       // Chunks: about 512 (two per CU), and at least 2 * kk so that every
       // query gets >= 4 * kk stage-1 maxima when the index has the tiles.
@@ -1205,36 +1295,55 @@ struct Sq8Index {
       // Stage 1 visits the tiles t % sample == 0; with chunks of >= sample
       // tiles every full chunk holds one (a chunk without one only adds
       // INT_MIN entries, which never raise the threshold).
-      const int target = std::min(std::min(SQ_MAX_CHUNKS, ntiles), std::max(512, 2 * kk));
+      // With row groups each chunk gives RS times the maxima, and one chunk
+      // per CU starts its pipeline once.
+      const int target = std::min(std::min(SQ_MAX_CHUNKS, ntiles),
+                                  RS > 1 ? std::max(256, (2 * kk + RS - 1) / RS) : std::max(512, 2 * kk));
       int tpc = (ntiles + target - 1) / target;
       int sample = SQ_SAMPLE;
-      if (tpc < SQ_SAMPLE) {
+      if (RS > 1) {
+        // A scan bound by the codes' bytes: stage 1 costs their share of it
+        // (5.8 TB/s measured), and a query's about kk * sample passing rows go
+        // through its counter one after another (about 30 ns each measured).
+        // The least of the sum: 33 queries, 1M x 128 bytes, kk = 100: stages 1
+        // and 2 take 6 and 51 us at one tile in 12, 11 and 31 us at one in 3.
+        const double scan_us = (double)N * (double)KP / 5.8e6;
+        sample = (int)std::lround(std::sqrt(scan_us / (0.03 * kk)));
+        sample = std::max(1, std::min({sample, SQ_SAMPLE, tpc}));
+      } else if (tpc < SQ_SAMPLE) {
         sample = 1;
         while (sample * 2 <= tpc) sample *= 2;
         tpc = sample;
       }
       const int nchunks = (ntiles + tpc - 1) / tpc;
       if (nchunks > SQ_MAX_CHUNKS) internal_error("sq8", "chunk count above the stage-1 limit");
-      const int qgroups = (int)((nq + SQ_NW * QT * 32 - 1) / (SQ_NW * QT * 32));
-      const int E = nchunks * 2;
+      const int per_wg = SQ_NW / RS * QT * 32;  // queries
+      const int qgroups = (int)((nq + per_wg - 1) / per_wg);
+      const int E = nchunks * 2 * RS;
       const int cap_c = kk <= 32 ? 1024 : 4096;
       int* tmax = (int*)sc.get(9, nq * E * 4);
       int* thr = (int*)sc.get(10, nq * 4);
-      int* ccount = (int*)sc.get(11, nq * 4);
+      int* ccount = (int*)sc.get(11, nq * SQ_CSTRIDE * 4);
       uint64_t* cand = (uint64_t*)sc.get(12, nq * cap_c * 8);
       const dim3 grid((unsigned)((nchunks * qgroups + 7) / 8 * 8));
-#define PXG_SQ_SCAN_Q(KBV, ST, QTV)                                                                                 \
-  hipLaunchKernelGGL((sq8_mfma_scan<KBV, ST, QTV>), grid, dim3(SQ_NW * 64), 0, s, (const int8_t*)Qc, (int)nq,      \
+#define PXG_SQ_SCAN_Q(KBV, ST, QTV, RSV)                                                                            \
+  hipLaunchKernelGGL((sq8_mfma_scan<KBV, ST, QTV, RSV>), grid, dim3(SQ_NW * 64), 0, s, (const int8_t*)Qc, (int)nq,      \
                      (const int8_t*)codes.p, N, d_live.p, d_accept, ranks.rank.p, nchunks, qgroups, tpc, sample,       \
                      (const int*)thr, tmax,                                                                        \
                      ccount, cand, cap_c)
-#define PXG_SQ_SCAN(KBV, ST)             \
-  if (qtt == 1)                          \
-    PXG_SQ_SCAN_Q(KBV, ST, 1);           \
-  else if (qtt == 2)                     \
-    PXG_SQ_SCAN_Q(KBV, ST, 2);           \
-  else                                   \
-    PXG_SQ_SCAN_Q(KBV, ST, 0)
+#define PXG_SQ_SCAN(KBV, ST)                              \
+  if (RS == 8)                                            \
+    PXG_SQ_SCAN_Q(KBV, ST, 1, (KBV <= 4 ? 8 : 4));        \
+  else if (RS == 4)                                       \
+    PXG_SQ_SCAN_Q(KBV, ST, 1, 4);                         \
+  else if (RS == 2)                                       \
+    PXG_SQ_SCAN_Q(KBV, ST, 1, 2);                         \
+  else if (qtt == 1)                                      \
+    PXG_SQ_SCAN_Q(KBV, ST, 1, 1);                         \
+  else if (qtt == 2)                                      \
+    PXG_SQ_SCAN_Q(KBV, ST, 2, 1);                         \
+  else                                                    \
+    PXG_SQ_SCAN_Q(KBV, ST, 0, 1)
 #define PXG_SQ_SWITCH(ST)                  \
   switch (KB) {                            \
     case 1: PXG_SQ_SCAN(1, ST); break;     \
@@ -1251,8 +1360,8 @@ struct Sq8Index {
       PXG_SQ_SWITCH(true)
       PXG_HIP(hipGetLastError());
       hipLaunchKernelGGL(sq8_thresholds, dim3((unsigned)nq), dim3(256), 0, s, (const int*)tmax, E, kk, thr);
-      hipLaunchKernelGGL(fill_u32, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, (uint32_t*)ccount, (size_t)nq,
-                         0u);
+      hipLaunchKernelGGL(fill_u32, dim3((unsigned)((nq * SQ_CSTRIDE + 255) / 256)), dim3(256), 0, s, (uint32_t*)ccount,
+                         (size_t)nq * SQ_CSTRIDE, 0u);
       tm.mark(1);
       PXG_SQ_SWITCH(false)
 #undef PXG_SQ_SWITCH
@@ -1260,8 +1369,14 @@ struct Sq8Index {
 #undef PXG_SQ_SCAN_Q
       PXG_HIP(hipGetLastError());
       tm.mark(2);
-      hipLaunchKernelGGL(sq8_finish, dim3((unsigned)nq), dim3(256), (size_t)cap_c * 8, s, (const int*)ccount,
-                         (const uint64_t*)cand, cap_c, kk, okeys, ocount, flag_list, flag_count);
+      int fP = 1;
+      while (fP < kk) fP <<= 1;
+      if (cap_c == 1024)
+        hipLaunchKernelGGL(sq8_finish<4>, dim3((unsigned)nq), dim3(256), (size_t)fP * 8, s, (const int*)ccount,
+                           (const uint64_t*)cand, cap_c, kk, okeys, ocount, flag_list, flag_count);
+      else
+        hipLaunchKernelGGL(sq8_finish<16>, dim3((unsigned)nq), dim3(256), (size_t)fP * 8, s, (const int*)ccount,
+                           (const uint64_t*)cand, cap_c, kk, okeys, ocount, flag_list, flag_count);
       PXG_HIP(hipGetLastError());
       // The results go out before the one host round trip; a query listed
       // for the exact scan has none yet, and its results are emitted again

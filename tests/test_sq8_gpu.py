@@ -280,3 +280,34 @@ def test_sq8_errors_and_edges(gpu):
     assert len(idx.search(x[0], 1000)) == 100  # k above len
     st = idx.stats()
     assert st.len == 100 and st.graph_bytes == 16 * 3 * 4
+
+
+@pytest.mark.parametrize("dim", [20, 100, 150, 256])
+@pytest.mark.parametrize("metric", [1, 2])
+def test_row_group_batches(gpu, dim, metric):
+    """Batches on both sides of the row-group edges (32, 64 and 128 queries;
+    tiles of eight and of four row blocks), with removed rows, a filter, many
+    equal scores (coarse codes of repeated rows) and rescoring, against the
+    oracle bit for bit."""
+    rng = np.random.default_rng(dim)
+    n = 9001
+    x = uniform(rng, n, dim)
+    x[4000:4100] = x[3]
+    idx = gpu.Sq8Index(gpu.VectorSpace(dim, metric))
+    idx.train(x[:3000])
+    idx.insert_batch(np.arange(n, dtype=np.uint64), x)
+    idx.set_search_mode(1)
+    codes, ranges = oracle_index(x, x[:3000], metric=metric)
+    live = np.ones(n, np.uint8)
+    for i in (0, 255, 256, n - 1):
+        idx.remove(i)
+        live[i] = 0
+    accept = (rng.random(n) < 0.6).astype(np.uint8)
+    qa = uniform(rng, 129, dim)
+    qa[1] = x[3]
+    for nq in (1, 31, 32, 33, 64, 65, 128, 129):
+        for k, rescore in ((10, 0), (20, 100)):
+            want = oracle_search(codes, np.arange(n), qa[:nq], ranges, k, metric=metric, live=live, rescore=rescore)
+            assert_same(idx.search_batch(qa[:nq], k, rescore=rescore), want)
+    want = oracle_search(codes, np.arange(n), qa[:33], ranges, 40, metric=metric, live=live, accept=accept)
+    assert_same(idx.search_batch(qa[:33], 40, filter=lambda i, _m: bool(accept[i])), want)
