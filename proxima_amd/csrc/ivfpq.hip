@@ -65,7 +65,9 @@
 namespace pxg {
 
 constexpr uint32_t UNASSIGNED = 0xFFFFFFFFu;
+constexpr int IVF_PGMAX = 32;  // probes per scan workgroup, at most
 constexpr int IVF_MAX_M = 128;
+constexpr size_t IVF_LDS = 160 * 1024;  // of a workgroup
 thread_local uint64_t g_last_scanned = 0;
 
 // ---------------------------------------------------------------------------
@@ -121,11 +123,24 @@ __device__ inline void wave_compact(uint64_t* wb, int cnt, int kk, int lane) {
   }
 }
 
+// General form (any subspace layout, shortlists up to IVF_MAX_SHORT): one
+// workgroup per (query, group of pg probes), the table in LDS, the waves'
+// candidate lists kept across the group's probes. The cosine table is the
+// query's own and is built once per workgroup; the L2 table is rebuilt per
+// probe (the residual's rounding is part of the result).
+// What bounds it: building tables for lists of a few hundred entries. The
+// query (or residual) is staged in LDS (when it fits beside the table) and
+// codebook rows whose widths are multiples of four come as float4 loads, two
+// instead of eight per entry at 8-wide subspaces; an entry's slot and rank are
+// fetched only if its distance can enter the list. 100 cosine queries, 12 x 8
+// dimensions, 16 probes of about 490 entries, shortlist 100: 120 us with a
+// workgroup and a table per probe -> 49 us.
 template <int CAPW, int METRIC>
 __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, int ld, int dim, int M,
-                                                const int* __restrict__ probes, int nprobe,
-                                                const float* __restrict__ cents, const float* __restrict__ books,
-                                                const int* __restrict__ sub_off, const int* __restrict__ book_off,
+                                                const int* __restrict__ probes, int nprobe, int pg, int groups,
+                                                int staged, const float* __restrict__ cents,
+                                                const float* __restrict__ books, const int* __restrict__ sub_off,
+                                                const int* __restrict__ book_off,
                                                 const uint32_t* __restrict__ list_beg,
                                                 const uint32_t* __restrict__ list_end,
                                                 const uint32_t* __restrict__ list_slot,
@@ -134,55 +149,77 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
                                                 const uint32_t* __restrict__ slot_rank,
                                                 const uint8_t* __restrict__ accept, int kk,
                                                 uint64_t* __restrict__ out) {
-  extern __shared__ float lut[];  // M * 256 floats
+  extern __shared__ __align__(16) float lut[];  // M * 256 floats, then (staged) dim of the query or residual
   __shared__ uint64_t wbuf[4][CAPW];
-  __shared__ float s_qdc;
-  const int q = blockIdx.x / nprobe, p = blockIdx.x % nprobe;
-  const int l = probes[(size_t)q * nprobe + p];
+  __shared__ float s_qdc[METRIC == 1 ? IVF_PGMAX : 1];
+  const int q = blockIdx.x / groups, g = blockIdx.x % groups;
+  const int p0 = g * pg, p1 = min(nprobe, p0 + pg);
   const float* qv = Qp + (size_t)q * ld;
-  const float* cv = cents + (size_t)l * ld;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  float* const sres = lut + M * 256;
 
-  if constexpr (METRIC == 1) {
-    // q . c for the cosine decomposition (ivfpq.rs:1068-1072, dot_unrolled)
-    if (tid < 8) {
-      const float d = -dist_group8<2>(qv, cv, dim, tid);
-      if (tid == 0) s_qdc = d;
-    }
-  }
   // Distance table (product.rs:416-433). L2: on the residual q - c
-  // (ivfpq.rs:1052-1054); cosine: on the query itself (shared table).
-  for (int e = tid; e < M * 256; e += 256) {
-    const int s = e >> 8, c = e & 255;
-    const int w_s = sub_off[s + 1] - sub_off[s];
-    const float* b = books + book_off[s] + c * w_s;
-    const int o = sub_off[s];
-    float acc = 0.0f;
-    for (int j = 0; j < w_s; ++j) {
-      if constexpr (METRIC == 0) {
-        const float r = qv[o + j] - cv[o + j];
-        const float d = r - b[j];
-        acc += d * d;
-      } else {
-        acc += qv[o + j] * b[j];
-      }
+  // (ivfpq.rs:1052-1054); cosine: on the query itself.
+  auto build = [&](const float* cv) {
+    if (staged) {
+      for (int j = tid; j < dim; j += 256) sres[j] = METRIC == 0 ? qv[j] - cv[j] : qv[j];
+      __syncthreads();
     }
-    lut[e] = acc;
+    for (int e = tid; e < M * 256; e += 256) {
+      const int s = e >> 8, c = e & 255;
+      const int o = sub_off[s], w_s = sub_off[s + 1] - o, bo = book_off[s];
+      const float* b = books + bo + c * w_s;
+      float acc = 0.0f;
+      auto add = [&](float r, float x) {
+        if constexpr (METRIC == 0) {
+          const float d = r - x;
+          acc += d * d;
+        } else {
+          acc += r * x;
+        }
+      };
+      if (staged && ((w_s | bo | o) & 3) == 0) {
+        for (int j = 0; j < w_s; j += 4) {
+          const float4 x = *reinterpret_cast<const float4*>(b + j);
+          const float4 r = *reinterpret_cast<const float4*>(sres + o + j);
+          add(r.x, x.x);
+          add(r.y, x.y);
+          add(r.z, x.z);
+          add(r.w, x.w);
+        }
+      } else {
+        for (int j = 0; j < w_s; ++j)
+          add(staged ? sres[o + j] : (METRIC == 0 ? qv[o + j] - cv[o + j] : qv[o + j]), b[j]);
+      }
+      lut[e] = acc;
+    }
+  };
+  if constexpr (METRIC == 1) {
+    // q . c of every probe for the cosine decomposition (ivfpq.rs:1068-1072,
+    // dot_unrolled), eight threads each
+    for (int i = tid >> 3; i < p1 - p0; i += 32) {
+      const float d = -dist_group8<2>(qv, cents + (size_t)probes[(size_t)q * nprobe + p0 + i] * ld, dim, tid & 7);
+      if ((tid & 7) == 0) s_qdc[i] = d;
+    }
+    build(qv);
   }
-  __syncthreads();
-  const float one_minus_qdc = METRIC == 1 ? arm_nan(1.0f - s_qdc) : 0.0f;
 
   uint64_t* wb = wbuf[w];
   uint64_t thr = KEY_MAX;
   int cnt = 0;
-  const uint32_t begin = list_beg[l], end = list_end[l];
-  for (uint32_t e0 = begin + w * 64; e0 < end; e0 += 256) {
-    const uint32_t e = e0 + lane;
-    uint64_t key = KEY_MAX;
-    if (e < end) {
-      const uint32_t sl = list_slot[e];
-      if (accept == nullptr || accept[sl]) {
-        const uint32_t rk = slot_rank[sl];
+  for (int p = p0; p < p1; ++p) {
+    const int l = probes[(size_t)q * nprobe + p];
+    if constexpr (METRIC == 0) {
+      if (p > p0) __syncthreads();  // the previous probe's lookups are done
+      build(cents + (size_t)l * ld);
+    }
+    if (METRIC == 0 || p == p0) __syncthreads();
+    const float one_minus_qdc = METRIC == 1 ? arm_nan(1.0f - s_qdc[p - p0]) : 0.0f;
+    const uint32_t begin = list_beg[l], end = list_end[l];
+    for (uint32_t e0 = begin + w * 64; e0 < end; e0 += 256) {
+      const uint32_t e = e0 + lane;
+      uint64_t key = KEY_MAX;
+      if (e < end) {
         const uint8_t* code = list_codes + (size_t)e * M;
         float sum = 0.0f;  // DistanceTable::squared_l2 / inner_product, product.rs:580-603
         if (M == 16) {
@@ -190,26 +227,37 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
           const uint32_t wv[4] = {cw.x, cw.y, cw.z, cw.w};
 #pragma unroll
           for (int s = 0; s < 16; ++s) sum += lut[s * 256 + ((wv[s >> 2] >> (8 * (s & 3))) & 255)];
+        } else if ((M & 3) == 0) {
+          for (int s = 0; s < M; s += 4) {
+            const uint32_t cw = *reinterpret_cast<const uint32_t*>(code + s);
+            sum += lut[s * 256 + (cw & 255)];
+            sum += lut[s * 256 + 256 + ((cw >> 8) & 255)];
+            sum += lut[s * 256 + 512 + ((cw >> 16) & 255)];
+            sum += lut[s * 256 + 768 + (cw >> 24)];
+          }
         } else {
           for (int s = 0; s < M; ++s) sum += lut[s * 256 + code[s]];
         }
-        const float score = METRIC == 0 ? sum : ivf_cos_score(one_minus_qdc, sum);
-        key = ((uint64_t)ord_key(score) << 32) | rk;
+        const uint32_t dk = ord_key(METRIC == 0 ? sum : ivf_cos_score(one_minus_qdc, sum));
+        if (dk <= (uint32_t)(thr >> 32)) {
+          const uint32_t sl = list_slot[e];
+          if (accept == nullptr || accept[sl]) key = ((uint64_t)dk << 32) | slot_rank[sl];
+        }
       }
-    }
-    const bool pass = key < thr;
-    const uint64_t mask = __ballot(pass);
-    const int pos = cnt + __popcll(mask & ((1ull << lane) - 1));
-    if (pass) wb[pos] = key;
-    cnt += __popcll(mask);
-    if (cnt > CAPW - 64) {
-      wave_compact<CAPW>(wb, cnt, kk, lane);
-      cnt = kk;
-      thr = wb[kk - 1];
+      const bool pass = key < thr;
+      const uint64_t mask = __ballot(pass);
+      const int pos = cnt + __popcll(mask & ((1ull << lane) - 1));
+      if (pass) wb[pos] = key;
+      cnt += __popcll(mask);
+      if (cnt > CAPW - 64) {
+        wave_compact<CAPW>(wb, cnt, kk, lane);
+        cnt = kk;
+        thr = wb[kk - 1];
+      }
     }
   }
   wave_compact<CAPW>(wb, cnt, kk, lane);
-  uint64_t* o = out + (((size_t)q * nprobe + p) * 4 + w) * kk;
+  uint64_t* o = out + (((size_t)q * groups + g) * 4 + w) * kk;
   for (int i = lane; i < kk; i += 64) o[i] = i < cnt ? wb[i] : KEY_MAX;
 }
 
@@ -686,7 +734,6 @@ __global__ void ivf_transpose_cents(const float* __restrict__ C, int ld, int dim
   cT[t] = c < produced ? C[(size_t)c * ld + i] : 0.0f;
 }
 
-constexpr int IVF_PGMAX = 32;   // probes per scan workgroup, at most
 constexpr int IVF_SW = 8;       // waves per scan workgroup
 
 // ADC scan, register-resident codebooks (uniform subspace width W, M*W = dim
@@ -1229,6 +1276,11 @@ __global__ __launch_bounds__(IVF_SW * 64) void ivf_scan16(const float* __restric
 // ---------------------------------------------------------------------------
 constexpr int IVF_MAX_SHORT = 960;
 
+// PER > 0: the query's keys fit PER per thread and are read once; the select
+// starts at the highest bit in which they differ. 0: any number, read on every
+// pass. 100 queries, shortlist 100, exact rerank: 56 us over 6400 keys (one
+// list per probe and wave) -> 28.5 us over 3200.
+template <int PER>
 __global__ __launch_bounds__(256) void ivf_merge(const uint64_t* __restrict__ cand, int n_per_q, int kk, int k,
                                                  int rerank, const float* __restrict__ Qp, int ld, int dim,
                                                  int metric, const float* __restrict__ X,
@@ -1241,39 +1293,61 @@ __global__ __launch_bounds__(256) void ivf_merge(const uint64_t* __restrict__ ca
   __shared__ uint64_t sel[1024];
   __shared__ int n_sel, n_valid;
   const uint64_t* base = cand + (size_t)q * n_per_q;
-  auto get = [&](int i) -> uint64_t { return base[i]; };
   if (threadIdx.x == 0) {
     n_sel = 0;
     n_valid = 0;
   }
-  __syncthreads();
+  uint64_t v[PER > 0 ? PER : 1], lo = KEY_MAX, hi = 0;
   int local = 0;
-  // four keys per thread per step, loaded together before any is used
-  for (int i0 = threadIdx.x; i0 < n_per_q; i0 += 4 * blockDim.x) {
-    uint64_t x[4];
+  if constexpr (PER > 0) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = base[min(i0 + u * (int)blockDim.x, n_per_q - 1)];
+    for (int j = 0; j < PER; ++j) v[j] = base[min((int)threadIdx.x + j * 256, n_per_q - 1)];  // unconditional loads
 #pragma unroll
-    for (int u = 0; u < 4; ++u) local += (i0 + u * (int)blockDim.x < n_per_q && x[u] != KEY_MAX) ? 1 : 0;
+    for (int j = 0; j < PER; ++j) {
+      if ((int)threadIdx.x + j * 256 >= n_per_q) v[j] = KEY_MAX;
+      if (v[j] != KEY_MAX) {
+        ++local;
+        lo = min(lo, v[j]);
+        hi = max(hi, v[j]);
+      }
+    }
   }
-  atomicAdd(&n_valid, local);
+  // every key of this thread, in order: f(x)
+  auto each = [&](auto f) {
+    if constexpr (PER > 0) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (v[j] != KEY_MAX) f(v[j]);
+    } else {
+      // four keys per thread per step, loaded together before any is used
+      for (int i0 = threadIdx.x; i0 < n_per_q; i0 += 4 * 256) {
+        uint64_t x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = base[min(i0 + u * 256, n_per_q - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i0 + u * 256 < n_per_q && x[u] != KEY_MAX) f(x[u]);
+      }
+    }
+  };
+  if constexpr (PER == 0)
+    each([&](uint64_t x) {
+      ++local;
+      lo = min(lo, x);
+      hi = max(hi, x);
+    });
+  __syncthreads();
+  if (local) atomicAdd(&n_valid, local);
   __syncthreads();
   const int ksel = min(kk, n_valid);
   if (ksel == 0) {
     if (threadIdx.x == 0) out_count[q] = 0;
     return;
   }
-  const uint64_t pivot = n_per_q <= 16 * (int)blockDim.x
-                             ? block_radix_select<decltype(get), 64, 16>(get, n_per_q, ksel, hist, sh)
-                             : block_radix_select(get, n_per_q, ksel, hist, sh);
-  for (int i0 = threadIdx.x; i0 < n_per_q; i0 += 4 * blockDim.x) {
-    uint64_t x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = base[min(i0 + u * (int)blockDim.x, n_per_q - 1)];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u * (int)blockDim.x < n_per_q && x[u] <= pivot && x[u] != KEY_MAX) sel[atomicAdd(&n_sel, 1)] = x[u];
-  }
+  const uint64_t pivot = block_radix_select_range<256>(each, lo, hi, ksel, hist, sh);
+  each([&](uint64_t x) {
+    if (x <= pivot) sel[atomicAdd(&n_sel, 1) & 1023] = x;
+  });
   __syncthreads();
   int P = 1;
   while (P < ksel) P <<= 1;
@@ -2446,7 +2520,13 @@ struct IvfPqIndex {
       const uint64_t shortlist =
           std::min<uint64_t>(cfg.rerank > 0 ? std::max<uint64_t>(cfg.rerank, kq) : kq, by_id.size());
       // beyond the block selections, or tables beyond the LDS: sorted segments
-      const bool wide = shortlist > IVF_MAX_SHORT || M() > IVF_MAX_M;
+      // (the general scan's LDS: the table, four candidate lists, and for
+      // cosine the probes' products; 128 cosine subspaces with a shortlist
+      // above 448 are 128 bytes past the 160 KB)
+      const size_t scan_lds = (size_t)M() * 1024 +
+                              (size_t)4 * (shortlist <= 192 ? 256 : shortlist <= 448 ? 512 : 1024) * 8 +
+                              (metric == PXG_COSINE ? IVF_PGMAX * 4 : 0);
+      const bool wide = shortlist > IVF_MAX_SHORT || M() > IVF_MAX_M || scan_lds > IVF_LDS;
       const int kk = (int)std::min<uint64_t>(shortlist, IVF_MAX_SHORT);
       uint64_t* ck = (uint64_t*)sc.get(8, (size_t)nq * produced * 8);
       int* probes = (int*)sc.get(9, (size_t)nq * np * 4);
@@ -2509,6 +2589,21 @@ struct IvfPqIndex {
                              (metric == PXG_COSINE || M() <= 64);
       const bool staged16 = reg_shape && M() == 16 && kk <= 128;
       const bool reg_path = reg_shape && (kk <= 64 || staged16);
+      auto merge = [&](const uint64_t* cand, int n_per_q) {
+#define PXG_IVF_MERGE(PERV)                                                                                       \
+  hipLaunchKernelGGL(ivf_merge<PERV>, dim3((unsigned)nq), dim3(256), 0, s, cand, n_per_q, kk, (int)ldo,           \
+                     rerank ? 1 : 0, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank_slot.p, d_ids.p, d_oid, d_od, \
+                     d_oc)
+        if (n_per_q <= 4 * 256)
+          PXG_IVF_MERGE(4);
+        else if (n_per_q <= 16 * 256)
+          PXG_IVF_MERGE(16);
+        else if (n_per_q <= 32 * 256)
+          PXG_IVF_MERGE(32);
+        else
+          PXG_IVF_MERGE(0);
+#undef PXG_IVF_MERGE
+      };
       if (reg_path) {
         const size_t lds = (size_t)(metric == PXG_COSINE ? 1 : 2) * M() * 256 * 4;
         // probes per workgroup: up to IVF_PGMAX, fewer when that would leave
@@ -2572,9 +2667,7 @@ struct IvfPqIndex {
         PXG_HIP(hipGetLastError());
         tm.mark(2);
         if (!fused) {
-          hipLaunchKernelGGL(ivf_merge, dim3((unsigned)nq), dim3(256), 0, s, cand, groups * IVF_SW * kk, kk, (int)ldo,
-                             rerank ? 1 : 0, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank_slot.p, d_ids.p, d_oid, d_od,
-                             d_oc);
+          merge(cand, groups * IVF_SW * kk);
           PXG_HIP(hipGetLastError());
         }
       } else if (wide) {
@@ -2583,14 +2676,21 @@ struct IvfPqIndex {
                                            s, ldo);
         scanned_dev = nullptr;
       } else {
-      const size_t lds = (size_t)M() * 256 * 4;
-      uint64_t* cand = (uint64_t*)sc.get(10, (size_t)nq * np * 4 * kk * 8);
-      const int grid = (int)(nq * np);
+      // probes per workgroup as on the register path; the query (or residual)
+      // is staged beside the table where the LDS holds both
+      int pg = IVF_PGMAX;
+      while (pg > 1 && (int64_t)nq * ((np + pg - 1) / pg) < 512) pg >>= 1;
+      const int groups = (np + pg - 1) / pg;
+      const size_t table = (size_t)M() * 256 * 4;
+      const int staged = scan_lds + dim * 4 + 64 <= IVF_LDS ? 1 : 0;
+      const size_t lds = table + (staged ? (size_t)dim * 4 : 0);
+      uint64_t* cand = (uint64_t*)sc.get(10, (size_t)nq * groups * 4 * kk * 8);
+      const int grid = (int)(nq * groups);
       tm.mark(1);
 #define PXG_SCAN(CAPW, MET)                                                                                       \
   hipLaunchKernelGGL((ivf_scan<CAPW, MET>), dim3(grid), dim3(256), lds, s, Qp, (int)ld, (int)dim, (int)M(), probes, \
-                     np, cents.p, books.p, d_sub_off.p, d_book_off.p, list_beg.p, list_end.p, list_slot.p, list_codes.p,       \
-                     ranks.rank_slot.p, ranks.rank.p, d_accept, kk, cand)
+                     np, pg, groups, staged, cents.p, books.p, d_sub_off.p, d_book_off.p, list_beg.p, list_end.p,  \
+                     list_slot.p, list_codes.p, ranks.rank_slot.p, ranks.rank.p, d_accept, kk, cand)
       if (kk <= 192) {
         if (metric == PXG_COSINE) PXG_SCAN(256, 1); else PXG_SCAN(256, 0);
       } else if (kk <= 448) {
@@ -2601,9 +2701,7 @@ struct IvfPqIndex {
 #undef PXG_SCAN
       PXG_HIP(hipGetLastError());
       tm.mark(2);
-      hipLaunchKernelGGL(ivf_merge, dim3((unsigned)nq), dim3(256), 0, s, cand, np * 4 * kk, kk, (int)ldo,
-                         rerank ? 1 : 0, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank_slot.p, d_ids.p, d_oid, d_od,
-                         d_oc);
+      merge(cand, groups * 4 * kk);
       PXG_HIP(hipGetLastError());
       }
     }

@@ -633,3 +633,31 @@ def test_list_view_growth_and_compaction(gpu):
     assert_same(idx.search_batch(q, 5, nprobe=2),
                 orc.ivf_search(0, cents, books, codes3, list_of3, ids, q, 5, 2, m, live=live, threads=8))
     assert idx.view_stats()[0] == r1 + 1
+
+
+@pytest.mark.parametrize("metric", [0, 1])
+@pytest.mark.parametrize("dim,m,k,rerank,nq", [(50, 7, 70, 0, 5), (96, 12, 10, 100, 3), (96, 12, 10, 100, 700),
+                                               (64, 16, 300, 0, 9), (128, 128, 500, 0, 6), (44, 11, 10, 800, 3),
+                                               (24, 6, 80, 90, 530)])
+def test_general_scan_probe_groups(gpu, metric, dim, m, k, rerank, nq):
+    """The general scan with one and with several probes per workgroup, widths
+    that are and are not multiples of four, uneven widths, tables that leave
+    no LDS to stage the query beside them, shortlists of every buffer size and
+    merges of every size, against the oracle bit for bit; then with a filter."""
+    rng = np.random.default_rng(dim + m)
+    n, nlist = 2400, 24
+    data = corpus(n, dim, 24) + rng.standard_normal((n, dim)).astype(np.float32) * 0.3
+    prep = orc.prepare_rows(metric, data)
+    cents, books, _ = orc.ivf_train(prep, nlist, m, max_iter=3, seed=5)
+    codes, list_of = orc.ivf_encode(prep, cents, books, m)
+    idx = build(gpu, data, gpu.IvfPqConfig(nlist, m).with_train_threshold(1 << 62).with_rerank(rerank), metric)
+    idx.load_trained(cents, books, codes, list_of)
+    q = (data[rng.integers(0, n, nq)] + 0.05).astype(np.float32)
+    qp = orc.prepare_rows(metric, q)
+    accept = (rng.random(n) < 0.5).astype(np.uint8)
+    for nprobe in (1, 5, 24):
+        kw = dict(vectors=prep if rerank else None, rerank=rerank, threads=8)
+        want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), qp, k, nprobe, m, **kw)
+        assert_same(idx.search_batch(q, k, nprobe=nprobe), want)
+    want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), qp, k, 5, m, accept=accept, **kw)
+    assert_same(idx.search_batch(q, k, lambda i, _m: bool(accept[i]), nprobe=5), want)
