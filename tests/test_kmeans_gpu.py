@@ -298,6 +298,22 @@ def test_pq_train_and_encode_bit_exact(gpu, dim, m, count, seed):
     assert np.array_equal(pq.encode(t), orc.pq_encode(books, dim, m, t))
 
 
+@pytest.mark.parametrize("dim,m", [(6, 3), (32, 8), (30, 5), (64, 8), (36, 3), (48, 3), (48, 2), (64, 2), (50, 4), (80, 2)])
+def test_pq_encode_widths(gpu, dim, m):
+    """Equal widths with a kernel of their own (2 to 32), uneven ones and one
+    above them, at a ragged count, with codewords at equal distance."""
+    px = gpu
+    rng = np.random.default_rng(dim * 100 + m)
+    t = rng.standard_normal((700, dim)).astype(np.float32)
+    pq = px.ProductQuantizer.train(px.VectorSpace(dim, px.Metric.EUCLIDEAN), t, px.PqConfig(m).with_seed(3))
+    books = pq.codebooks
+    x = rng.standard_normal((1301, dim)).astype(np.float32)
+    x[::7] = 0.5 * (t[0] + t[1])
+    x[3] = np.inf
+    x[5, 0] = np.nan
+    assert np.array_equal(pq.encode(x), orc.pq_encode(books, dim, m, x))
+
+
 @pytest.mark.parametrize("after", [0, 5])
 def test_pq_train_in_order_path(gpu, monkeypatch, after):
     """The subspaces seed at once from predicted generator states; the
