@@ -2390,15 +2390,29 @@ static void launch_farthest(const float* dist, size_t n, unsigned long long* par
 // point is in it), so that array's row w is its old centroid if w > E[i] and
 // its new mean if w < E[i], and the point's nearest distance there is at
 // most ub_i = d_old or squared(p, new_w) accordingly; a NaN distance
-// (overflow) counts as +inf, and a nearest distance is never NaN. Take as
-// the pool the points of the largest ub_i and let theta be the largest ub_i
-// outside it: every point outside has distance <= theta. So if the largest
-// exact distance over the pool is above theta, the farthest point (the
-// first index among equal distances) is in the pool, and is the pool's. Each
-// empty cluster then costs a sort of the bounds and an exact scan of the
-// pool instead of passes over every point; if the test fails at any empty
-// cluster, the segment passes redo them all.
-constexpr size_t RESEED_POOL = 8192;
+// (overflow) counts as +inf, and a nearest distance is never NaN. The points
+// are binned by the upper 16 bits of ub; the pool is the points of the largest
+// bins that hold at most PL points together, and theta the largest bound that
+// the bins left out can hold: every point outside the pool has distance <=
+// theta. So if the largest exact distance over the pool is above theta, the
+// farthest point (the first index among equal distances) is in the pool, and
+// is the pool's. An empty cluster then costs an exact scan of its pool and a
+// reduction instead of passes over every point; if the test fails at any
+// empty cluster, the segment passes redo them all. The bounds don't depend on
+// the victims, so three launches make the pools of RESEED_BATCH empty
+// clusters (a sort of the bounds takes 40 us at 60k points, per cluster). A
+// victim brings down the points around it, in clustered data about n / k,
+// whose bounds stay: each victim so far adds twice that many points.
+// 60k x 100, 300 clusters, 18 empty ones in 8 iterations: a call 3.2 ms with
+// a sort, two copies of the array, an exact scan of 8192 points and three more
+// launches per empty cluster -> 2.5 ms; 2M x 128, 4096 clusters, 18 empty
+// ones: 0.61 -> 0.24 ms each.
+constexpr size_t RESEED_POOL = 8192;  // points of a pool, at most
+constexpr size_t RESEED_BASE = 1024;  // at the iteration's first empty cluster
+constexpr size_t RESEED_BATCH = 32;   // empty clusters whose pools are made together (4 MB of counts)
+constexpr int RESEED_BINS = 32768;    // upper 16 bits of a float >= 0
+constexpr int RESEED_TILE = 8192;     // points per workgroup of the two passes
+constexpr int KP_WAVES = 8;           // of a workgroup of the pool's exact scan
 
 // squared(p, new_w) per point (NaN as +inf): the reference's sequential sum,
 // staged through LDS as in km_mfma_verify (rows 16-byte aligned, dim a
@@ -2439,40 +2453,208 @@ __global__ __launch_bounds__(256) void km_reseed_bound(const float* __restrict__
   if (t < KV_PB && i < n) dnew[i] = sum == sum ? sum : INFINITY;
 }
 
-// ub_i per point as a descending sort key (~ its bits; ub_i >= 0), with the
-// point's index as the value, for the empty cluster e.
-__global__ __launch_bounds__(256) void km_reseed_keys(const uint32_t* __restrict__ assign,
-                                                      const float* __restrict__ dold, const float* __restrict__ dnew,
-                                                      int n, uint32_t e, uint32_t* __restrict__ key,
-                                                      uint32_t* __restrict__ idx) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float ub = assign[i] > e ? dold[i] : dnew[i];
-  key[i] = ~__float_as_uint(ub + 0.0f);
-  idx[i] = (uint32_t)i;
+// Points per bin of ub for the empty cluster E[blockIdx.y]: 16-bit counts in
+// LDS (a workgroup has 8192 points), added to the global ones where not zero.
+__device__ __forceinline__ uint32_t reseed_bin(const uint32_t* assign, const float* dold, const float* dnew, int i,
+                                               uint32_t e) {
+  return __float_as_uint((assign[i] > e ? dold[i] : dnew[i]) + 0.0f) >> 16;
+}
+__global__ __launch_bounds__(1024) void km_reseed_hist(const uint32_t* __restrict__ assign,
+                                                       const float* __restrict__ dold, const float* __restrict__ dnew,
+                                                       int n, const uint32_t* __restrict__ E,
+                                                       uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[RESEED_BINS / 2];
+  const int tid = threadIdx.x;
+  const uint32_t e = E[blockIdx.y];
+  hist += (size_t)blockIdx.y * RESEED_BINS;
+  for (int t = tid; t < RESEED_BINS / 2; t += 1024) h[t] = 0;
+  __syncthreads();
+  const int i0 = blockIdx.x * RESEED_TILE, i1 = min(n, i0 + RESEED_TILE);
+  for (int i = i0 + tid; i < i1; i += 1024) {
+    const uint32_t b = reseed_bin(assign, dold, dnew, i, e);
+    atomicAdd(&h[b >> 1], 1u << (16 * (b & 1)));
+  }
+  __syncthreads();
+  for (int t = tid; t < RESEED_BINS / 2; t += 1024) {
+    const uint32_t v = h[t];
+    if (v & 0xFFFFu) atomicAdd(hist + 2 * t, v & 0xFFFFu);
+    if (v >> 16) atomicAdd(hist + 2 * t + 1, v >> 16);
+  }
 }
 
-// The pool's farthest point: the largest distance, then the smallest index
-// (the largest key, as in km_farthest_part). *fail is set unless that
-// distance is above theta = the largest ub outside the pool (theta_key holds
-// its sort key; none when the pool holds every point).
-__global__ __launch_bounds__(256) void km_pool_farthest(const uint32_t* __restrict__ rows,
-                                                        const float* __restrict__ d, int m,
-                                                        const uint32_t* __restrict__ theta_key, int force_fail,
-                                                        long long* __restrict__ out, int* __restrict__ fail) {
-  __shared__ unsigned long long sh[4];
+// cut[b]: the lowest bin of cluster b's bounds with at most PL points above
+// it. One workgroup per cluster, 32 bins per thread from the top; the pools'
+// counts are cleared.
+__global__ __launch_bounds__(1024) void km_reseed_cut(const uint32_t* __restrict__ hist, uint32_t PL0, uint32_t per,
+                                                      uint32_t pool_max,
+                                                      uint32_t* __restrict__ cut, uint32_t* __restrict__ count) {
+  __shared__ uint32_t sw[16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int top = RESEED_BINS - 1 - tid * 32;
+  const uint32_t PL = min(pool_max, PL0 + blockIdx.x * per);
+  hist += (size_t)blockIdx.x * RESEED_BINS;
+  uint32_t v[32], sum = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const uint4 x = *reinterpret_cast<const uint4*>(hist + top - 4 * q - 3);
+    v[4 * q] = x.w; v[4 * q + 1] = x.z; v[4 * q + 2] = x.y; v[4 * q + 3] = x.x;
+    sum += x.x + x.y + x.z + x.w;
+  }
+  uint32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o, WAVE);
+    if (lane >= o) incl += y;
+  }
+  if (lane == 63) sw[w] = incl;
+  __syncthreads();
+  uint32_t above = incl - sum;
+  for (int j = 0; j < w; ++j) above += sw[j];
+  // the bins down to the first that would take the count over PL (n > PL, so
+  // there is one); its thread writes it
+  if (above <= PL && above + sum > PL) {
+    uint32_t acc = above;
+    int at = 0;
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      at = acc <= PL ? q : at;
+      acc += v[q];
+    }
+    cut[blockIdx.x] = (uint32_t)(top - at);
+  }
+  if (tid == 0) count[blockIdx.x] = 0;
+}
+
+// The points of the bins above the cut, in no particular order: a workgroup's
+// points are gathered in LDS and placed by one addition to the pool's count.
+__global__ __launch_bounds__(1024) void km_reseed_list(const uint32_t* __restrict__ assign,
+                                                       const float* __restrict__ dold, const float* __restrict__ dnew,
+                                                       int n, const uint32_t* __restrict__ E,
+                                                       const uint32_t* __restrict__ cut, int PL,
+                                                       uint32_t* __restrict__ count, uint32_t* __restrict__ list) {
+  __shared__ uint32_t ids[RESEED_TILE];
+  __shared__ uint32_t s_n, s_at;
+  const int tid = threadIdx.x;
+  const uint32_t e = E[blockIdx.y], cb = cut[blockIdx.y];
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  const int i0 = blockIdx.x * RESEED_TILE, i1 = min(n, i0 + RESEED_TILE);
+  for (int i = i0 + tid; i < i1; i += 1024)
+    if (reseed_bin(assign, dold, dnew, i, e) > cb) ids[atomicAdd(&s_n, 1u)] = (uint32_t)i;
+  __syncthreads();
+  const uint32_t m = s_n;
+  if (m == 0) return;
+  if (tid == 0) s_at = atomicAdd(count + blockIdx.y, m);
+  __syncthreads();
+  for (uint32_t t = tid; t < m; t += 1024) list[(size_t)blockIdx.y * PL + s_at + t] = ids[t];
+}
+
+// Exact nearest distances of a pool, for the array of the new means below row
+// e and the old rows from it on; the reference's sequential sums. Eight points
+// per workgroup, in LDS (rows four floats apart in their banks); a wave takes
+// 16 centroids at a time, four adjacent lanes to a centroid with two points
+// each: a load then takes 16 lines, and the eight waves' lines fit L1 (12 us for
+// 1024 points, 300 clusters of 100; with a lane per centroid 21, with the
+// centroid's lanes 16 apart 19). Rows 16-byte aligned, dim a multiple of 4.
+__global__ __launch_bounds__(KP_WAVES * WAVE) void km_exact_pool(const float* __restrict__ P, int ldp,
+                                                                 const uint32_t* __restrict__ list,
+                                                                 const uint32_t* __restrict__ count, uint32_t e,
+                                                                 int dim, const float* __restrict__ newc,
+                                                                 const float* __restrict__ cents, int k,
+                                                                 float* __restrict__ out) {
+  extern __shared__ float4 kp_sm[];
+  const float* sp = reinterpret_cast<const float*>(kp_sm);  // [KX_PB][dim + 4]
+  __shared__ float sbd[KP_WAVES][KX_PB];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int p0 = blockIdx.x * KX_PB, np = min(KX_PB, (int)*count - p0);
+  if (np <= 0) return;
+  const int d4 = dim >> 2, ls = dim + 4;
+  for (int t = tid; t < KX_PB * d4; t += KP_WAVES * WAVE) {
+    const int i = t / d4, j = t - i * d4;
+    kp_sm[i * (d4 + 1) + j] = *reinterpret_cast<const float4*>(P + (size_t)list[p0 + min(i, np - 1)] * ldp + 4 * j);
+  }
+  __syncthreads();
+  const int g = (lane & 3) * 2;  // the lane's two points
+  const float* a = sp + g * ls;
+  const float* b = a + ls;
+  float ba = INFINITY, bb = INFINITY;
+  for (int c = w * 16 + (lane >> 2); c < k; c += KP_WAVES * 16) {
+    const float* cr = (c < (int)e ? newc : cents) + (size_t)c * dim;
+    float sa = 0.0f, sb = 0.0f;
+#pragma unroll 4
+    for (int j = 0; j < dim; j += 4) {
+      const float4 y = *reinterpret_cast<const float4*>(cr + j);
+      const float4 x = *reinterpret_cast<const float4*>(a + j);
+      const float4 z = *reinterpret_cast<const float4*>(b + j);
+      float d = x.x - y.x;
+      sa += d * d;
+      d = z.x - y.x;
+      sb += d * d;
+      d = x.y - y.y;
+      sa += d * d;
+      d = z.y - y.y;
+      sb += d * d;
+      d = x.z - y.z;
+      sa += d * d;
+      d = z.z - y.z;
+      sb += d * d;
+      d = x.w - y.w;
+      sa += d * d;
+      d = z.w - y.w;
+      sb += d * d;
+    }
+    if (sa < ba) ba = sa;
+    if (sb < bb) bb = sb;
+  }
+#pragma unroll
+  for (int o = 4; o < 64; o <<= 1) {
+    ba = fminf(ba, __shfl_xor(ba, o, WAVE));
+    bb = fminf(bb, __shfl_xor(bb, o, WAVE));
+  }
+  if (lane < 4) {
+    sbd[w][g] = ba;
+    sbd[w][g + 1] = bb;
+  }
+  __syncthreads();
+  if (tid < np) {
+    float m = sbd[0][tid];
+#pragma unroll
+    for (int v = 1; v < KP_WAVES; ++v) m = fminf(m, sbd[v][tid]);
+    out[p0 + tid] = m;
+  }
+}
+
+// The pool's farthest point (the first index among equal distances), whose
+// row becomes row e of the new array; *fail is set where theta is not below
+// its distance (or the test hook asks for it). Distances compare as their
+// bits (all >= 0), theta as the cut's bits with every lower bit set.
+__global__ __launch_bounds__(1024) void km_pool_farthest(const float* __restrict__ P, int ldp, int dim,
+                                                         const uint32_t* __restrict__ list,
+                                                         const uint32_t* __restrict__ count,
+                                                         const float* __restrict__ d,
+                                                         const uint32_t* __restrict__ cut, int force_fail,
+                                                         float* __restrict__ row_out, int* __restrict__ fail) {
+  __shared__ unsigned long long sh[16];
+  const int tid = threadIdx.x, m = (int)*count;
   unsigned long long best = 0;
-  for (int j = threadIdx.x; j < m; j += 256) {
+#pragma unroll 4
+  for (int j = tid; j < m; j += 1024) {
     const unsigned long long key =
-        ((unsigned long long)__float_as_uint(d[j] + 0.0f) << 32) | (0xFFFFFFFFu - rows[j]);
+        ((unsigned long long)__float_as_uint(d[j] + 0.0f) << 32) | (0xFFFFFFFFu - list[j]);
     best = key > best ? key : best;
   }
-  best = block_max_u64_256(best, sh);
-  if (threadIdx.x == 0) {
-    *out = (long long)(0xFFFFFFFFu - (uint32_t)best);
-    const float dmax = __uint_as_float((uint32_t)(best >> 32));
-    if (force_fail || (theta_key && !(dmax > __uint_as_float(~*theta_key)))) *fail = 1;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long y = shfl_xor64(best, o);
+    best = y > best ? y : best;
   }
+  if ((tid & 63) == 0) sh[tid >> 6] = best;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) best = sh[w] > best ? sh[w] : best;
+  const uint32_t row = best != 0 ? 0xFFFFFFFFu - (uint32_t)best : 0u;  // an empty pool fails the test below
+  for (int j = tid; j < dim; j += 1024) row_out[j] = P[(size_t)row * ldp + j];
+  if (tid == 0 && (force_fail || (uint32_t)(best >> 32) <= ((*cut << 16) | 0xFFFFu))) *fail = 1;
 }
 
 // Optional phase timings on stderr (PXG_TRAIN_VERBOSE=1), for tuning.
@@ -2513,19 +2695,19 @@ KmeansOut kmeans_device(const float* P, size_t n, int dim, int ldp, size_t k_req
   DevBuf<float> dist(n), newc(k * dim), work(k * dim);
   DevBuf<int> changed(1), pool_fail(1);
   DevBuf<long long> far(1);
-  // the reseed pool's bounds, their sorted order, and the pool's exact scan
-  DevBuf<uint32_t> rs_key, rs_skey, rs_idx, rs_rows, pool_a;
+  // the reseed pool's bounds, their counts and lists, and the pool's exact scan
+  DevBuf<uint32_t> rs_hist, rs_list, rs_e;  // rs_e: clusters, cuts, counts
   DevBuf<float> rs_dnew, pool_d;
   size_t pool_reseeds = 0, pool_fallbacks = 0;
   // PXG_RESEED_POOL=size sets the pool size (0: no pool), so that small
   // inputs can take the pool path; PXG_RESEED_FAIL_AT=i fails the pool's test
   // at empty cluster i, so that the fallback runs after victims were placed
   // (test hooks; the results are the same either way)
-  size_t pool = RESEED_POOL;
-  if (const char* e = std::getenv("PXG_RESEED_POOL")) pool = (size_t)std::strtoull(e, nullptr, 10);
+  size_t pool_max = RESEED_POOL;
+  if (const char* e = std::getenv("PXG_RESEED_POOL")) pool_max = (size_t)std::strtoull(e, nullptr, 10);
   const char* fail_env = std::getenv("PXG_RESEED_FAIL_AT");
   const long long fail_at = fail_env ? std::atoll(fail_env) : -1;
-  const bool pool_fits = pool > 0 && n > 4 * pool && dim % 4 == 0 && dim <= KW_DMAX && ldp % 4 == 0 &&
+  const bool pool_fits = pool_max > 0 && n > 4 * pool_max && dim % 4 == 0 && dim <= KW_DMAX && ldp % 4 == 0 &&
                          ((uintptr_t)P & 15) == 0;
   DevBuf<unsigned long long> far_part(KF_BLOCKS);
   NearestWork nw;  // the points do not change during the run
@@ -2589,32 +2771,45 @@ KmeansOut kmeans_device(const float* P, size_t n, int dim, int ldp, size_t k_req
       if (h_counts[c] == 0) E.push_back(c);
     const size_t m = E.size();
     if (m >= 1 && pool_fits) {
-      rs_key.reserve(n);
-      rs_skey.reserve(n);
-      rs_idx.reserve(n);
-      rs_rows.reserve(n);
+      const size_t per = 2 * ((n + k - 1) / k);
+      const auto pool_at = [&](size_t i) { return std::min(pool_max, RESEED_BASE + i * per); };
+      const size_t pool = pool_at(m - 1);
+      const size_t mb = std::min(m, RESEED_BATCH);
+      rs_hist.reserve(mb * RESEED_BINS);
+      rs_list.reserve(mb * pool);
+      rs_e.reserve(3 * RESEED_BATCH);
       rs_dnew.reserve(n);
-      pool_a.reserve(pool);
       pool_d.reserve(pool);
       hipLaunchKernelGGL(km_reseed_bound, dim3((unsigned)((n + KV_PB - 1) / KV_PB)), dim3(256), 0, s, P, ldp, (int)n,
                          dim, (const float*)newc.p, (const uint32_t*)assign.p, rs_dnew.p);
       PXG_HIP(hipMemsetAsync(pool_fail.p, 0, 4, s));
-      for (size_t ii = 0; ii < m; ++ii) {
-        const size_t c = E[ii];
-        hipLaunchKernelGGL(km_reseed_keys, gn, dim3(256), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
-                           (const float*)rs_dnew.p, (int)n, (uint32_t)c, rs_key.p, rs_idx.p);
-        PXG_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, rs_key.p, rs_skey.p, rs_idx.p, rs_rows.p, (int)n,
-                                                   0, 32, s));
-        PXG_HIP(hipMemcpyAsync(work.p, newc.p, c * dim * 4, hipMemcpyDeviceToDevice, s));
-        PXG_HIP(hipMemcpyAsync(work.p + c * dim, cents.p + c * dim, (k - c) * dim * 4, hipMemcpyDeviceToDevice, s));
-        hipLaunchKernelGGL(km_exact_multi<false>, dim3((unsigned)((pool + KX_PB - 1) / KX_PB)), dim3(256),
-                           (size_t)KX_PB * dim * 4, s, P, ldp, (const uint32_t*)rs_rows.p, (int)pool, dim,
-                           (const float*)work.p, dim, (int)k, pool_a.p, pool_d.p);
-        hipLaunchKernelGGL(km_pool_farthest, dim3(1), dim3(256), 0, s, (const uint32_t*)rs_rows.p,
-                           (const float*)pool_d.p, (int)pool, (const uint32_t*)(rs_skey.p + pool),
-                           (int)((long long)ii == fail_at), far.p, pool_fail.p);
-        hipLaunchKernelGGL(copy_row_at, dim3(1), dim3(256), 0, s, P, ldp, (const long long*)far.p, dim,
-                           newc.p + c * dim);
+      uint32_t* cut = rs_e.p + RESEED_BATCH;
+      uint32_t* cnt = cut + RESEED_BATCH;
+      uint32_t h_e[RESEED_BATCH];
+      for (size_t i0 = 0; i0 < m; i0 += mb) {
+        const size_t b = std::min(mb, m - i0);
+        if (i0 > 0) PXG_HIP(hipStreamSynchronize(s));  // h_e is still being read
+        for (size_t ii = 0; ii < b; ++ii) h_e[ii] = (uint32_t)E[i0 + ii];
+        PXG_HIP(hipMemcpyAsync(rs_e.p, h_e, b * 4, hipMemcpyHostToDevice, s));
+        PXG_HIP(hipMemsetAsync(rs_hist.p, 0, b * RESEED_BINS * 4, s));
+        const dim3 gr((unsigned)((n + RESEED_TILE - 1) / RESEED_TILE), (unsigned)b);
+        hipLaunchKernelGGL(km_reseed_hist, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
+                           (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, rs_hist.p);
+        hipLaunchKernelGGL(km_reseed_cut, dim3((unsigned)b), dim3(1024), 0, s, (const uint32_t*)rs_hist.p,
+                           (uint32_t)pool_at(i0), (uint32_t)per, (uint32_t)pool_max, cut, cnt);
+        hipLaunchKernelGGL(km_reseed_list, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
+                           (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, (const uint32_t*)cut, (int)pool,
+                           cnt, rs_list.p);
+        for (size_t ii = 0; ii < b; ++ii) {
+          const size_t c = E[i0 + ii];
+          const uint32_t* list = rs_list.p + ii * pool;
+          hipLaunchKernelGGL(km_exact_pool, dim3((unsigned)((pool_at(i0 + ii) + KX_PB - 1) / KX_PB)), dim3(KP_WAVES * WAVE),
+                             (size_t)KX_PB * (dim + 4) * 4, s, P, ldp, list, (const uint32_t*)(cnt + ii), (uint32_t)c, dim,
+                             (const float*)newc.p, (const float*)cents.p, (int)k, pool_d.p);
+          hipLaunchKernelGGL(km_pool_farthest, dim3(1), dim3(1024), 0, s, P, ldp, dim, list,
+                             (const uint32_t*)(cnt + ii), (const float*)pool_d.p, (const uint32_t*)(cut + ii),
+                             (int)((long long)(i0 + ii) == fail_at), newc.p + c * dim, pool_fail.p);
+        }
         PXG_HIP(hipGetLastError());
       }
       int h_fail = 0;

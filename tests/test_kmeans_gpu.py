@@ -108,6 +108,25 @@ def test_lloyd_several_empty_clusters_in_one_iteration(gpu, monkeypatch, path):
     assert got[2] == want[2] and got[3] == want[3]
 
 
+@pytest.mark.parametrize("dim", [4, 100, 132])
+def test_lloyd_pools_of_many_empty_clusters(gpu, monkeypatch, dim):
+    """40 centroids that attract nothing, the first and the last among them:
+    more than one batch of pools, each larger than the last up to the limit, at widths of one, 25 and 33 float4."""
+    px = gpu
+    reseed_path(monkeypatch, "pool", 2400)
+    rng = np.random.default_rng(dim)
+    pts = clustered(rng, 10001, dim, 200, 0.4)
+    init = pts[:300].copy()  # every cluster has one
+    init[np.r_[0, 299, rng.choice(np.arange(200, 299), 38, replace=False)]] += np.float32(2000.0)
+    got = px.kmeans_lloyd(pts, init, 3)
+    check_reseed_path(px, "pool", True)
+    assert px.kmeans_last_reseeds()["pool"] >= 40
+    want = orc.kmeans_lloyd(pts, init, 3)
+    assert np.array_equal(bits(got[0]), bits(want[0]))
+    assert np.array_equal(got[1], want[1])
+    assert got[2] == want[2] and got[3] == want[3]
+
+
 @pytest.mark.parametrize("path", RESEED_PATHS)
 @pytest.mark.parametrize("empties", [(7,), (7, 60)])
 def test_farthest_point_ties_take_the_first_index(gpu, monkeypatch, empties, path):
