@@ -304,6 +304,50 @@ __device__ inline void wave_bitonic_sort(uint64_t (&k)[E], int lane) {
   }
 }
 
+// 64-bit shuffle: lane `src`'s value.
+__device__ inline uint64_t shfl64(uint64_t v, int src) {
+  const uint32_t lo = __shfl((uint32_t)v, src, WAVE), hi = __shfl((uint32_t)(v >> 32), src, WAVE);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+// The 64 smallest of two ascending lists of 64 across one wavefront, ascending:
+// lane L holds one list's element L and the other's element 63 - L.
+__device__ inline uint64_t wave_merge64(uint64_t key, uint64_t rev, int lane) {
+  key = rev < key ? rev : key;
+#pragma unroll
+  for (int j = WAVE / 2; j > 0; j >>= 1) {
+    const uint64_t p = shfl_xor64(key, j);
+    const bool take = (lane & j) == 0 ? p < key : key < p;
+    key = take ? p : key;
+  }
+  return key;
+}
+
+// Leaves the 64 smallest keys in keys[0 .. 63], ascending, for n a multiple of
+// 64: each of the first WAVES wavefronts sorts its 64-key parts in registers,
+// the first merges the wavefronts' lists. All threads of the block call it;
+// ends without a barrier, the result is the first wavefront's to read.
+template <int WAVES>
+__device__ inline void block_smallest64(uint64_t* keys, int n) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (w < WAVES) {
+    uint64_t top = KEY_MAX;
+    for (int p = w * WAVE; p < n; p += WAVES * WAVE) {
+      uint64_t x[1] = {keys[p + lane]};
+      wave_bitonic_sort<1>(x, lane);
+      top = p == w * WAVE ? x[0] : wave_merge64(top, shfl64(x[0], 63 - lane), lane);
+    }
+    keys[w * WAVE + lane] = top;  // over the wavefront's own part
+  }
+  __syncthreads();
+  if (w == 0) {
+    uint64_t top = keys[lane];
+#pragma unroll
+    for (int v = 1; v < WAVES; ++v) top = wave_merge64(top, keys[v * WAVE + 63 - lane], lane);
+    keys[lane] = top;
+  }
+}
+
 // Ascending bitonic sort of 64 (key, value) pairs across one wavefront, one
 // pair per lane: afterwards lane L holds the L-th smallest key and its value.
 __device__ inline void wave_sort_kv64(uint64_t& key, uint32_t& val, int lane) {

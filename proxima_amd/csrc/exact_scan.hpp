@@ -139,10 +139,15 @@ __device__ inline void block_bitonic_sort(uint64_t* keys, int n) {
 // queries are staged in LDS and each lane pair loads a row chunk once for the
 // whole group (dist_pair4_multi), so the store streams through L2 once per
 // group instead of once per query (exact_query_group decides when). Each query's keys are sorted on their own,
-// and its kk smallest go to ecand[(f * nchunks + c) * kk], as with QG = 1.
+// and its kk smallest, ascending, go to ecand[(f * nchunks + c) * kk], as with
+// QG = 1. Up to 64 of them come from sorts in registers (a block-wide sort of
+// 256 keys has 36 barriers), and 256-row chunks, which a launch has few of,
+// take 512 threads so that every row's loads are in flight at once: one query
+// over 100k x 128 @S@.
 constexpr int EXACT_QG_MAXD = 1024;
+constexpr int exact_threads(int CH, int QG) { return CH == 256 && QG == 1 ? 512 : 256; }
 template <int CH, int QG = 1>
-[[maybe_unused]] static __global__ __launch_bounds__(256) void flat_exact_candidates(
+[[maybe_unused]] static __global__ __launch_bounds__(exact_threads(CH, QG)) void flat_exact_candidates(
     const int* __restrict__ qlist, const int* __restrict__ qcount, int nchunks, const float* __restrict__ Qp, int ld,
     int dim, int metric, const float* __restrict__ X, int N, const uint8_t* __restrict__ live,
     const uint8_t* __restrict__ accept, const uint32_t* __restrict__ rank, int k, uint64_t* __restrict__ ecand) {
@@ -153,6 +158,7 @@ template <int CH, int QG = 1>
   const int total = ng * nchunks;
   const int g = threadIdx.x & 7, grp = threadIdx.x >> 3;
   const int kk = min(k, CH);
+  constexpr int NT = exact_threads(CH, QG);
   // Chunk-major work order, dealt to the XCDs in contiguous ranges: the
   // query groups of one chunk run on one XCD at about the same time and share
   // its L2 copy of the chunk's rows. Workgroup ids go round-robin over the 8
@@ -185,7 +191,7 @@ template <int CH, int QG = 1>
       // scored from a clamped row (both lanes of a pair take part in its
       // shuffle) and keep KEY_MAX
       const int h = threadIdx.x & 1;
-      for (int s = threadIdx.x >> 1; s < CH; s += 128) {
+      for (int s = threadIdx.x >> 1; s < CH; s += NT / 2) {
         const int slot = base + s;
         const bool u = slot < N && live[slot] && (accept == nullptr || accept[slot]);
         uint64_t key[QG];
@@ -209,7 +215,7 @@ template <int CH, int QG = 1>
       }
     } else {
       // rows narrower than one 8-wide chunk: eight lanes per row
-      for (int s = grp; s < CH; s += 32) {
+      for (int s = grp; s < CH; s += NT / 8) {
         const int slot = base + s;
         uint64_t key = KEY_MAX;
         if (slot < N && live[slot] && (accept == nullptr || accept[slot])) {
@@ -221,8 +227,13 @@ template <int CH, int QG = 1>
     }
     __syncthreads();
     for (int j = 0; j < nv; ++j) {
-      block_bitonic_sort(keys[j], CH);
       uint64_t* out = ecand + ((size_t)(f0 + j) * nchunks + c) * kk;
+      if (kk <= WAVE) {
+        block_smallest64<4>(keys[j], CH);
+        if ((int)threadIdx.x < kk) out[threadIdx.x] = keys[j][threadIdx.x];
+        continue;
+      }
+      block_bitonic_sort(keys[j], CH);
       for (int i = threadIdx.x; i < kk; i += blockDim.x) out[i] = keys[j][i];
     }
     __syncthreads();
@@ -247,6 +258,12 @@ inline int exact_query_group(size_t nq, size_t dim, size_t N) {
 
 constexpr int EXACT_MERGE_MAXK = 1024;
 
+// The k smallest keys of a query's chunk lists (each ascending, padded with
+// KEY_MAX). For k up to 64 the lists' heads are read first: only the at most k
+// lists whose head is among the k smallest heads can hold a result, and those
+// are merged in registers by the four wavefronts; a select over every key
+// took, for 391 lists of 10, 16 us, all of it passes over keys that cannot be
+// results -> @M@.
 template <int CH>
 [[maybe_unused]] static __global__ __launch_bounds__(256) void flat_merge_exact(const int* __restrict__ qlist, const int* __restrict__ qcount,
                                                         const uint64_t* __restrict__ ecand, int nchunks, int k,
@@ -271,6 +288,65 @@ template <int CH>
     n_valid = 0;
   }
   __syncthreads();
+  if (k <= WAVE) {
+    static_assert(CH >= WAVE && EXACT_MERGE_MAXK >= 4 * WAVE, "whole lists, room for four");
+    __shared__ int lists[WAVE];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint64_t top = KEY_MAX;
+    for (int c0 = w * WAVE; c0 < nchunks; c0 += 4 * 256) {
+      uint64_t x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = c0 + u * 256 + lane;
+        x[u] = base[(size_t)min(c, nchunks - 1) * k];
+        x[u] = c < nchunks ? x[u] : KEY_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (!__any(x[u] < shfl64(top, 63))) continue;
+        uint64_t y[1] = {x[u]};
+        wave_bitonic_sort<1>(y, lane);
+        top = wave_merge64(top, shfl64(y[0], 63 - lane), lane);
+      }
+    }
+    sel[w * WAVE + lane] = top;
+    __syncthreads();
+    top = sel[lane];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) top = wave_merge64(top, sel[v * WAVE + 63 - lane], lane);
+    const uint64_t T = shfl64(top, k - 1);  // the k-th smallest head (KEY_MAX: fewer heads)
+    for (int c = threadIdx.x; c < nchunks; c += 256) {
+      const uint64_t x = base[(size_t)c * k];
+      if (x <= T && x != KEY_MAX) lists[atomicAdd(&n_sel, 1)] = c;  // keys differ: at most k
+    }
+    __syncthreads();
+    const int nl = n_sel, back = 63 - lane;
+    top = KEY_MAX;
+    for (int i0 = w; i0 < nl; i0 += 4 * 4) {
+      uint64_t x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        x[u] = i0 + 4 * u < nl && back < k ? base[(size_t)lists[i0 + 4 * u] * k + back] : KEY_MAX;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + 4 * u < nl) top = wave_merge64(top, x[u], lane);
+    }
+    sel[w * WAVE + lane] = top;
+    __syncthreads();
+    if (w != 0) return;
+#pragma unroll
+    for (int v = 1; v < 4; ++v) top = wave_merge64(top, sel[v * WAVE + back], lane);
+    const bool valid = lane < k && top != KEY_MAX;
+    const uint64_t m = __ballot(valid);
+    if (valid && out_keys) {
+      out_keys[(size_t)q * ldo + lane] = top;
+    } else if (valid) {
+      out_ids[(size_t)q * ldo + lane] = ids[rank_slot[(uint32_t)top]];
+      out_d[(size_t)q * ldo + lane] = key_float((uint32_t)(top >> 32));
+    }
+    if (lane == 0) out_count[q] = __popcll(m);
+    return;
+  }
   int local = 0;
   // four keys per thread per step, loaded together before any is used
   for (int i0 = threadIdx.x; i0 < n; i0 += 4 * blockDim.x) {

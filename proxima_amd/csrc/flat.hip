@@ -1176,8 +1176,8 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
       }
 #define PXG_EXACT_SCAN(CHV, QGV)                                                                              \
   hipLaunchKernelGGL((flat_exact_candidates<CHV, QGV>), dim3((std::min((gn + QGV - 1) / QGV * nchunks, 4096) + 7) / 8 * 8), \
-                     dim3(256), 0, s, flag_list + g0, count, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N,       \
-                     d_live.p, d_accept, ranks.rank.p, (int)kq, ecand)
+                     dim3(exact_threads(CHV, QGV)), 0, s, flag_list + g0, count, nchunks, Qp, (int)ld, (int)dim, metric, X.p,    \
+                     (int)N, d_live.p, d_accept, ranks.rank.p, (int)kq, ecand)
 #define PXG_EXACT_MERGE(CHV)                                                                                  \
   hipLaunchKernelGGL(flat_merge_exact<CHV>, dim3((unsigned)gn), dim3(256), 0, s, flag_list + g0, count, ecand, \
                      nchunks, (int)kq, ranks.rank_slot.p, d_ids.p, d_oid, d_od, d_oc, (uint64_t*)nullptr, ldo)

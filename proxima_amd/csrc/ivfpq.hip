@@ -2495,8 +2495,8 @@ struct IvfPqIndex {
       tm.mark(1);
 #define PXG_EXACT_SCAN(CHV, QGV)                                                                                  \
   hipLaunchKernelGGL((flat_exact_candidates<CHV, QGV>),                                                           \
-                     dim3((std::min<int>(((int)nq + QGV - 1) / QGV * nchunks, 4096) + 7) / 8 * 8), dim3(256), 0, s, \
-                     qlist, flag_count, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N, d_live.p, d_accept,  \
+                     dim3((std::min<int>(((int)nq + QGV - 1) / QGV * nchunks, 4096) + 7) / 8 * 8),                \
+                     dim3(exact_threads(CHV, QGV)), 0, s, qlist, flag_count, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N, d_live.p, d_accept,  \
                      ranks.rank.p, (int)kq, ecand)
 #define PXG_EXACT_MERGE(CHV)                                                                                      \
   hipLaunchKernelGGL(flat_merge_exact<CHV>, dim3((unsigned)nq), dim3(256), 0, s, qlist, flag_count, ecand, nchunks, \

@@ -573,3 +573,28 @@ def test_k_far_above_the_live_count(gpu):
         assert_same((gi[:, :100], gd[:, :100], gc), want)
     with pytest.raises(px.Configuration):
         idx.search_batch(q, (1 << 24) + 1)
+
+
+@pytest.mark.parametrize("k", [1, 10, 63, 64, 65])
+@pytest.mark.parametrize("n,dim,nq", [(257, 5, 1), (5001, 24, 1), (20000, 16, 1), (70001, 256, 5), (300, 12, 90)])
+def test_exact_scan_selection(gpu, n, dim, nq, k):
+    """The exact scan's chunk lists and their merge on both sides of 64
+    results: chunks of 256 and 1024 rows, a ragged last chunk, more lists than
+    one pass of the merge's heads, grouped queries, rows at equal distance,
+    and a filter that leaves a chunk without a row and fewer rows than k."""
+    px = gpu
+    rng = np.random.default_rng(n + k)
+    data = rng.standard_normal((n, dim)).astype(np.float32)
+    data[n // 2:n // 2 + 40] = data[0]
+    queries = data[rng.integers(0, n, nq)] + np.float32(0.1) * rng.standard_normal((nq, dim)).astype(np.float32)
+    queries[0] = data[0]
+    ids = rng.permutation(n).astype(np.uint64)
+    accept = np.ones(n, np.uint8)
+    accept[:256] = 0
+    few = np.zeros(n, np.uint8)
+    few[n - 30:] = 1
+    idx = make_index(px, data, 0, ids, mode=2)
+    for a in (None, accept, few):
+        by_id = None if a is None else dict(zip(ids.tolist(), a.tolist()))
+        got = idx.search_batch(queries, k, None if a is None else (lambda i, _m, by_id=by_id: by_id[i] == 1))
+        assert_same(got, oracle_search(px, data, ids, 0, queries, k, accept=a))
