@@ -844,18 +844,22 @@ __global__ __launch_bounds__(NT) void flat_merge(
 // Host side
 // ---------------------------------------------------------------------------
 // Whether the exact scan is expected to finish nq queries over N rows of dim
-// floats sooner than the MFMA candidate path. Both estimates are fitted to
-// timings of the two paths at 20k x 128, 100k x 128, 300k x 256, 1M x 96 and
-// 1M x 768 with 1 to 128 queries (the crossover, 4 to 50 queries over those
-// stores, lands within one measured batch size): the MFMA path costs about
-// 0.1 ms of fixed work plus its GEMM, whole 128-query blocks at about 80% of
-// the FP32 MFMA peak; the exact scan reads the store from HBM once (about
-// 5 TB/s) and streams it through L2 again for every further query (about
-// 0.4 ns per 1000 floats).
-static bool exact_scan_cheaper(size_t N, size_t dim, size_t nq) {
+// floats sooner than the MFMA candidate path (`split`: its split pass). Fitted
+// to both paths at 5k to 1M rows of 32 to 768 floats with 1 to 128 queries,
+// k = 10, device pointers. Either path reads the store from memory once; the
+// candidate path has more launches (48 us; 62 in f32, and whole 128-query
+// blocks at 80% of the FP32 matrix peak), the exact scan streams the store
+// through L2 again for every further query. Measured, candidates / exact, us:
+// 100k x 128 59/51 at 2 queries, 60/67 at 3, 61/121 at 16 (the scan was taken
+// up to 13: 100); 20k x 128 54/47 at 12, 55/63 at 16, 55/74 at 32 (taken up
+// to 52); 300k x 256 97/119 at 1, 99/195 at 6 (taken up to 5); 1M x 768
+// 589/595 at 1, 580/1140 at 4 (taken up to 4); 100k x 32 in f32 69/72 at 12,
+// 70/110 at 32; 20k x 32 70/58 at 48, 72/78 at 96.
+static bool exact_scan_cheaper(size_t N, size_t dim, size_t nq, bool split) {
   const double nd = (double)N * (double)dim;
-  const double t_mfma = 1.0e-4 + (double)((nq + 127) / 128) * nd * 256.0 / 1.25e14;
-  const double t_exact = 5.0e-5 + nd * 4.0 / 5.0e12 + (double)(nq - 1) * nd * 4.0e-13;
+  const double t_mfma = split ? 4.8e-5 + nd * 4.0 / 5.2e12 + (double)nq * (2.0e-7 + nd * 2.4e-15)
+                              : 6.2e-5 + (double)nq * 1.0e-7 + (double)((nq + 127) / 128) * nd * 256.0 / 1.25e14;
+  const double t_exact = 3.5e-5 + nd * 4.0 / 4.2e12 + (double)(nq - 1) * (2.0e-7 + (double)N * 1.0e-11 + nd * 3.5e-13);
   return t_exact < t_mfma;
 }
 
@@ -1002,8 +1006,9 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   // Manhattan has no inner-product form and k beyond FAST_KMAX exceeds the
   // candidate buffers: both take the exact scan, as do stores under 4096
   // rows and batches the exact scan finishes sooner.
+  const bool split_ok = dim >= SPLIT_MIN_DIM && split_norm_ok(maxnorm);
   const bool exact_all = mode == 2 || metric == PXG_MANHATTAN || kq > FAST_KMAX ||
-                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq)));
+                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq, split_ok)));
   const int Kp = (int)std::min<uint64_t>(kq + MARGIN, (uint64_t)FAST_KMAX + MARGIN);
   // a row's buffer holds its Kp keys, one tile's appends (FB_N) and at
   // least 64 more before it must be compacted
@@ -1018,7 +1023,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   const int nKs = (int)((dim + FB_K - 1) / FB_K);
   const size_t split_bytes = nq * nKs * 128 + nq * 4 + (d_accept ? (size_t)tiles * FB_N * 4 : 0) + 4096;
   const size_t exact_bytes = (N / 256 + 1) * std::min<size_t>(kq, EXACT_CH) * 8 + 4096;
-  const bool split = !exact_all && kq > 0 && dim >= SPLIT_MIN_DIM && split_norm_ok(maxnorm) &&
+  const bool split = !exact_all && kq > 0 && split_ok &&
                      sc.room() >= split_bytes + std::max(per_split_bytes, exact_bytes);
   hipLaunchKernelGGL(init_search_flags, dim3(1), dim3(64), 0, s, bad, flag_count);
   _Float16* Qs = nullptr;

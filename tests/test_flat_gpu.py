@@ -432,6 +432,25 @@ def test_default_mode_path_crossover(gpu, n, dim, nqs):
         assert_same(idx.search_batch(q[:nq], 10), oracle_search(px, data, ids, 0, q[:nq], 10, threads=16))
 
 
+@pytest.mark.parametrize("n,dim,nqs", [(100_000, 128, (1, 2, 3, 4)), (300_000, 256, (1, 2)),
+                                       (20_000, 128, (10, 11, 12, 13)), (20_000, 32, (40, 70))])
+def test_default_mode_small_batches(gpu, n, dim, nqs):
+    """Few queries on either side of the default mode's crossover, with a
+    filter and without: the same results from either path."""
+    px = gpu
+    rng = np.random.default_rng(n + dim + 1)
+    data = rng.standard_normal((n, dim)).astype(np.float32)
+    ids = rng.permutation(n).astype(np.uint64)
+    keep = set(ids[rng.random(n) < 0.3].tolist())
+    acc = np.array([i in keep for i in ids.tolist()], np.uint8)
+    idx = make_index(px, data, 0, ids, 0)
+    q = rng.standard_normal((max(nqs), dim)).astype(np.float32)
+    for nq in nqs:
+        assert_same(idx.search_batch(q[:nq], 10), oracle_search(px, data, ids, 0, q[:nq], 10, threads=16))
+    assert_same(idx.search_batch(q[:nq], 70, lambda i, _m: i in keep),
+                oracle_search(px, data, ids, 0, q[:nq], 70, accept=acc, threads=16))
+
+
 def test_search_mode_range(gpu):
     """Search modes are 0 (automatic), 1 (MFMA path) and 2 (exact scan);
     others are refused as a configuration error naming the parameter, and
