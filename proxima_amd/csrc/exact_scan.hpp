@@ -20,10 +20,10 @@ inline int exact_chunk_rows(size_t nq, size_t N) {
 
 // Small fills done by kernels rather than memsets (so that a caller's stream
 // holds only kernel work): the query flag word ~0, the flagged-query count 0.
-[[maybe_unused]] static __global__ void init_search_flags(unsigned long long* bad, int* flag_count) {
+[[maybe_unused]] static __global__ void init_search_flags(unsigned long long* bad, int* flag_count, int count = 0) {
   if (threadIdx.x == 0) {
     *bad = ~0ull;
-    *flag_count = 0;
+    *flag_count = count;
   }
 }
 // init_search_flags that also clears the n 64-bit words at `words` (a
@@ -48,17 +48,27 @@ inline int exact_chunk_rows(size_t nq, size_t N) {
 // 1. query preparation
 // ---------------------------------------------------------------------------
 // One 64-thread workgroup per row: validate, (cosine) normalise, pad to ld.
+// `alone`: the only workgroup, which writes the flag word instead of lowering
+// it (a launch before it to set the word costs a single query 4 us).
 __device__ inline void prep_query_row(const float* __restrict__ raw, int dim, int ld, int metric, int do_prepare,
                                       float* __restrict__ Qp, float* __restrict__ qb, float* __restrict__ qn,
-                                      unsigned long long* __restrict__ bad) {
+                                      unsigned long long* __restrict__ bad, bool alone = false) {
   const int q = blockIdx.x;
   const int lane = threadIdx.x;
   const float* v = raw + (size_t)q * dim;
   float* out = Qp + (size_t)q * ld;
   __shared__ float s_inv;
   // validate: first non-finite component (space.rs:104-121)
-  for (int i = lane; i < dim; i += 64) {
-    if (!isfinite(v[i])) atomicMin(bad, ((unsigned long long)q << 32) | (unsigned)i);
+  if (alone) {
+    int first = 0x7FFFFFFF;
+    for (int i = lane; i < dim; i += 64) first = isfinite(v[i]) ? first : min(first, i);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, WAVE));
+    if (lane == 0) *bad = first == 0x7FFFFFFF ? ~0ull : (unsigned long long)first;
+  } else {
+    for (int i = lane; i < dim; i += 64) {
+      if (!isfinite(v[i])) atomicMin(bad, ((unsigned long long)q << 32) | (unsigned)i);
+    }
   }
   if (lane < 8) {
     float d = dist_group8<2>(v, v, dim, lane);  // = -dot_unrolled(v, v)
@@ -101,14 +111,20 @@ __device__ inline void prep_query_row(const float* __restrict__ raw, int dim, in
 }
 
 // flat_prep_queries for a flat search, which also sets each query's shared
-// candidate threshold to its initial "none" (~0), saving the search a fill
-// launch ahead of its candidate passes.
+// candidate threshold to its initial "none" (~0) and, with `list`, lists every
+// query for the exact scan, saving the search two launches ahead of its
+// passes.
 [[maybe_unused]] static __global__ __launch_bounds__(64) void flat_prep_search_queries(
     const float* __restrict__ raw, int dim, int ld, int metric, int do_prepare, float* __restrict__ Qp,
     float* __restrict__ qb, float* __restrict__ qn, unsigned long long* __restrict__ bad,
-    unsigned long long* __restrict__ gthr) {
-  if (threadIdx.x == 0) gthr[blockIdx.x] = ~0ull;
-  prep_query_row(raw, dim, ld, metric, do_prepare, Qp, qb, qn, bad);
+    unsigned long long* __restrict__ gthr, int* __restrict__ flag_count, int* __restrict__ list) {
+  const bool alone = gridDim.x == 1;
+  if (threadIdx.x == 0) {
+    gthr[blockIdx.x] = ~0ull;
+    if (list) list[blockIdx.x] = (int)blockIdx.x;
+    if (alone) *flag_count = list ? 1 : 0;
+  }
+  prep_query_row(raw, dim, ld, metric, do_prepare, Qp, qb, qn, bad, alone);
 }
 
 // ---------------------------------------------------------------------------
@@ -143,7 +159,8 @@ __device__ inline void block_bitonic_sort(uint64_t* keys, int n) {
 // QG = 1. Up to 64 of them come from sorts in registers (a block-wide sort of
 // 256 keys has 36 barriers), and 256-row chunks, which a launch has few of,
 // take 512 threads so that every row's loads are in flight at once: one query
-// over 100k x 128 @S@.
+// over 100k x 128 21.7 -> 14.7 us (3.5 TB/s; memory latency and the last
+// chunks' sorts bound the rest).
 constexpr int EXACT_QG_MAXD = 1024;
 constexpr int exact_threads(int CH, int QG) { return CH == 256 && QG == 1 ? 512 : 256; }
 template <int CH, int QG = 1>
@@ -263,7 +280,8 @@ constexpr int EXACT_MERGE_MAXK = 1024;
 // lists whose head is among the k smallest heads can hold a result, and those
 // are merged in registers by the four wavefronts; a select over every key
 // took, for 391 lists of 10, 16 us, all of it passes over keys that cannot be
-// results -> @M@.
+// results -> 8.8, two dependent reads
+// and the sorts.
 template <int CH>
 [[maybe_unused]] static __global__ __launch_bounds__(256) void flat_merge_exact(const int* __restrict__ qlist, const int* __restrict__ qcount,
                                                         const uint64_t* __restrict__ ecand, int nchunks, int k,

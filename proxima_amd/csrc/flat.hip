@@ -979,7 +979,7 @@ void check_query_flags(const unsigned long long* words) {
 
 void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, uint64_t k, const uint8_t* d_accept,
                               uint64_t* d_oid, float* d_od, uint32_t* d_oc, Scratch& sc, hipStream_t s,
-                              uint64_t* fallbacks, size_t ldo, bool* deferred) {
+                              uint64_t* fallbacks, size_t ldo, unsigned long long* flags, bool* deferred) {
   if (deferred) *deferred = false;
   check_k(k);
   *fallbacks = 0;
@@ -997,7 +997,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   float* Qp = (float*)sc.get(1, nq * ld * 4);
   float* qb = (float*)sc.get(2, nq * 4);
   float* qn = (float*)sc.get(3, nq * 4);
-  unsigned long long* bad = (unsigned long long*)sc.get(4, 8 + 8);
+  unsigned long long* bad = flags ? flags : (unsigned long long*)sc.get(4, 8 + 8);
   int* flag_count = (int*)(bad + 1);
   int* grp_count = flag_count + 1;
   // per query, the least threshold any split has published (MFMA path),
@@ -1025,7 +1025,10 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   const size_t exact_bytes = (N / 256 + 1) * std::min<size_t>(kq, EXACT_CH) * 8 + 4096;
   const bool split = !exact_all && kq > 0 && split_ok &&
                      sc.room() >= split_bytes + std::max(per_split_bytes, exact_bytes);
-  hipLaunchKernelGGL(init_search_flags, dim3(1), dim3(64), 0, s, bad, flag_count);
+  const bool list_all = exact_all && kq > 0 && kq <= EXACT_MERGE_MAXK;  // the preparation lists every query
+  int* flag_list = list_all ? (int*)sc.get(5, nq * 4) : nullptr;
+  if (nq > 1)  // one query's preparation writes its flags itself
+    hipLaunchKernelGGL(init_search_flags, dim3(1), dim3(64), 0, s, bad, flag_count, list_all ? (int)nq : 0);
   _Float16* Qs = nullptr;
   float* cq = nullptr;
   const float* xbias = xb.p;
@@ -1034,7 +1037,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     Qs = (_Float16*)sc.get(26, nq * nKs * 128);
     cq = (float*)sc.get(27, nq * 4);
     hipLaunchKernelGGL(flat_prep_split_queries, dim3((unsigned)nq), dim3(64), 0, s, d_raw, (int)dim, (int)ld, metric,
-                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr, Qs, nKs, scale, sx, cq);
+                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr, flag_count, Qs, nKs, scale, sx, cq);
     if (d_accept) {
       float* mb = (float*)sc.get(28, (size_t)tiles * FB_N * 4);
       hipLaunchKernelGGL(flat_mask_bias, dim3((unsigned)((tiles * FB_N + 255) / 256)), dim3(256), 0, s, xb.p, d_accept,
@@ -1043,7 +1046,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     }
   } else {
     hipLaunchKernelGGL(flat_prep_search_queries, dim3((unsigned)nq), dim3(64), 0, s, d_raw, (int)dim, (int)ld, metric,
-                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr);
+                       do_prepare ? 1 : 0, Qp, qb, qn, bad, gthr, flag_count, flag_list);
   }
   PXG_HIP(hipGetLastError());
   unsigned long long* tail = sc.host_words();
@@ -1066,8 +1069,8 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
     return;
   }
 
-  int* flag_list = (int*)sc.get(5, nq * 4);
   if (!exact_all) {
+    flag_list = (int*)sc.get(5, nq * 4);
     // queries per workgroup: FB_M, or 32 or 64 for a smaller batch on the
     // split pass
     const int QT = !split || nq > 64 ? 4 : nq > 32 ? 2 : 1;
@@ -1145,10 +1148,6 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
       PXG_MERGE(512, 8192);
 #undef PXG_MERGE
     PXG_HIP(hipGetLastError());
-  } else {
-    hipLaunchKernelGGL(iota_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, flag_list, (int)nq,
-                       flag_count);
-    PXG_HIP(hipGetLastError());
   }
   // exact scan for flagged queries (all of them on the exact path, where the
   // count is known here and the flags are read once, with the results)
@@ -1199,9 +1198,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
       PXG_HIP(hipGetLastError());
     }
     if (exact_all && deferred) {
-      // the caller waits once, for this copy and its own result copies
-      PXG_HIP(hipMemcpyAsync(tail, bad, 16, hipMemcpyDeviceToHost, s));
-      *deferred = true;
+      *deferred = true;  // the caller waits once, for its copy of results and flags
     } else if (exact_all) {
       read_flags(nullptr);  // waits for the results; a non-finite query fails the call
     } else {
@@ -1442,16 +1439,15 @@ int pxg_flat_search(const pxg_flat* index, const float* queries, uint64_t nq, ui
       d_acc = ctx->get(21, N);
       PXG_HIP(hipMemcpyAsync(d_acc, accept, N, hipMemcpyHostToDevice, s));
     }
-    uint64_t* d_oid = (uint64_t*)ctx->get(22, nq * kq * 8);
-    float* d_od = (float*)ctx->get(23, nq * kq * 4);
-    uint32_t* d_oc = (uint32_t*)ctx->get(24, nq * 4);
+    const pxg::ResultBlock out(*ctx.c, nq, kq);
     PXG_HIP(hipMemcpyAsync(d_q, prep.data(), prep.size() * 4, hipMemcpyHostToDevice, s));
     uint64_t fb = 0;
     bool deferred = false;
-    f.search_device(d_q, false, nq, kq, d_acc, d_oid, d_od, d_oc, sc, s, &fb, kq, &deferred);
-    pxg::results_to_host(*ctx.c, s, nq, k, kq, kq, d_oid, d_od, d_oc, out_ids, out_dist, out_count, [&] {
-      if (deferred) pxg::check_query_flags(sc.host_words());
-    });
+    f.search_device(d_q, false, nq, kq, d_acc, out.ids, out.dist, out.count, sc, s, &fb, kq, out.flags, &deferred);
+    pxg::results_to_host(*ctx.c, s, nq, k, kq, kq, out, out_ids, out_dist, out_count,
+                         [&](const unsigned long long* flags) {
+                           if (deferred) pxg::check_query_flags(flags);
+                         });
     pxg::g_last_fallbacks = fb;
   });
 }

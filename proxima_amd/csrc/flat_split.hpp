@@ -19,12 +19,17 @@
 static __global__ __launch_bounds__(64) void flat_prep_split_queries(
     const float* __restrict__ raw, int dim, int ld, int metric, int do_prepare, float* __restrict__ Qp,
     float* __restrict__ qb, float* __restrict__ qn, unsigned long long* __restrict__ bad,
-    unsigned long long* __restrict__ gthr, _Float16* __restrict__ Qs, int nK, float scale, float sx,
+    unsigned long long* __restrict__ gthr, int* __restrict__ flag_count, _Float16* __restrict__ Qs, int nK,
+    float scale, float sx,
     float* __restrict__ cq) {
   const int q = blockIdx.x, lane = threadIdx.x;
   __shared__ float s_sq;
-  if (lane == 0) gthr[q] = ~0ull;
-  prep_query_row(raw, dim, ld, metric, do_prepare, Qp, qb, qn, bad);
+  const bool alone = gridDim.x == 1;
+  if (lane == 0) {
+    gthr[q] = ~0ull;
+    if (alone) *flag_count = 0;
+  }
+  prep_query_row(raw, dim, ld, metric, do_prepare, Qp, qb, qn, bad, alone);
   if (lane == 0) {  // the lane that wrote qn[q]
     const float nv = qn[q];
     const bool ok = nv == 0.0f || split_norm_ok(nv);

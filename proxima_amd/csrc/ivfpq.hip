@@ -3039,12 +3039,12 @@ int pxg_ivfpq_search(const pxg_ivfpq* index, const float* queries, uint64_t nq, 
       d_acc = ctx->get(21, N);
       PXG_HIP(hipMemcpyAsync(d_acc, accept, N, hipMemcpyHostToDevice, s));
     }
-    uint64_t* d_oid = (uint64_t*)ctx->get(22, nq * kq * 8);
-    float* d_od = (float*)ctx->get(23, nq * kq * 4);
-    uint32_t* d_oc = (uint32_t*)ctx->get(24, nq * 4);
+    const pxg::ResultBlock out(*ctx.c, nq, kq);
     PXG_HIP(hipMemcpyAsync(d_q, prep.data(), prep.size() * 4, hipMemcpyHostToDevice, s));
-    f.search_device(d_q, false, nq, kq, nprobe ? nprobe : f.cfg.nprobe, d_acc, d_oid, d_od, d_oc, sc, s, kq);
-    pxg::results_to_host(*ctx.c, s, nq, k, kq, kq, d_oid, d_od, d_oc, out_ids, out_dist, out_count, [] {});
+    f.search_device(d_q, false, nq, kq, nprobe ? nprobe : f.cfg.nprobe, d_acc, out.ids, out.dist, out.count, sc, s,
+                    kq);
+    pxg::results_to_host(*ctx.c, s, nq, k, kq, kq, out, out_ids, out_dist, out_count,
+                         [](const unsigned long long*) {});
   });
 }
 

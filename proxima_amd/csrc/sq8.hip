@@ -1710,9 +1710,7 @@ static int sq8_search_host(const pxg_sq8* index, const float* queries, const int
     // caller's rows of k
     const uint64_t kq = std::min<uint64_t>(k, f.by_id.size());
     const size_t kk = std::max<size_t>(kq, 1);
-    uint64_t* d_oid = (uint64_t*)ctx->get(22, nq * kk * 8);
-    float* d_od = (float*)ctx->get(23, nq * kk * 4);
-    uint32_t* d_oc = (uint32_t*)ctx->get(24, nq * 4);
+    const pxg::ResultBlock out(*ctx.c, nq, kk);
     float* d_q = nullptr;
     int8_t* d_qc = nullptr;
     if (queries) {
@@ -1723,8 +1721,9 @@ static int sq8_search_host(const pxg_sq8* index, const float* queries, const int
       PXG_HIP(hipMemcpyAsync(d_qc, qcodes, nq * f.dim, hipMemcpyHostToDevice, s));
     }
     uint64_t fb = 0;
-    f.search_device(d_q, d_qc, nq, kq, rescore, d_acc, d_oid, d_od, d_oc, sc, s, &fb, kk);
-    pxg::results_to_host(*ctx.c, s, nq, k, kq, kk, d_oid, d_od, d_oc, out_ids, out_dist, out_count, [] {});
+    f.search_device(d_q, d_qc, nq, kq, rescore, d_acc, out.ids, out.dist, out.count, sc, s, &fb, kk);
+    pxg::results_to_host(*ctx.c, s, nq, k, kq, kk, out, out_ids, out_dist, out_count,
+                         [](const unsigned long long*) {});
     pxg::g_sq8_fallbacks = fb;
   });
 }

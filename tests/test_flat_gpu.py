@@ -451,6 +451,33 @@ def test_default_mode_small_batches(gpu, n, dim, nqs):
                 oracle_search(px, data, ids, 0, q[:nq], 70, accept=acc, threads=16))
 
 
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("nq", [1, 2])
+def test_device_flags_of_one_and_two_queries(gpu, nq, mode):
+    """One query's preparation sets its own flag word; two share one set ahead
+    of it. Either names the first non-finite component, and the next search
+    starts clean."""
+    import torch
+    px = gpu
+    rng = np.random.default_rng(nq)
+    data = rng.standard_normal((9000, 130)).astype(np.float32)
+    idx = make_index(px, data, 0, mode=mode)
+    q = rng.standard_normal((nq, 130)).astype(np.float32)
+    oi = torch.zeros((nq, 5), dtype=torch.int64, device="cuda")
+    od = torch.zeros((nq, 5), dtype=torch.float32, device="cuda")
+    oc = torch.zeros(nq, dtype=torch.int32, device="cuda")
+    bad = torch.from_numpy(q).cuda()
+    bad[nq - 1, 129] = float("inf")
+    bad[nq - 1, 71] = float("nan")
+    with pytest.raises(px.NonFinite) as e:
+        idx.search_device(bad, 5, oi, od, oc)
+    assert e.value.index == 71
+    idx.search_device(torch.from_numpy(q).cuda(), 5, oi, od, oc)
+    torch.cuda.synchronize()
+    want = oracle_search(px, data, np.arange(9000, dtype=np.uint64), 0, q, 5)
+    assert_same((oi.cpu().numpy().view(np.uint64), od.cpu().numpy(), oc.cpu().numpy().astype(np.uint32)), want)
+
+
 def test_search_mode_range(gpu):
     """Search modes are 0 (automatic), 1 (MFMA path) and 2 (exact scan);
     others are refused as a configuration error naming the parameter, and
