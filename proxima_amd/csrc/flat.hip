@@ -23,17 +23,13 @@
 //                         come from the f16 matrix cores instead
 //                         (flat_split_candidates, flat_split.hpp), with the
 //                         same tiles, buffers, thresholds and merge.
-//  3. flat_merge_rescore  per query: radix-select the k' best approximate
-//                         keys over all splits, rescore those k' exactly with
-//                         the reference's 8-lane arithmetic, sort by
-//                         (total_cmp(distance), id) and keep k. A query whose
-//                         k-th exact distance is not below the k'-th
-//                         approximate one minus the MFMA error bound is
-//                         flagged. flat_merge_rescore_reg does the same
-//                         when a query's keys fit eight per thread and k'
-//                         one wavefront: its keys are read once into
-//                         registers and one wavefront sorts the rescored
-//                         ones.
+//  3. flat_merge          per query: gathers the listed keys at or below the
+//                         shared threshold, selects the k' best, rescores
+//                         those exactly with the reference's 8-lane
+//                         arithmetic, sorts by (total_cmp(distance), id) and
+//                         keeps k. A query whose k-th exact distance is not
+//                         below the k'-th approximate one minus the
+//                         candidate pass's error bound is flagged.
 //  4. flat_exact_candidates + flat_merge_exact   exact VALU scan for flagged
 //                         queries (and the whole batch for Manhattan, small
 //                         problems, or when forced). Distances are the
