@@ -13,7 +13,8 @@
 // flat_prep_search_queries for the split pass: also each query's parts, as
 // records of 32 hi then 32 lo halves per 32 dimensions (nK records per query,
 // zeros past dim), and the factor cq that takes an accumulated product back
-// to scale * (q . x), scale / (sq sx). A query whose norm the scales cannot
+// to scale * (q . x), scale / sq / sx (down to 2^-148: a power of two, so
+// exact as a subnormal float too). A query whose norm the scales cannot
 // hold gets an infinite norm, so its certificate fails and it is scanned
 // exactly.
 static __global__ __launch_bounds__(64) void flat_prep_split_queries(
@@ -35,7 +36,7 @@ static __global__ __launch_bounds__(64) void flat_prep_split_queries(
     const bool ok = nv == 0.0f || split_norm_ok(nv);
     const float sq = ok ? split_scale(nv) : 0.0f;
     s_sq = sq;
-    cq[q] = ok ? scale / (sq * sx) : 0.0f;
+    cq[q] = ok ? scale / sq / sx : 0.0f;  // sq * sx may exceed f32
     if (!ok) qn[q] = INFINITY;
   }
   __syncthreads();

@@ -48,7 +48,8 @@ __host__ __device__ inline float split_scale(float norm) {
   (void)frexpf(norm, &ex);
   return ldexpf(1.0f, 15 - ex);
 }
-// Norms whose scales, and their product's inverse, stay normal floats.
+// Norms whose scales stay normal floats. Two such scales can multiply past f32
+// (2^75 each), so they are divided by one after the other, never multiplied.
 __host__ __device__ inline bool split_norm_ok(float norm) { return norm >= 0x1p-60f && norm <= 0x1p+60f; }
 
 // One x * s as its two f16 parts (the fma forms are exact: s is a power of

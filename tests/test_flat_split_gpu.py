@@ -70,6 +70,20 @@ def test_norm_range(gpu, metric, rows, queries):
     _check(gpu, _index(gpu, data, metric), data, metric, q, 10)
 
 
+@pytest.mark.parametrize("k", [1, 10])
+@pytest.mark.parametrize("metric,rows,queries", [
+    (0, 1e-16, 1e-16), (0, 3e-17, 1e-16), (2, 1e-16, 1e-16),
+])
+def test_norm_range_inside(gpu, metric, rows, queries, k):
+    """Rows and queries inside 2^-60 .. 2^60 whose factor back from the scaled
+    product is at the end of f32."""
+    rng = np.random.default_rng(18)
+    data, q = _clustered(rng, 6000, 80, 400)
+    data, q = (data * np.float32(rows)).astype(np.float32), (q * np.float32(queries)).astype(np.float32)
+    q[3] = 0.0
+    _check(gpu, _index(gpu, data, metric), data, metric, q, k)
+
+
 @pytest.mark.parametrize("metric", [0, 1, 2])
 def test_mixed_norms_and_ties(gpu, metric):
     """Rows of very different norms under one scale, and repeated rows (ties by id)."""
