@@ -14,9 +14,9 @@
 // records of 32 hi then 32 lo halves per 32 dimensions (nK records per query,
 // zeros past dim), and the factor cq that takes an accumulated product back
 // to scale * (q . x), scale / sq / sx (down to 2^-148: a power of two, so
-// exact as a subnormal float too). A query whose norm the scales cannot
-// hold gets an infinite norm, so its certificate fails and it is scanned
-// exactly.
+// exact as a subnormal float too). qn becomes the norm that the certificate
+// counts with: for a query above the scales' range infinity, so that it is
+// scanned exactly.
 static __global__ __launch_bounds__(64) void flat_prep_split_queries(
     const float* __restrict__ raw, int dim, int ld, int metric, int do_prepare, float* __restrict__ Qp,
     float* __restrict__ qb, float* __restrict__ qn, unsigned long long* __restrict__ bad,
@@ -32,12 +32,16 @@ static __global__ __launch_bounds__(64) void flat_prep_split_queries(
   }
   prep_query_row(raw, dim, ld, metric, do_prepare, Qp, qb, qn, bad, alone);
   if (lane == 0) {  // the lane that wrote qn[q]
-    const float nv = qn[q];
-    const bool ok = nv == 0.0f || split_norm_ok(nv);
+    // A norm below the scales' range stands as its lower end: f32 squares may
+    // have underflowed (up to sqrt(dim) 2^-75 is missing, 0.1% of 2^-60 at
+    // 2^20 dimensions, inside merge_certified's 1%), also in a norm of zero,
+    // so neither the scale nor the certificate may rest on it.
+    const float nv = qn[q] < 0x1p-60f ? 0x1p-60f : qn[q];
+    const bool ok = split_norm_ok(nv);
     const float sq = ok ? split_scale(nv) : 0.0f;
     s_sq = sq;
     cq[q] = ok ? scale / sq / sx : 0.0f;  // sq * sx may exceed f32
-    if (!ok) qn[q] = INFINITY;
+    qn[q] = ok ? nv : INFINITY;
   }
   __syncthreads();
   const float sq = s_sq;

@@ -72,16 +72,29 @@ def test_norm_range(gpu, metric, rows, queries):
 
 @pytest.mark.parametrize("k", [1, 10])
 @pytest.mark.parametrize("metric,rows,queries", [
-    (0, 1e-16, 1e-16), (0, 3e-17, 1e-16), (2, 1e-16, 1e-16),
+    (0, 1e-16, 1e-16), (0, 3e-17, 1e-16), (2, 1e-16, 1e-16), (2, 5e16, 1e-24), (2, 8e16, 4e-24), (2, 8e16, 2e-23),
+    (0, 8e16, 1e-24),
 ])
 def test_norm_range_inside(gpu, metric, rows, queries, k):
-    """Rows and queries inside 2^-60 .. 2^60 whose factor back from the scaled
-    product is at the end of f32."""
+    """Rows inside 2^-60 .. 2^60 with queries whose factor back from the scaled
+    product is at the end of f32 (1e-16 on both sides), or whose squared norm
+    underflows to zero, or nearly, though they are not zero."""
     rng = np.random.default_rng(18)
     data, q = _clustered(rng, 6000, 80, 400)
     data, q = (data * np.float32(rows)).astype(np.float32), (q * np.float32(queries)).astype(np.float32)
     q[3] = 0.0
     _check(gpu, _index(gpu, data, metric), data, metric, q, k)
+
+
+def test_tiny_queries_are_certified(gpu):
+    """Queries far below the scales' range against ordinary rows stay with the
+    candidate pass: what they lose is far inside the Euclidean certificate."""
+    rng = np.random.default_rng(19)
+    data, q = _clustered(rng, 6000, 80, 400)
+    q = (q * np.float32(1e-25)).astype(np.float32)
+    idx = _index(gpu, data, 0)
+    _check(gpu, idx, data, 0, q, 10)
+    assert gpu.FlatIndex.last_fallbacks() == 0
 
 
 @pytest.mark.parametrize("metric", [0, 1, 2])
