@@ -15,7 +15,7 @@
 // zeros past dim), and the factor cq that takes an accumulated product back
 // to scale * (q . x), scale / sq / sx (down to 2^-148: a power of two, so
 // exact as a subnormal float too). qn becomes the norm that the certificate
-// counts with: for a query above the scales' range infinity, so that it is
+// counts with; where the squares overflow it is infinite, and the query is
 // scanned exactly.
 static __global__ __launch_bounds__(64) void flat_prep_split_queries(
     const float* __restrict__ raw, int dim, int ld, int metric, int do_prepare, float* __restrict__ Qp,
@@ -37,7 +37,9 @@ static __global__ __launch_bounds__(64) void flat_prep_split_queries(
     // 2^20 dimensions, inside merge_certified's 1%), also in a norm of zero,
     // so neither the scale nor the certificate may rest on it.
     const float nv = qn[q] < 0x1p-60f ? 0x1p-60f : qn[q];
-    const bool ok = split_norm_ok(nv);
+    // above it the scale and the factor stay normal floats up to the largest
+    // norm there is, 2^64
+    const bool ok = nv <= 0x1p+64f;
     const float sq = ok ? split_scale(nv) : 0.0f;
     s_sq = sq;
     cq[q] = ok ? scale / sq / sx : 0.0f;  // sq * sx may exceed f32

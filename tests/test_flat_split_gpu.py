@@ -86,14 +86,16 @@ def test_norm_range_inside(gpu, metric, rows, queries, k):
     _check(gpu, _index(gpu, data, metric), data, metric, q, k)
 
 
-def test_tiny_queries_are_certified(gpu):
-    """Queries far below the scales' range against ordinary rows stay with the
-    candidate pass: what they lose is far inside the Euclidean certificate."""
+@pytest.mark.parametrize("metric,queries", [(0, 1e-25), (2, 1e18)])
+def test_far_queries_are_certified(gpu, metric, queries):
+    """Queries far below or above 2^-60 .. 2^60 against ordinary rows stay with
+    the candidate pass: for the small ones, what they lose is far inside the
+    Euclidean certificate."""
     rng = np.random.default_rng(19)
     data, q = _clustered(rng, 6000, 80, 400)
-    q = (q * np.float32(1e-25)).astype(np.float32)
-    idx = _index(gpu, data, 0)
-    _check(gpu, idx, data, 0, q, 10)
+    q = (q * np.float32(queries)).astype(np.float32)
+    idx = _index(gpu, data, metric)
+    _check(gpu, idx, data, metric, q, 10)
     assert gpu.FlatIndex.last_fallbacks() == 0
 
 
