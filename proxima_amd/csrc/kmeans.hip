@@ -2137,12 +2137,15 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   const int nb = (int)((n + PP_ROWS - 1) / PP_ROWS);
   DevBuf<float> ns(n);
   DevBuf<double> ps(nb);
-  DevBuf<int> pe(nb), flags(2);
+  // status, rounds in the fixed order, and the picked row: a pick that fails
+  // writes no row, and the rounds queued behind it still read the last one
+  DevBuf<int> pe(nb), flags(3);
+  int* const picked = flags.p + 2;
   DevBuf<ChaCha8> drng(1);
   const size_t first = rng.gen_range_usize(n);
   hipLaunchKernelGGL(copy_row, dim3(1), dim3(256), 0, s, P, ldp, first, dim, cents);
   PXG_HIP(hipMemcpyAsync(drng.p, &rng, sizeof(ChaCha8), hipMemcpyHostToDevice, s));
-  PXG_HIP(hipMemsetAsync(flags.p, 0, 8, s));
+  PXG_HIP(hipMemsetAsync(flags.p, 0, 12, s));
   const int vec4 = (ldp % 4 == 0 && dim % 4 == 0 && ((uintptr_t)P & 15) == 0) ? 1 : 0;
   hipLaunchKernelGGL(km_pp_round, dim3(nb), dim3(256), 0, s, P, ldp, (int)n, dim, cents, ns.p, 1, ps.p, pe.p, vec4);
   PXG_HIP(hipGetLastError());
@@ -2152,7 +2155,7 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   const int kq = (dim + 3) / 4 * 4, words4 = (dim + 31) / 32 * 4;
   DevBuf<int8_t> Q(q8 ? n * kq : 0);
   DevBuf<float> qscale(q8 ? n : 0), qdelta(q8 ? n : 0);
-  DevBuf<int> qnorm(q8 ? n : 0), picked(1);
+  DevBuf<int> qnorm(q8 ? n : 0);
   // four blocks of points per workgroup once that still gives every CU two
   const bool wide = nb >= 4 * 512;
   DevBuf<uint32_t> q4(q8 && wide ? n * words4 : 0), qmeta4(q8 ? n : 0);
@@ -2168,7 +2171,7 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   for (size_t chosen = 1; chosen < k; ++chosen) {
     float* c = cents + chosen * dim;
     hipLaunchKernelGGL(km_pp_pick, dim3(1), dim3(1024), 0, s, P, ldp, (int)n, dim, ns.p, ps.p, pe.p, nb, drng.p, c,
-                       flags.p, flags.p + 1, picked.p);
+                       flags.p, flags.p + 1, picked);
     if (chosen + 1 < k) {
       if (q8) {
         hipLaunchKernelGGL(km_pp_cdist, dim3((unsigned)((chosen + 15) / 16)), dim3(256), 0, s, (const float*)cents,
@@ -2176,7 +2179,7 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
 #define PXG_PP(LPV, SUBV)                                                                                            \
   hipLaunchKernelGGL((km_pp_round_q8<LPV, SUBV>), dim3((nb + SUBV - 1) / SUBV), dim3(256), 0, s, P, ldp, (int)n, dim, \
                      (const int8_t*)Q.p, kq, (const float*)qscale.p, (const float*)qdelta.p, (const int*)qnorm.p,    \
-                     (const uint32_t*)q4.p, (const uint32_t*)qmeta4.p, words4, (const int*)picked.p, ns.p, ps.p,     \
+                     (const uint32_t*)q4.p, (const uint32_t*)qmeta4.p, words4, (const int*)picked, ns.p, ps.p,       \
                      pe.p, gamma, near.p, (const float*)tnear.p, (int)chosen)
         if (!wide) {
           if (dim <= 256) PXG_PP(8, 1); else PXG_PP(16, 1);

@@ -474,3 +474,15 @@ def test_kmeans_pp_four_bit_rounds(gpu, dim, k):
     got = gpu.kmeans_pp(pts, k, 11)
     want = orc.kmeans_pp(pts, k, 11)
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("n,dim,k", [(5000, 40, 6), (5000, 300, 6), (5000, 20, 6)])
+def test_kmeans_pp_sums_that_are_not_finite_are_refused(gpu, n, dim, k):
+    """Coordinates whose squares overflow f32: the first pick fails, and the
+    rounds queued behind it find a row that exists."""
+    pts = (np.random.default_rng(3).standard_normal((n, dim)) * 1e25).astype(np.float32)
+    with pytest.raises(gpu.Internal, match="not finite"):
+        gpu.kmeans_pp(pts, k, 5)
+    # the next call is served
+    ok = (pts * np.float32(1e-25)).astype(np.float32)
+    assert np.array_equal(bits(gpu.kmeans_pp(ok, k, 5)), bits(orc.kmeans_pp(ok, k, 5)))
