@@ -1013,11 +1013,11 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   const float scale = metric == PXG_EUCLIDEAN ? 2.0f : 1.0f;
   const int tiles = (int)((N + FB_N - 1) / FB_N);
   // The split candidate pass: for widths it is at least as accurate on, norms
-  // its scales can hold, and scratch for its operands beside one split of
-  // candidates and the exact scan of one query (a fixed scratch that holds
-  // those only without them takes the f32 pass).
+  // its scales can hold, and scratch for its operands and the flag list beside
+  // one split of candidates and the exact scan of one query (a fixed scratch
+  // that holds those only without the operands takes the f32 pass).
   const int nKs = (int)((dim + FB_K - 1) / FB_K);
-  const size_t split_bytes = nq * nKs * 128 + nq * 4 + (d_accept ? (size_t)tiles * FB_N * 4 : 0) + 4096;
+  const size_t split_bytes = nq * nKs * 128 + nq * 4 * 2 + (d_accept ? (size_t)tiles * FB_N * 4 : 0) + 4096;
   const size_t exact_bytes = (N / 256 + 1) * std::min<size_t>(kq, EXACT_CH) * 8 + 4096;
   const bool split = !exact_all && kq > 0 && split_ok &&
                      sc.room() >= split_bytes + std::max(per_split_bytes, exact_bytes);

@@ -112,3 +112,19 @@ def test_noalloc_capacity_after_queued_stages(gpu):
     q = big[:3000].contiguous()
     _same(_run(px, na, idx, q, 100), _run(px, ref, idx, q, 100))
     _same(_run(px, na, idx, q[:64], 10), _run(px, ref, idx, q[:64], 10))
+
+
+@pytest.mark.parametrize("nq", [43_200, 43_380, 43_500])
+def test_noalloc_split_operands_at_the_limit(gpu, nq):
+    # either side of the batch whose f16 operands, flag list and one
+    # split of candidates (3096 bytes a query) just fill the 128 MiB at 43351
+    # queries: above it the operands are left out and the f32 pass answers
+    import torch
+    px = gpu
+    rng = np.random.default_rng(10)
+    n, dim = 4200, 128
+    idx = px.FlatIndex(px.VectorSpace(dim, 0), n)
+    idx.insert_batch(np.arange(n, dtype=np.uint64), rng.standard_normal((n, dim)).astype(np.float32))
+    idx.set_search_mode(1)
+    q = torch.from_numpy(rng.standard_normal((nq, dim)).astype(np.float32)).cuda()
+    _same(_run(px, _noalloc(px), idx, q, 10), _run(px, px._lib.pxg_flat_search_device, idx, q, 10))
