@@ -615,7 +615,8 @@ constexpr int MERGE_MAXP = 512;  // k' at most, as a power of two
 // and s = q + x:
 //   f32 pass: 4 d s^2 (Euclidean), 4 d q x (else), generous for both the MFMA
 //     sum and the reference's.
-//   split pass: the products' 3.75 d + 6 (split.hpp) times 2 q x or q x; the
+//   split pass: the products' 3.75 D + 8 (split.hpp; D is d rounded up to
+//     whole MFMAs of 16 terms) times 2 q x or q x; the
 //     reference's own sum, d / 8 + 5 of the distance (at most s^2, or q x);
 //     for Euclidean also the two squared norms' d / 8 + 3 each and two
 //     roundings of at most s^2. The norms are themselves within d / 8 + 3,
@@ -629,10 +630,10 @@ __device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric,
   const float d = (float)dim, qx = qnv * maxnorm, s = qnv + maxnorm;
   float eps;
   if (split) {
-    const float d8 = 0.125f * d;
-    eps = metric == 0 ? 1.01f * U * ((7.5f * d + 12.0f) * qx + (d8 + 3.0f) * (qnv * qnv + maxnorm * maxnorm) +
+    const float d8 = 0.125f * d, prod = 3.75f * (float)((dim + 15) & ~15) + 8.0f;
+    eps = metric == 0 ? 1.01f * U * (2.0f * prod * qx + (d8 + 3.0f) * (qnv * qnv + maxnorm * maxnorm) +
                                      (d8 + 7.0f) * s * s)
-                      : 1.01f * U * (3.75f * d + 6.0f + d8 + 6.0f) * qx + 2.4e-7f;
+                      : 1.01f * U * (prod + d8 + 6.0f) * qx + 2.4e-7f;
   } else {
     eps = metric == 0 ? 4.0f * d * U * s * s : 4.0f * d * U * qx + 2.4e-7f;
   }

@@ -229,9 +229,10 @@ static void launch_assign(const float* P, int ldp, const uint32_t* rows, size_t 
 // eps: the fp32 dot product and norms over d terms, the final rounding and
 // the exact sequential (or 8-lane) sum of squares each stay within
 // (2d + 6) * 2^-24 * s^2, s = |p| + max|c|; twice that is used. km_split's
-// products are within (3.75 d + 6) * 2^-24 * |p||c| (split.hpp), twice that
-// in the distance and 4 |p||c| <= s^2; with the exact sum's d + 3, the
-// centroid norm's d / 8 + 3 and the last rounding: 3 d + 11 of the 4 d + 12.
+// products are within (3.75 D + 8) * 2^-24 * |p||c| (split.hpp; D <= d + 15),
+// twice that in the distance and 4 |p||c| <= s^2: 1.875 d + 33; with the exact
+// sum's d + 3, the centroid norm's d / 8 + 3 and the last rounding: 3 d + 40
+// of the 4 d + 12, from 64 dimensions on.
 //
 // Non-finite values: with finite coordinates every partial sum of the
 // approximation is at most (|p| + |c|)^2 in magnitude, which is below s^2 in
