@@ -156,15 +156,19 @@ __device__ inline void block_bitonic_sort(uint64_t* keys, int n) {
 // whole group (dist_pair4_multi), so the store streams through L2 once per
 // group instead of once per query (exact_query_group decides when). Each query's keys are sorted on their own,
 // and its kk smallest, ascending, go to ecand[(f * nchunks + c) * kk], as with
-// QG = 1. Up to 64 of them come from sorts in registers (a block-wide sort of
-// 256 keys has 36 barriers), and 256-row chunks, which a launch has few of,
-// take 512 threads so that every row's loads are in flight at once: one query
-// over 100k x 128 21.7 -> 14.7 us (3.5 TB/s; memory latency and the last
-// chunks' sorts bound the rest).
+// QG = 1. REG, for up to 64 of them: they come from sorts in registers (a
+// block-wide sort of 256 keys has 36 barriers), and 256-row chunks, which a
+// launch has few of, take 512 threads so that every row's loads are in flight
+// at once: one query over 100k x 128 21.7 -> 14.7 us (3.5 TB/s; memory latency
+// and the last chunks' sorts bound the rest). More keys take the block-wide
+// sort, with 256 threads: in one kernel with the sorts in registers, 33 queries
+// of k = 100 over 4500 x 64 took 26.0 us with 512 threads (17.7 with 256), and
+// 257 Manhattan queries of k = 100 over 100k x 128 1393 instead of 1277 (the
+// registers of the other branch).
 constexpr int EXACT_QG_MAXD = 1024;
-constexpr int exact_threads(int CH, int QG) { return CH == 256 && QG == 1 ? 512 : 256; }
-template <int CH, int QG = 1>
-[[maybe_unused]] static __global__ __launch_bounds__(exact_threads(CH, QG)) void flat_exact_candidates(
+constexpr int exact_threads(int CH, int QG, bool REG) { return REG && CH == 256 && QG == 1 ? 512 : 256; }
+template <int CH, int QG, bool REG>
+[[maybe_unused]] static __global__ __launch_bounds__(exact_threads(CH, QG, REG)) void flat_exact_candidates(
     const int* __restrict__ qlist, const int* __restrict__ qcount, int nchunks, const float* __restrict__ Qp, int ld,
     int dim, int metric, const float* __restrict__ X, int N, const uint8_t* __restrict__ live,
     const uint8_t* __restrict__ accept, const uint32_t* __restrict__ rank, int k, uint64_t* __restrict__ ecand) {
@@ -175,7 +179,7 @@ template <int CH, int QG = 1>
   const int total = ng * nchunks;
   const int g = threadIdx.x & 7, grp = threadIdx.x >> 3;
   const int kk = min(k, CH);
-  constexpr int NT = exact_threads(CH, QG);
+  constexpr int NT = exact_threads(CH, QG, REG);
   // Chunk-major work order, dealt to the XCDs in contiguous ranges: the
   // query groups of one chunk run on one XCD at about the same time and share
   // its L2 copy of the chunk's rows. Workgroup ids go round-robin over the 8
@@ -245,13 +249,13 @@ template <int CH, int QG = 1>
     __syncthreads();
     for (int j = 0; j < nv; ++j) {
       uint64_t* out = ecand + ((size_t)(f0 + j) * nchunks + c) * kk;
-      if (kk <= WAVE) {
+      if constexpr (REG) {
         block_smallest64<4>(keys[j], CH);
         if ((int)threadIdx.x < kk) out[threadIdx.x] = keys[j][threadIdx.x];
-        continue;
+      } else {
+        block_bitonic_sort(keys[j], CH);
+        for (int i = threadIdx.x; i < kk; i += blockDim.x) out[i] = keys[j][i];
       }
-      block_bitonic_sort(keys[j], CH);
-      for (int i = threadIdx.x; i < kk; i += blockDim.x) out[i] = keys[j][i];
     }
     __syncthreads();
   }
@@ -271,6 +275,35 @@ template <int CH, int QG = 1>
 inline int exact_query_group(size_t nq, size_t dim, size_t N) {
   const size_t items = (nq + 3) / 4 * ((N + EXACT_CH - 1) / EXACT_CH);
   return (nq >= 4 && dim >= 256 && dim <= EXACT_QG_MAXD && items >= 512) ? 4 : 1;
+}
+
+// The scan of `count` listed queries (at most gn) in chunks of CH rows, QG
+// queries to a group (four only in EXACT_CH-row chunks: their 512 items are
+// more than exact_chunk_rows splits further); k as flat_exact_candidates.
+[[maybe_unused]] static void launch_exact_candidates(int CH, int QG, const int* qlist, const int* count, int gn,
+                                                     int nchunks, const float* Qp, int ld, int dim, int metric,
+                                                     const float* X, int N, const uint8_t* live,
+                                                     const uint8_t* accept, const uint32_t* rank, int k,
+                                                     uint64_t* ecand, hipStream_t s) {
+  const dim3 grid((std::min((gn + QG - 1) / QG * nchunks, 4096) + 7) / 8 * 8);
+#define PXG_EXACT_SCAN(CHV, QGV, REGV)                                                                               \
+  hipLaunchKernelGGL((flat_exact_candidates<CHV, QGV, REGV>), grid, dim3(exact_threads(CHV, QGV, REGV)), 0, s, qlist, \
+                     count, nchunks, Qp, ld, dim, metric, X, N, live, accept, rank, k, ecand)
+#define PXG_EXACT_SCAN_K(CHV, QGV) \
+  if (k <= WAVE)                   \
+    PXG_EXACT_SCAN(CHV, QGV, true); \
+  else                             \
+    PXG_EXACT_SCAN(CHV, QGV, false)
+  if (QG == 4) {
+    PXG_EXACT_SCAN_K(EXACT_CH, 4);
+  } else if (CH == 256) {
+    PXG_EXACT_SCAN_K(256, 1);
+  } else {
+    PXG_EXACT_SCAN_K(EXACT_CH, 1);
+  }
+#undef PXG_EXACT_SCAN_K
+#undef PXG_EXACT_SCAN
+  PXG_HIP(hipGetLastError());
 }
 
 constexpr int EXACT_MERGE_MAXK = 1024;

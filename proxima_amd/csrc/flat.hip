@@ -1175,22 +1175,13 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
         hipLaunchKernelGGL(set_int, dim3(1), dim3(64), 0, s, grp_count, gn);
         count = grp_count;
       }
-#define PXG_EXACT_SCAN(CHV, QGV)                                                                              \
-  hipLaunchKernelGGL((flat_exact_candidates<CHV, QGV>), dim3((std::min((gn + QGV - 1) / QGV * nchunks, 4096) + 7) / 8 * 8), \
-                     dim3(exact_threads(CHV, QGV)), 0, s, flag_list + g0, count, nchunks, Qp, (int)ld, (int)dim, metric, X.p,    \
-                     (int)N, d_live.p, d_accept, ranks.rank.p, (int)kq, ecand)
 #define PXG_EXACT_MERGE(CHV)                                                                                  \
   hipLaunchKernelGGL(flat_merge_exact<CHV>, dim3((unsigned)gn), dim3(256), 0, s, flag_list + g0, count, ecand, \
                      nchunks, (int)kq, ranks.rank_slot.p, d_ids.p, d_oid, d_od, d_oc, (uint64_t*)nullptr, ldo)
-      if (CH == 256) {
-        if (QG == 4) PXG_EXACT_SCAN(256, 4); else PXG_EXACT_SCAN(256, 1);
-      } else {
-        if (QG == 4) PXG_EXACT_SCAN(EXACT_CH, 4); else PXG_EXACT_SCAN(EXACT_CH, 1);
-      }
-      PXG_HIP(hipGetLastError());
+      launch_exact_candidates(CH, QG, flag_list + g0, count, gn, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N,
+                              d_live.p, d_accept, ranks.rank.p, (int)kq, ecand, s);
       if (exact_all && g0 == 0) tm.mark(2);
       if (CH == 256) PXG_EXACT_MERGE(256); else PXG_EXACT_MERGE(EXACT_CH);
-#undef PXG_EXACT_SCAN
 #undef PXG_EXACT_MERGE
       PXG_HIP(hipGetLastError());
     }

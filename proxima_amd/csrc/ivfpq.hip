@@ -2493,23 +2493,13 @@ struct IvfPqIndex {
       const int kk = (int)std::min<uint64_t>(kq, (uint64_t)CH);
       uint64_t* ecand = (uint64_t*)sc.get(7, (size_t)nq * nchunks * kk * 8);
       tm.mark(1);
-#define PXG_EXACT_SCAN(CHV, QGV)                                                                                  \
-  hipLaunchKernelGGL((flat_exact_candidates<CHV, QGV>),                                                           \
-                     dim3((std::min<int>(((int)nq + QGV - 1) / QGV * nchunks, 4096) + 7) / 8 * 8),                \
-                     dim3(exact_threads(CHV, QGV)), 0, s, qlist, flag_count, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N, d_live.p, d_accept,  \
-                     ranks.rank.p, (int)kq, ecand)
 #define PXG_EXACT_MERGE(CHV)                                                                                      \
   hipLaunchKernelGGL(flat_merge_exact<CHV>, dim3((unsigned)nq), dim3(256), 0, s, qlist, flag_count, ecand, nchunks, \
                      (int)kq, ranks.rank_slot.p, d_ids.p, d_oid, d_od, d_oc, (uint64_t*)nullptr, ldo)
-      if (CH == 256) {
-        if (QG == 4) PXG_EXACT_SCAN(256, 4); else PXG_EXACT_SCAN(256, 1);
-      } else {
-        if (QG == 4) PXG_EXACT_SCAN(EXACT_CH, 4); else PXG_EXACT_SCAN(EXACT_CH, 1);
-      }
-      PXG_HIP(hipGetLastError());
+      launch_exact_candidates(CH, QG, qlist, flag_count, (int)nq, nchunks, Qp, (int)ld, (int)dim, metric, X.p, (int)N,
+                              d_live.p, d_accept, ranks.rank.p, (int)kq, ecand, s);
       tm.mark(2);
       if (CH == 256) PXG_EXACT_MERGE(256); else PXG_EXACT_MERGE(EXACT_CH);
-#undef PXG_EXACT_SCAN
 #undef PXG_EXACT_MERGE
       PXG_HIP(hipGetLastError());
     } else {
