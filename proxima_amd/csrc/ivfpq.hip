@@ -123,22 +123,131 @@ __device__ inline void wave_compact(uint64_t* wb, int cnt, int kk, int lane) {
   }
 }
 
+// One distance table (product.rs:416-433), by all 256 threads. L2: on the
+// residual q - c (ivfpq.rs:1052-1054); cosine: on the query itself. Out of
+// line, so that its loads in flight do not shape the scan's registers (with
+// LDS pointers as such: a function's plain ones are flat accesses).
+typedef __attribute__((address_space(3))) float lds_float;
+typedef float f4v __attribute__((ext_vector_type(4)));
+template <int METRIC>
+__device__ __attribute__((noinline)) void ivf_table(lds_float* lut, lds_float* sres, const float* qv, const float* cv,
+                                                    int dim, int M, int w_eq, int staged, const float* books,
+                                                    const int* sub_off, const int* book_off) {
+  auto add = [](float& acc, float r, float x) {
+    if constexpr (METRIC == 0) {
+      const float d = r - x;
+      acc += d * d;
+    } else {
+      acc += r * x;
+    }
+  };
+  auto at = [&](int i) { return METRIC == 0 ? qv[i] - cv[i] : qv[i]; };
+  // equal widths: entry e is codebook row e against the dimensions from
+  // (e / 256) w_eq on; 1 and 2 wide, several entries' loads are in flight
+  auto one = [&](auto value) {
+#pragma unroll 4
+    for (int e = threadIdx.x; e < M * 256; e += 256) {
+      float acc = 0.0f;
+      add(acc, value(e >> 8), books[e]);
+      lut[e] = acc;
+    }
+  };
+  auto two = [&](auto value) {
+#pragma unroll 4
+    for (int e = threadIdx.x; e < M * 256; e += 256) {
+      const float2 x = *reinterpret_cast<const float2*>(books + 2 * e);
+      float acc = 0.0f;
+      add(acc, value((e >> 8) * 2), x.x);
+      add(acc, value((e >> 8) * 2 + 1), x.y);
+      lut[e] = acc;
+    }
+  };
+  // any widths
+  auto rows = [&](auto value) {
+    for (int e = threadIdx.x; e < M * 256; e += 256) {
+      const int s = e >> 8, c = e & 255;
+      const int w_s = sub_off[s + 1] - sub_off[s];
+      const float* b = books + book_off[s] + c * w_s;
+      const int o = sub_off[s];
+      float acc = 0.0f;
+      for (int j = 0; j < w_s; ++j) add(acc, value(o + j), b[j]);
+      lut[e] = acc;
+    }
+  };
+  if (staged) {
+    for (int j = threadIdx.x; j < dim; j += 256) sres[j] = at(j);
+    __syncthreads();
+    auto row = [&](int i) { return sres[i]; };
+    if (w_eq == 1) {
+      one(row);
+    } else if (w_eq == 2) {
+      two(row);
+    } else if (w_eq == 0) {
+      rows(row);
+    } else {
+      for (int e = threadIdx.x; e < M * 256; e += 256) {
+        const float* b = books + (size_t)e * w_eq;
+        const lds_float* r = sres + (e >> 8) * w_eq;
+        float acc = 0.0f;
+        if ((w_eq & 3) == 0) {
+          for (int j = 0; j < w_eq; j += 4) {
+            const float4 x = *reinterpret_cast<const float4*>(b + j);
+            const f4v y = *(const __attribute__((address_space(3))) f4v*)(r + j);
+            add(acc, y.x, x.x);
+            add(acc, y.y, x.y);
+            add(acc, y.z, x.z);
+            add(acc, y.w, x.w);
+          }
+        } else {
+          for (int j = 0; j < w_eq; ++j) add(acc, r[j], b[j]);
+        }
+        lut[e] = acc;
+      }
+    }
+  } else if (w_eq == 1) {
+    one(at);
+  } else if (w_eq == 2) {
+    two(at);
+  } else if (w_eq > 0 && (w_eq & 3) == 0) {
+    for (int e = threadIdx.x; e < M * 256; e += 256) {
+      const float* b = books + (size_t)e * w_eq;
+      const int o = (e >> 8) * w_eq;
+      float acc = 0.0f;
+      for (int j = 0; j < w_eq; j += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(b + j);
+        add(acc, at(o + j), x.x);
+        add(acc, at(o + j + 1), x.y);
+        add(acc, at(o + j + 2), x.z);
+        add(acc, at(o + j + 3), x.w);
+      }
+      lut[e] = acc;
+    }
+  } else {
+    rows(at);
+  }
+}
+
 // General form (any subspace layout, shortlists up to IVF_MAX_SHORT): one
 // workgroup per (query, group of pg probes), the table in LDS, the waves'
 // candidate lists kept across the group's probes. The cosine table is the
 // query's own and is built once per workgroup; the L2 table is rebuilt per
 // probe (the residual's rounding is part of the result).
-// What bounds it: building tables for lists of a few hundred entries. The
-// query (or residual) is staged in LDS (when it fits beside the table) and
-// codebook rows whose widths are multiples of four come as float4 loads, two
-// instead of eight per entry at 8-wide subspaces; an entry's slot and rank are
-// fetched only if its distance can enter the list. 100 cosine queries, 12 x 8
-// dimensions, 16 probes of about 490 entries, shortlist 100: 120 us with a
-// workgroup and a table per probe -> 49 us.
+// What bounds it: building tables for lists of a few hundred entries. With
+// `staged` the query or residual is in LDS; codebook rows of multiples of four
+// come as float4 loads, two instead of eight per entry at 8-wide subspaces,
+// and 1- and 2-wide ones with four entries' loads in flight. An entry's slot
+// and rank are fetched only if its distance can enter the list. 100 cosine
+// queries, 12 x 8 dimensions, 16 probes of about 490 entries, shortlist 100:
+// 120 us with a workgroup and a table per probe -> 49 us. 128 two-wide
+// subspaces, lists of 625, 8 probes: one L2 query 155 -> 65 us, 100 cosine
+// ones 331 -> 146 us (one width loop for all, read through the offsets, and a
+// code word at a time -> these); 300 L2 queries of 64 one-wide subspaces, 8
+// probes, shortlist 300: 566 us with the residual staged and one workgroup per
+// CU left, 288 before it was staged.
 template <int CAPW, int METRIC>
 __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, int ld, int dim, int M,
                                                 const int* __restrict__ probes, int nprobe, int pg, int groups,
-                                                int staged, const float* __restrict__ cents,
+                                                int w_eq, int staged, const float* __restrict__ cents,
                                                 const float* __restrict__ books, const int* __restrict__ sub_off,
                                                 const int* __restrict__ book_off,
                                                 const uint32_t* __restrict__ list_beg,
@@ -158,41 +267,8 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   float* const sres = lut + M * 256;
 
-  // Distance table (product.rs:416-433). L2: on the residual q - c
-  // (ivfpq.rs:1052-1054); cosine: on the query itself.
   auto build = [&](const float* cv) {
-    if (staged) {
-      for (int j = tid; j < dim; j += 256) sres[j] = METRIC == 0 ? qv[j] - cv[j] : qv[j];
-      __syncthreads();
-    }
-    for (int e = tid; e < M * 256; e += 256) {
-      const int s = e >> 8, c = e & 255;
-      const int o = sub_off[s], w_s = sub_off[s + 1] - o, bo = book_off[s];
-      const float* b = books + bo + c * w_s;
-      float acc = 0.0f;
-      auto add = [&](float r, float x) {
-        if constexpr (METRIC == 0) {
-          const float d = r - x;
-          acc += d * d;
-        } else {
-          acc += r * x;
-        }
-      };
-      if (staged && ((w_s | bo | o) & 3) == 0) {
-        for (int j = 0; j < w_s; j += 4) {
-          const float4 x = *reinterpret_cast<const float4*>(b + j);
-          const float4 r = *reinterpret_cast<const float4*>(sres + o + j);
-          add(r.x, x.x);
-          add(r.y, x.y);
-          add(r.z, x.z);
-          add(r.w, x.w);
-        }
-      } else {
-        for (int j = 0; j < w_s; ++j)
-          add(staged ? sres[o + j] : (METRIC == 0 ? qv[o + j] - cv[o + j] : qv[o + j]), b[j]);
-      }
-      lut[e] = acc;
-    }
+    ivf_table<METRIC>((lds_float*)lut, (lds_float*)sres, qv, cv, dim, M, w_eq, staged, books, sub_off, book_off);
   };
   if constexpr (METRIC == 1) {
     // q . c of every probe for the cosine decomposition (ivfpq.rs:1068-1072,
@@ -228,6 +304,7 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
 #pragma unroll
           for (int s = 0; s < 16; ++s) sum += lut[s * 256 + ((wv[s >> 2] >> (8 * (s & 3))) & 255)];
         } else if ((M & 3) == 0) {
+#pragma unroll 4
           for (int s = 0; s < M; s += 4) {
             const uint32_t cw = *reinterpret_cast<const uint32_t*>(code + s);
             sum += lut[s * 256 + (cw & 255)];
@@ -2666,20 +2743,26 @@ struct IvfPqIndex {
                                            s, ldo);
         scanned_dev = nullptr;
       } else {
-      // probes per workgroup as on the register path; the query (or residual)
-      // is staged beside the table where the LDS holds both
+      // probes per workgroup as on the register path
       int pg = IVF_PGMAX;
       while (pg > 1 && (int64_t)nq * ((np + pg - 1) / pg) < 512) pg >>= 1;
       const int groups = (np + pg - 1) / pg;
       const size_t table = (size_t)M() * 256 * 4;
-      const int staged = scan_lds + dim * 4 + 64 <= IVF_LDS ? 1 : 0;
+      // the query (or residual) is staged beside the table where that takes at
+      // most one workgroup in four off a CU (64 one-wide subspaces and a
+      // shortlist of 300: the second of two, and the scan twice as long; 12
+      // eight-wide ones: the eighth of eight, and 115 -> 73 us a search)
+      const int w_eq = dim % M() == 0 ? W : 0;
+      const size_t with_row = scan_lds + dim * 4 + 64;
+      const int staged = with_row <= IVF_LDS &&
+                         4 * std::min<size_t>(IVF_LDS / with_row, 8) >= 3 * std::min<size_t>(IVF_LDS / scan_lds, 8);
       const size_t lds = table + (staged ? (size_t)dim * 4 : 0);
       uint64_t* cand = (uint64_t*)sc.get(10, (size_t)nq * groups * 4 * kk * 8);
       const int grid = (int)(nq * groups);
       tm.mark(1);
 #define PXG_SCAN(CAPW, MET)                                                                                       \
   hipLaunchKernelGGL((ivf_scan<CAPW, MET>), dim3(grid), dim3(256), lds, s, Qp, (int)ld, (int)dim, (int)M(), probes, \
-                     np, pg, groups, staged, cents.p, books.p, d_sub_off.p, d_book_off.p, list_beg.p, list_end.p,  \
+                     np, pg, groups, w_eq, staged, cents.p, books.p, d_sub_off.p, d_book_off.p, list_beg.p, list_end.p,  \
                      list_slot.p, list_codes.p, ranks.rank_slot.p, ranks.rank.p, d_accept, kk, cand)
       if (kk <= 192) {
         if (metric == PXG_COSINE) PXG_SCAN(256, 1); else PXG_SCAN(256, 0);

@@ -661,3 +661,25 @@ def test_general_scan_probe_groups(gpu, metric, dim, m, k, rerank, nq):
         assert_same(idx.search_batch(q, k, nprobe=nprobe), want)
     want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), qp, k, 5, m, accept=accept, **kw)
     assert_same(idx.search_batch(q, k, lambda i, _m: bool(accept[i]), nprobe=5), want)
+
+
+@pytest.mark.parametrize("metric", [0, 1])
+@pytest.mark.parametrize("dim,m,shortlist", [
+    (24, 24, 100), (24, 12, 100), (48, 12, 100), (33, 11, 100), (37, 12, 100),  # the query staged beside the table
+    (64, 64, 200), (128, 64, 200), (256, 64, 200),  # staging would take the CU's second workgroup
+])
+def test_general_scan_tables(gpu, metric, dim, m, shortlist):
+    """Every form of the general scan's table build: one, two and four wide,
+    other equal widths and unequal ones, with the query staged and without."""
+    px = gpu
+    n, nlist = 1500, 6
+    data = corpus(n, dim, 12) + np.random.default_rng(dim + m).standard_normal((n, dim)).astype(np.float32) * 0.2
+    prep = orc.prepare_rows(metric, data)
+    cents, books, _ = orc.ivf_train(prep, nlist, m, max_iter=1, seed=1)
+    codes, list_of = orc.ivf_encode(prep, cents, books, m)
+    idx = build(px, data, px.IvfPqConfig(nlist, m).with_train_threshold(1 << 62), metric)
+    idx.load_trained(cents, books, codes, list_of)
+    q = data[::150] + np.float32(0.01)
+    want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), orc.prepare_rows(metric, q), shortlist, 3,
+                          m, threads=8)
+    assert_same(idx.search_batch(q, shortlist, nprobe=3), want)
