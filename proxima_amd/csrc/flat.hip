@@ -647,14 +647,17 @@ __device__ inline bool merge_certified(uint64_t pivot, uint64_t kth, int metric,
 // At least k' keys of the lists are at or below the query's shared threshold
 // (its seed, or the k'-th key some split published), so only those can be
 // among the k' smallest: they are gathered into LDS (16 threads per list, the
-// first 16 entries of four lists loaded together) and selected there. More
-// than LM of them are selected from memory instead.
+// first 16 entries of four lists loaded together) and selected there. Where
+// there are more than LM, the k'-th of the LM that were taken is a tighter
+// threshold, and the lists are gathered again.
 // What bounds it: round trips to memory (the lists, then rows, ranks and ids
 // together) and the select's barriers. 313 queries of 170 lists and k' = 116
 // (about 1600 gathered keys): 225 us when every list was padded to k' keys
 // and all 19,720 were selected over, 36 us here; 48 queries of 195 lists, k'
-// = 26: 16.2 -> 11.4 us; 1000 queries of 61 lists: 14.6 -> 16.6 us, for 7 us
-// less in the candidate pass, which no longer sorts and pads its lists.
+// = 26: 16.2 -> 11.4 us. With lst at 4096 or 8192 keys and a select from
+// memory beyond, 3000 queries of k = 64 over 20k x 32 took 135 us (83 over
+// padded lists), 53 now; 1024 of k = 100 over 1M x 128 (14,000 keys) 234 ->
+// 118 us.
 template <int NT, int LM>
 __global__ __launch_bounds__(NT) void flat_merge(
     const uint64_t* __restrict__ cand, int S, int CAP, int Kp, int k, const unsigned long long* __restrict__ gthr,
@@ -674,7 +677,7 @@ __global__ __launch_bounds__(NT) void flat_merge(
   __shared__ int n_list, n_valid, n_sel;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & (WAVE - 1);
   const uint64_t* base = cand + (size_t)q * S * CAP;
-  const uint64_t g = gthr[q];
+  uint64_t g = gthr[q];
   const int gl = tid & 15, grp = tid >> 4;
   // the counts and first 15 keys of the first 4 NG lists, in flight together
   uint64_t x[4];
@@ -692,6 +695,19 @@ __global__ __launch_bounds__(NT) void flat_merge(
     if (lane == leader) at = atomicAdd(&n_list, __popcll(m));
     at = __builtin_amdgcn_readlane(at, leader) + __popcll(m & ((1ull << lane) - 1));
     if (((m >> lane) & 1) != 0 && at < LM) lst[at] = x;
+  };
+  // the keys from `from` on of the group's four lists s0 + u NG + grp, c[u] long
+  auto gather = [&](int s0, int from, const int (&c)[4], int most) {
+    for (int j0 = from; __ballot(j0 < most) != 0; j0 += 16) {
+      uint64_t y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = min(s0 + u * NG + grp, S - 1);
+        y[u] = j0 + gl < c[u] ? base[(size_t)s * CAP + 1 + j0 + gl] : KEY_MAX;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) push(y[u]);
+    }
   };
   int mine = 0;  // keys of this group's lists
   for (int s0 = 0; s0 < S; s0 += 4 * NG) {  // uniform, so that every lane takes part in push
@@ -711,15 +727,7 @@ __global__ __launch_bounds__(NT) void flat_merge(
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) push(gl > 0 && gl <= c[u] ? x[u] : KEY_MAX);
-    for (int j0 = 15; __ballot(j0 < most) != 0; j0 += 16) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = min(s0 + u * NG + grp, S - 1);
-        x[u] = j0 + gl < c[u] ? base[(size_t)s * CAP + 1 + j0 + gl] : KEY_MAX;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) push(x[u]);
-    }
+    gather(s0, 15, c, most);
   }
   if (gl == 0 && mine) atomicAdd(&n_valid, mine);
   __syncthreads();
@@ -729,13 +737,44 @@ __global__ __launch_bounds__(NT) void flat_merge(
     if (tid == 0) out_count[q] = 0;
     return;
   }
-  const int n = n_list;
+  // More keys than lst holds: the ksel-th smallest of those it took bounds the
+  // query's, so the lists are gathered again up to it (strictly fewer keys
+  // each time, about ksel / LM of them).
+  int n = n_list;
+  while (n > LM) {
+    uint64_t v[PER], lo = KEY_MAX, hi = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      v[j] = lst[tid + j * NT];
+      lo = min(lo, v[j]);
+      hi = max(hi, v[j]);
+    }
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) f(v[j]);
+    };
+    g = block_radix_select_range<NT>(each, lo, hi, ksel, hist, sh);
+    if (tid == 0) n_list = 0;
+    __syncthreads();
+    for (int s0 = 0; s0 < S; s0 += 4 * NG) {
+      int c[4], most = 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = s0 + u * NG + grp;
+        c[u] = s < S ? (int)scnt[s] : 0;
+        most = max(most, c[u]);
+      }
+      gather(s0, 0, c, most);
+    }
+    __syncthreads();
+    n = n_list;
+  }
   uint64_t pivot;
-  if (n <= 2 * NT && gridDim.x <= 256) {
+  if (n <= 512 && n <= 2 * NT && gridDim.x <= 256) {
     // few keys, and one query per CU: each thread counts the keys below its
-    // own two (a chain of LDS reads instead of the select's barriers; with
-    // several queries per CU those reads are what they wait for: 1000 queries
-    // 18.6 -> 27.5 us)
+    // own one or two (a chain of LDS reads instead of the select's barriers;
+    // with several queries per CU those reads are what they wait for: 1000
+    // queries 18.6 -> 27.5 us, and 800 keys take 12 us longer than the select)
     const uint64_t a = tid < n ? lst[tid] : KEY_MAX, b = tid + NT < n ? lst[tid + NT] : KEY_MAX;
     int ra = 0, rb = 0;
     if (n <= NT) {
@@ -753,7 +792,7 @@ __global__ __launch_bounds__(NT) void flat_merge(
     if (b != KEY_MAX && rb < ksel) sel[rb] = b;
     __syncthreads();
     pivot = sel[ksel - 1];
-  } else if (n <= LM) {
+  } else {
     // the digits start at the highest bit in which the keys differ
     uint64_t v[PER], lo = KEY_MAX, hi = 0;
 #pragma unroll
@@ -770,18 +809,6 @@ __global__ __launch_bounds__(NT) void flat_merge(
         if (v[j] != KEY_MAX) f(v[j]);
     };
     pivot = block_radix_select_range<NT>(each, lo, hi, ksel, hist, sh);
-    each([&](uint64_t x) {
-      if (x <= pivot) sel[atomicAdd(&n_sel, 1) & (MERGE_MAXP - 1)] = x;
-    });
-  } else {
-    auto each = [&](auto f) {
-      for (int s = grp; s < S; s += NG)
-        for (int j = gl; j < (int)scnt[s]; j += 16) {
-          const uint64_t x = base[(size_t)s * CAP + 1 + j];
-          if (x <= g) f(x);
-        }
-    };
-    pivot = block_radix_select_each<64>(each, ksel, hist, sh);
     each([&](uint64_t x) {
       if (x <= pivot) sel[atomicAdd(&n_sel, 1) & (MERGE_MAXP - 1)] = x;
     });
@@ -1137,12 +1164,24 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
                      (int)kq, (const unsigned long long*)gthr, Qp, (int)ld, (int)dim, metric, X.p, ranks.rank.p,     \
                      ranks.rank_slot.p, d_ids.p, qn, q_add, maxnorm, d_oid, d_od, d_oc, flag_list, flag_count, \
                      ldo)
-    // the lists hold S * Kp keys at or below a query's threshold at most, far
-    // fewer where the seed is tight; the small form fits four blocks per CU
-    if ((size_t)S * Kp <= 8192 && Kp <= WAVE)
-      PXG_MERGE(256, 4096);
+    // A query has about Kp times a split's tiles keys at or below its seed
+    // (S * (CAP - 1) at most); lst holds a few times Kp, and more keys cost a
+    // second gather. Up to 768 queries, three to a CU, the time is one query's
+    // chain, shortest with 512 threads; beyond, it is how many queries a CU
+    // holds. Medians of 36 shapes from 4500 x 64 to 1M x 128, 512 / 256 / 128
+    // threads: 130 queries of k = 100 33 / 38 / 46 us; 1024 of k = 10 31 / 26
+    // / 30, of k = 256 90 / 71 / 123 (256 x 2048); 3000 of k = 10 73 / 54 / 37,
+    // of k = 100 141 / 100 / 86.
+    if (nq >= 2000 && Kp <= 128)
+      PXG_MERGE(128, 512);
+    else if (nq > 768 && Kp <= 128)
+      PXG_MERGE(256, 1024);
+    else if (nq > 768)
+      PXG_MERGE(256, 2048);
+    else if (nq <= 512 && Kp > WAVE)  // two to a CU hold the longer list
+      PXG_MERGE(512, 4096);
     else
-      PXG_MERGE(512, 8192);
+      PXG_MERGE(512, 2048);
 #undef PXG_MERGE
     PXG_HIP(hipGetLastError());
   }
