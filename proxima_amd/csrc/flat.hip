@@ -867,24 +867,56 @@ __global__ __launch_bounds__(NT) void flat_merge(
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
-// Whether the exact scan is expected to finish nq queries over N rows of dim
-// floats sooner than the MFMA candidate path (`split`: its split pass). Fitted
-// to both paths at 5k to 1M rows of 32 to 768 floats with 1 to 128 queries,
-// k = 10, device pointers. Either path reads the store from memory once; the
-// candidate path has more launches (48 us; 62 in f32, and whole 128-query
-// blocks at 80% of the FP32 matrix peak), the exact scan streams the store
-// through L2 again for every further query. Measured, candidates / exact, us:
-// 100k x 128 59/51 at 2 queries, 60/67 at 3, 61/121 at 16 (the scan was taken
-// up to 13: 100); 20k x 128 54/47 at 12, 55/63 at 16, 55/74 at 32 (taken up
-// to 52); 300k x 256 97/119 at 1, 99/195 at 6 (taken up to 5); 1M x 768
-// 589/595 at 1, 580/1140 at 4 (taken up to 4); 100k x 32 in f32 69/72 at 12,
-// 70/110 at 32; 20k x 32 70/58 at 48, 72/78 at 96.
-static bool exact_scan_cheaper(size_t N, size_t dim, size_t nq, bool split) {
-  const double nd = (double)N * (double)dim;
-  const double t_mfma = split ? 4.8e-5 + nd * 4.0 / 5.2e12 + (double)nq * (2.0e-7 + nd * 2.4e-15)
-                              : 6.2e-5 + (double)nq * 1.0e-7 + (double)((nq + 127) / 128) * nd * 256.0 / 1.25e14;
-  const double t_exact = 3.5e-5 + nd * 4.0 / 4.2e12 + (double)(nq - 1) * (2.0e-7 + (double)N * 1.0e-11 + nd * 3.5e-13);
-  return t_exact < t_mfma;
+// The candidate pass's tiling: 32 QT queries per workgroup (FB_M, or 32 or 64
+// for a smaller batch on the split pass), QB blocks of them, S splits of the
+// store, four tiles or more each and FLAT_MAX_SPLITS workgroups at most.
+struct FlatTiling {
+  int QT, QB, S;
+  FlatTiling(size_t nq, int tiles, bool split) {
+    QT = !split || nq > 64 ? 4 : nq > 32 ? 2 : 1;
+    QB = (int)((nq + 32 * QT - 1) / (32 * QT));
+    S = std::max(1, std::min(FLAT_MAX_SPLITS / QB, std::max(1, tiles / 4)));
+  }
+};
+
+// Whether the exact scan is expected to finish nq queries of kq results over
+// N rows of dim floats sooner than the candidate path (`split`: its split
+// pass). The constants (microseconds) are fitted to both paths' times at 13
+// stores of 4500 x 16 to 1M x 768 with 1 to 256 queries and k of 1 to 256,
+// device pointers, 884 pairs: the path taken is 0.1% behind the better one on
+// average and 11% at worst (10k x 768, 24 queries, k = 256).
+//
+// Candidates: launches, then the longer of reading the store and the slices of
+// 32 dimensions that a workgroup's tiles take one after another (few splits of
+// wide rows leave CUs without a workgroup: 30k x 768 takes 117 us for 3
+// queries, 77 by the exact scan), and part of the shorter; the merge of more
+// than 48 or 112 results. In f32 whole 128-query blocks at 80% of the FP32
+// matrix peak. Exact scan: the store from memory once and through L2 for every
+// further query, and beyond 64 results a select over every chunk's keys (100k
+// x 128, one query, k = 100: 168 us against 64). Both in us, candidates /
+// exact: 100k x 128 58/49 at 2 queries, 58/65 at 3; 20k x 128 54/47 at 12,
+// 54/61 at 16; 300k x 256 96/114 at 1; 1M x 768 568/587 at 1; 60k x 300 84/70
+// at 4, 84/100 at 6; 20k x 32 in f32 69/57 at 48, 71/78 at 96; 4500 x 64 58/51
+// at 64, 70/73 at 256.
+static bool exact_scan_cheaper(size_t N, size_t dim, size_t nq, uint64_t kq, bool split) {
+  const double n = (double)N, nd = n * (double)dim, q = (double)nq;
+  const int tiles = (int)((N + FB_N - 1) / FB_N);
+  double cand = kq + MARGIN <= 64 ? 0.0 : kq + MARGIN <= 128 ? 11.6 : 18.4;
+  if (split) {
+    const FlatTiling t(nq, tiles, true);
+    const double slices = (double)((tiles + t.S - 1) / t.S) * (double)((dim + FB_K - 1) / FB_K);
+    const double chain = 0.77 * slices, read = nd * 4.0 / 5.8e6;
+    cand += 39.3 + std::max(read, chain) + 0.63 * std::min(read, chain) + q * (0.237 + nd * 1.92e-9);
+  } else {
+    cand += 64.5 + q * 0.19 + (double)((nq + 127) / 128) * nd * 256.0 / 1.25e8;
+  }
+  double exact = 35.0 + nd * 4.0 / 3.41e6 + (q - 1.0) * (0.126 + n * 1.07e-5 + nd * 4.38e-7);
+  if (kq > WAVE) {
+    const size_t QG = (size_t)exact_query_group(nq, dim, N);
+    const size_t CH = (size_t)exact_chunk_rows((nq + QG - 1) / QG, N);
+    exact += 10.8 + 0.003 * (double)((N + CH - 1) / CH) * (double)std::min<uint64_t>(kq, CH);
+  }
+  return exact < cand;
 }
 
 FlatIndex::~FlatIndex() {
@@ -1032,7 +1064,7 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
   // rows and batches the exact scan finishes sooner.
   const bool split_ok = dim >= SPLIT_MIN_DIM && split_norm_ok(maxnorm);
   const bool exact_all = mode == 2 || metric == PXG_MANHATTAN || kq > FAST_KMAX ||
-                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq, split_ok)));
+                         (mode == 0 && (N < 4096 || exact_scan_cheaper(N, dim, nq, kq, split_ok)));
   const int Kp = (int)std::min<uint64_t>(kq + MARGIN, (uint64_t)FAST_KMAX + MARGIN);
   // a row's buffer holds its Kp keys, one tile's appends (FB_N) and at
   // least 64 more before it must be compacted
@@ -1095,11 +1127,9 @@ void FlatIndex::search_device(const float* d_raw, bool do_prepare, uint64_t nq, 
 
   if (!exact_all) {
     flag_list = (int*)sc.get(5, nq * 4);
-    // queries per workgroup: FB_M, or 32 or 64 for a smaller batch on the
-    // split pass
-    const int QT = !split || nq > 64 ? 4 : nq > 32 ? 2 : 1;
-    const int QB = (int)((nq + 32 * QT - 1) / (32 * QT));
-    int S = std::max(1, std::min(FLAT_MAX_SPLITS / QB, std::max(1, tiles / 4)));
+    const FlatTiling t(nq, tiles, split);
+    const int QT = t.QT, QB = t.QB;
+    int S = t.S;
     // a fixed scratch may hold fewer splits (the results do not depend on S)
     const size_t fit = sc.room() / per_split_bytes;
     if (fit == 0) (void)sc.get(6, per_split_bytes);  // raises the capacity error
