@@ -2401,12 +2401,17 @@ static void launch_farthest(const float* dist, size_t n, unsigned long long* par
 // theta. So if the largest exact distance over the pool is above theta, the
 // farthest point (the first index among equal distances) is in the pool, and
 // is the pool's. An empty cluster then costs an exact scan of its pool and a
-// reduction instead of passes over every point; if the test fails at any
-// empty cluster, the segment passes redo them all. The bounds don't depend on
-// the victims, so three launches make the pools of RESEED_BATCH empty
-// clusters (a sort of the bounds takes 40 us at 60k points, per cluster). A
-// victim brings down the points around it, in clustered data about n / k,
-// whose bounds stay: each victim so far adds twice that many points.
+// reduction instead of passes over every point. The bounds don't depend on the
+// victims, so three launches make the pools of RESEED_BATCH empty clusters (a
+// sort of the bounds takes 40 us at 60k points, per cluster). A victim brings
+// down the points around it, in clustered data about n / k, whose bounds stay:
+// each victim so far adds twice that many points. If the test fails at any
+// empty cluster (a far group of more points than that keeps its bounds after
+// the first victim out of it), pools of the largest size are tried where they
+// hold no more than n points together, and then the segment passes redo them
+// all: 300k x 128, 1024 clusters, 6000 points far off, a call with 2 empty
+// clusters 15.3 ms without the second try and 10.5 with it, with 20 18.0 and
+// 13.5; 60k x 768 with 20 the passes are the faster (9.7 against 11.4 ms).
 // 60k x 100, 300 clusters, 18 empty ones in 8 iterations: a call 3.2 ms with
 // a sort, two copies of the array, an exact scan of 8192 points and three more
 // launches per empty cluster -> 2.5 ms; 2M x 128, 4096 clusters, 18 empty
@@ -2775,50 +2780,55 @@ KmeansOut kmeans_device(const float* P, size_t n, int dim, int ldp, size_t k_req
       if (h_counts[c] == 0) E.push_back(c);
     const size_t m = E.size();
     if (m >= 1 && pool_fits) {
-      const size_t per = 2 * ((n + k - 1) / k);
-      const auto pool_at = [&](size_t i) { return std::min(pool_max, RESEED_BASE + i * per); };
-      const size_t pool = pool_at(m - 1);
       const size_t mb = std::min(m, RESEED_BATCH);
+      size_t base = RESEED_BASE, per = 2 * ((n + k - 1) / k);
+      const auto pool_at = [&](size_t i) { return std::min(pool_max, base + i * per); };
       rs_hist.reserve(mb * RESEED_BINS);
-      rs_list.reserve(mb * pool);
       rs_e.reserve(3 * RESEED_BATCH);
       rs_dnew.reserve(n);
-      pool_d.reserve(pool);
       hipLaunchKernelGGL(km_reseed_bound, dim3((unsigned)((n + KV_PB - 1) / KV_PB)), dim3(256), 0, s, P, ldp, (int)n,
                          dim, (const float*)newc.p, (const uint32_t*)assign.p, rs_dnew.p);
-      PXG_HIP(hipMemsetAsync(pool_fail.p, 0, 4, s));
-      uint32_t* cut = rs_e.p + RESEED_BATCH;
-      uint32_t* cnt = cut + RESEED_BATCH;
-      uint32_t h_e[RESEED_BATCH];
-      for (size_t i0 = 0; i0 < m; i0 += mb) {
-        const size_t b = std::min(mb, m - i0);
-        if (i0 > 0) PXG_HIP(hipStreamSynchronize(s));  // h_e is still being read
-        for (size_t ii = 0; ii < b; ++ii) h_e[ii] = (uint32_t)E[i0 + ii];
-        PXG_HIP(hipMemcpyAsync(rs_e.p, h_e, b * 4, hipMemcpyHostToDevice, s));
-        PXG_HIP(hipMemsetAsync(rs_hist.p, 0, b * RESEED_BINS * 4, s));
-        const dim3 gr((unsigned)((n + RESEED_TILE - 1) / RESEED_TILE), (unsigned)b);
-        hipLaunchKernelGGL(km_reseed_hist, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
-                           (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, rs_hist.p);
-        hipLaunchKernelGGL(km_reseed_cut, dim3((unsigned)b), dim3(1024), 0, s, (const uint32_t*)rs_hist.p,
-                           (uint32_t)pool_at(i0), (uint32_t)per, (uint32_t)pool_max, cut, cnt);
-        hipLaunchKernelGGL(km_reseed_list, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
-                           (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, (const uint32_t*)cut, (int)pool,
-                           cnt, rs_list.p);
-        for (size_t ii = 0; ii < b; ++ii) {
-          const size_t c = E[i0 + ii];
-          const uint32_t* list = rs_list.p + ii * pool;
-          hipLaunchKernelGGL(km_exact_pool, dim3((unsigned)((pool_at(i0 + ii) + KX_PB - 1) / KX_PB)), dim3(KP_WAVES * WAVE),
-                             (size_t)KX_PB * (dim + 4) * 4, s, P, ldp, list, (const uint32_t*)(cnt + ii), (uint32_t)c, dim,
-                             (const float*)newc.p, (const float*)cents.p, (int)k, pool_d.p);
-          hipLaunchKernelGGL(km_pool_farthest, dim3(1), dim3(1024), 0, s, P, ldp, dim, list,
-                             (const uint32_t*)(cnt + ii), (const float*)pool_d.p, (const uint32_t*)(cut + ii),
-                             (int)((long long)(i0 + ii) == fail_at), newc.p + c * dim, pool_fail.p);
-        }
-        PXG_HIP(hipGetLastError());
-      }
+      // a pool whose test fails is tried once more at the largest size
       int h_fail = 0;
-      PXG_HIP(hipMemcpyAsync(&h_fail, pool_fail.p, 4, hipMemcpyDeviceToHost, s));
-      PXG_HIP(hipStreamSynchronize(s));
+      for (bool again = true; again;) {
+        const size_t pool = pool_at(m - 1);
+        rs_list.reserve(mb * pool);
+        pool_d.reserve(pool);
+        PXG_HIP(hipMemsetAsync(pool_fail.p, 0, 4, s));
+        uint32_t* cut = rs_e.p + RESEED_BATCH;
+        uint32_t* cnt = cut + RESEED_BATCH;
+        uint32_t h_e[RESEED_BATCH];
+        for (size_t i0 = 0; i0 < m; i0 += mb) {
+          const size_t b = std::min(mb, m - i0);
+          if (i0 > 0) PXG_HIP(hipStreamSynchronize(s));  // h_e is still being read
+          for (size_t ii = 0; ii < b; ++ii) h_e[ii] = (uint32_t)E[i0 + ii];
+          PXG_HIP(hipMemcpyAsync(rs_e.p, h_e, b * 4, hipMemcpyHostToDevice, s));
+          PXG_HIP(hipMemsetAsync(rs_hist.p, 0, b * RESEED_BINS * 4, s));
+          const dim3 gr((unsigned)((n + RESEED_TILE - 1) / RESEED_TILE), (unsigned)b);
+          hipLaunchKernelGGL(km_reseed_hist, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
+                             (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, rs_hist.p);
+          hipLaunchKernelGGL(km_reseed_cut, dim3((unsigned)b), dim3(1024), 0, s, (const uint32_t*)rs_hist.p,
+                             (uint32_t)pool_at(i0), (uint32_t)per, (uint32_t)pool_max, cut, cnt);
+          hipLaunchKernelGGL(km_reseed_list, gr, dim3(1024), 0, s, (const uint32_t*)assign.p, (const float*)dist.p,
+                             (const float*)rs_dnew.p, (int)n, (const uint32_t*)rs_e.p, (const uint32_t*)cut, (int)pool,
+                             cnt, rs_list.p);
+          for (size_t ii = 0; ii < b; ++ii) {
+            const size_t c = E[i0 + ii];
+            const uint32_t* list = rs_list.p + ii * pool;
+            hipLaunchKernelGGL(km_exact_pool, dim3((unsigned)((pool_at(i0 + ii) + KX_PB - 1) / KX_PB)), dim3(KP_WAVES * WAVE),
+                               (size_t)KX_PB * (dim + 4) * 4, s, P, ldp, list, (const uint32_t*)(cnt + ii), (uint32_t)c, dim,
+                               (const float*)newc.p, (const float*)cents.p, (int)k, pool_d.p);
+            hipLaunchKernelGGL(km_pool_farthest, dim3(1), dim3(1024), 0, s, P, ldp, dim, list,
+                               (const uint32_t*)(cnt + ii), (const float*)pool_d.p, (const uint32_t*)(cut + ii),
+                               (int)((long long)(i0 + ii) == fail_at), newc.p + c * dim, pool_fail.p);
+          }
+          PXG_HIP(hipGetLastError());
+        }
+        PXG_HIP(hipMemcpyAsync(&h_fail, pool_fail.p, 4, hipMemcpyDeviceToHost, s));
+        PXG_HIP(hipStreamSynchronize(s));
+        again = h_fail != 0 && base < pool_max && m * pool_max <= n;
+        base = pool_max;
+      }
       if (h_fail) {
         ++pool_fallbacks;  // the passes below redo every empty cluster, victims included
       } else {

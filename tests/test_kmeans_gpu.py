@@ -486,3 +486,20 @@ def test_kmeans_pp_sums_that_are_not_finite_are_refused(gpu, n, dim, k):
     # the next call is served
     ok = (pts * np.float32(1e-25)).astype(np.float32)
     assert np.array_equal(bits(gpu.kmeans_pp(ok, k, 5)), bits(orc.kmeans_pp(ok, k, 5)))
+
+
+def test_lloyd_far_group_larger_than_the_first_pool(gpu):
+    """Two empty clusters and a far group of 3000 points: after the first victim
+    the second pool (1024 + 2 n / k points) holds nothing but that group, and
+    the largest one (8192) finds the next victim without the segment passes."""
+    rng = np.random.default_rng(12)
+    n, dim, k = 40_000, 8, 64
+    pts = clustered(rng, n, dim, 40, 0.3)
+    pts[:3000] = 60.0 + rng.standard_normal((3000, dim))
+    init = pts[3000::(n - 3000) // k][:k].copy()
+    init[0], init[5] = -900.0, -950.0
+    c, a, inertia, its = gpu.kmeans_lloyd(pts, init, 3)
+    stats = gpu.kmeans_last_reseeds()
+    assert stats["reseeds"] >= 2 and stats["pool"] == stats["reseeds"] and stats["pool_fallbacks"] == 0, stats
+    wc, wa, wi, wit = orc.kmeans_lloyd(pts, init, 3)
+    assert np.array_equal(bits(c), bits(wc)) and np.array_equal(a, wa) and inertia == wi and its == wit
