@@ -1543,9 +1543,9 @@ __global__ __launch_bounds__(256) void km_pp_round(const float* __restrict__ P, 
 //     point (kmeans.rs:169-186 picks rows) with an int8 copy: from the exact
 //     integer dot product, e = |s_i q_i - s_c q_c| and |p_i - c| >= e -
 //     delta_i - delta_c. Reads dim / 2 + 4 bytes.
-//  3. The same with the point's own int8 copy (scale max|p_i| / 119, so that
-//     a code is 16 a + b with a and b in [-8, 7], the two 4-bit words that
-//     step 2 multiplies). Reads dim + 12 bytes.
+//  3. The same with the point's own int8 copy (scale max|p_i| / 127; with step
+//     2 max|p_i| / 119, so that a code is 16 a + b with a and b in [-8, 7], the
+//     two 4-bit words that step 2 multiplies). Reads dim + 12 bytes.
 //
 // The points none of them settles (those the centre may capture) are scored
 // exactly as km_pp_round does. Blocks none of whose distances changed keep
@@ -1565,8 +1565,10 @@ constexpr int Q8_MAX = 119;
 __device__ __forceinline__ uint32_t bf16_up(float x) { return (__float_as_uint(x) + 0xFFFFu) >> 16; }
 
 // The copies, scales, deltas and the int8 copy's squared norm: one wave per
-// point. Q4: 16-byte chunks of 32 dimensions, dimension j the nibble j % 8 of
-// word j / 8; meta4: bf16 scale << 16 | bf16 delta.
+// point. FOUR: with the 4-bit copy, Q4 in 16-byte chunks of 32 dimensions,
+// dimension j the nibble j % 8 of word j / 8; meta4: bf16 scale << 16 | bf16
+// delta.
+template <bool FOUR>
 __global__ __launch_bounds__(256) void km_q8_prep(const float* __restrict__ P, int ldp, int n, int dim, int kq,
                                                   int8_t* __restrict__ Q, float* __restrict__ scale,
                                                   float* __restrict__ delta, int* __restrict__ qnorm, int words4,
@@ -1578,32 +1580,40 @@ __global__ __launch_bounds__(256) void km_q8_prep(const float* __restrict__ P, i
   float mx = 0.0f;
   for (int j = lane; j < dim; j += 64) mx = fmaxf(mx, fabsf(p[j]));
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  const float sc = mx / (float)Q8_MAX;
-  const float s4u = __uint_as_float(bf16_up(mx / 7.0f) << 16);
-  const float s4 = isfinite(s4u) ? s4u : 0.0f;
-  double d2 = 0.0, d42 = 0.0;
+  constexpr int QM = FOUR ? Q8_MAX : 127;
+  const float sc = mx / (float)QM;
+  [[maybe_unused]] float s4 = 0.0f;
+  if constexpr (FOUR) {
+    const float s4u = __uint_as_float(bf16_up(mx / 7.0f) << 16);
+    s4 = isfinite(s4u) ? s4u : 0.0f;
+  }
+  double d2 = 0.0;
+  [[maybe_unused]] double d42 = 0.0;
   int qn = 0;
-  for (int j0 = 0; j0 < words4 * 8; j0 += 64) {
+  for (int j0 = 0; j0 < (FOUR ? words4 * 8 : kq); j0 += 64) {
     const int j = j0 + lane;
     const float x = j < dim ? p[j] : 0.0f;
-    int q = 0, q4 = 0;
-    if (sc > 0.0f) q = max(-Q8_MAX, min(Q8_MAX, (int)rintf(x / sc)));
-    if (s4 > 0.0f) q4 = max(-7, min(7, (int)rintf(x / s4)));
-    const double r = (double)x - (double)q * (double)sc, r4 = (double)x - (double)q4 * (double)s4;
+    int q = 0;
+    if (sc > 0.0f) q = max(-QM, min(QM, (int)rintf(x / sc)));
+    const double r = (double)x - (double)q * (double)sc;
     d2 += r * r;
-    d42 += r4 * r4;
     qn += q * q;
     if (j < kq) Q[(size_t)i * kq + j] = (int8_t)q;
+    if constexpr (!FOUR) continue;
+    int q4 = 0;
+    if (s4 > 0.0f) q4 = max(-7, min(7, (int)rintf(x / s4)));
+    const double r4 = (double)x - (double)q4 * (double)s4;
+    d42 += r4 * r4;
     // eight lanes' nibbles to one word
     uint32_t w = (uint32_t)(q4 & 15) << (4 * (lane & 7));
     w |= xor_lane<1>(w);
     w |= xor_lane<2>(w);
     w |= xor_lane<4>(w);
-    if (Q4 != nullptr && (lane & 7) == 0 && j < words4 * 8) Q4[(size_t)i * words4 + (j >> 3)] = w;
+    if ((lane & 7) == 0 && j < words4 * 8) Q4[(size_t)i * words4 + (j >> 3)] = w;
   }
   for (int o = 32; o > 0; o >>= 1) {
     d2 += __shfl_xor(d2, o, 64);
-    d42 += __shfl_xor(d42, o, 64);
+    if constexpr (FOUR) d42 += __shfl_xor(d42, o, 64);
     qn += __shfl_xor(qn, o, 64);
   }
   if (lane == 0) {
@@ -1616,7 +1626,7 @@ __global__ __launch_bounds__(256) void km_q8_prep(const float* __restrict__ P, i
       return isfinite(mx) ? df : INFINITY;
     };
     delta[i] = up(d2);
-    meta4[i] = (__float_as_uint(s4) & 0xFFFF0000u) | bf16_up(up(d42));
+    if constexpr (FOUR) meta4[i] = (__float_as_uint(s4) & 0xFFFF0000u) | bf16_up(up(d42));
     qnorm[i] = qn;
   }
 }
@@ -1656,13 +1666,10 @@ __device__ __forceinline__ bool km_pp_keeps(float cur, double sp, double qn, dou
   return isfinite(cur) && L > 0.0 && L * L * (1.0 - gamma) >= (double)cur + 1e-35;
 }
 
-// One round. SUB blocks of PP_ROWS points per workgroup: four for stores whose
-// copies are read from memory (half a million points on), with LP lanes per
-// 4-bit row; one for smaller ones, which leave out step 2 (their round is a
-// chain of dependent loads and not bytes: with it 100k x 96 takes 8.6 us
-// instead of 7.9). Eight workgroups fit a CU (64 VGPRs, 15 KB of LDS up to 256
-// dimensions), so a round's workgroups are all resident at once and their
-// chains of dependent loads overlap.
+// One round. SUB blocks of PP_ROWS points per workgroup: four with step 2 (LP
+// lanes per 4-bit row), one without it. Eight workgroups fit a CU (64 VGPRs,
+// 15 KB of LDS up to 256 dimensions), so a round's workgroups are all resident
+// at once and their chains of dependent loads overlap.
 template <int LP, int SUB>
 __global__ __launch_bounds__(256, 8) void km_pp_round_q8(const float* __restrict__ P, int ldp, int n, int dim,
                                                          const int8_t* __restrict__ Q, int kq,
@@ -1678,6 +1685,7 @@ __global__ __launch_bounds__(256, 8) void km_pp_round_q8(const float* __restrict
   static_assert(PP_ROWS == 256, "one point per thread and sub-block");
   constexpr int PTS = SUB * PP_ROWS;
   constexpr bool FOUR = SUB > 1;
+  static_assert(!FOUR || LP <= 8, "a 4-bit row's chunks, one per lane");
   constexpr int WMAX = (LP < 16 ? 32 * LP : KW_DMAX) / 8;  // words of 8 nibbles
   __shared__ __align__(16) uint32_t ch4[FOUR ? WMAX : 4], cl4[FOUR ? WMAX : 4];  // the centre's 4-bit words
   __shared__ int qc[2 * WMAX];                             // its int8 codes
@@ -1747,59 +1755,38 @@ __global__ __launch_bounds__(256, 8) void km_pp_round_q8(const float* __restrict
       uint32_t mt[PER];
 #pragma unroll
       for (int x = 0; x < PER; ++x) mt[x] = meta4[base + act[min(u0 + ((sub + x * LP) & 3) * G + g, m1 - 1)]];
-      if constexpr (LP < 16) {
-        // at most LP chunks: one load per point and lane
-        uint4 v[4];
-        const bool on = sub < chunks;
+      // at most LP chunks: one load per point and lane
+      uint4 v[4];
+      const bool on = sub < chunks;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const size_t i = base + act[min(u0 + e * G + g, m1 - 1)];
-          v[e] = *reinterpret_cast<const uint4*>(Q4 + i * words4 + 4 * (on ? sub : 0));
+      for (int e = 0; e < 4; ++e) {
+        const size_t i = base + act[min(u0 + e * G + g, m1 - 1)];
+        v[e] = *reinterpret_cast<const uint4*>(Q4 + i * words4 + 4 * (on ? sub : 0));
+      }
+      uint4 ca = make_uint4(0, 0, 0, 0), cb = ca;
+      if (on) {
+        ca = *reinterpret_cast<const uint4*>(ch4 + 4 * sub);
+        cb = *reinterpret_cast<const uint4*>(cl4 + 4 * sub);
+      }
+      const int cav[4] = {(int)ca.x, (int)ca.y, (int)ca.z, (int)ca.w};
+      const int cbv[4] = {(int)cb.x, (int)cb.y, (int)cb.z, (int)cb.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int w[4] = {(int)v[e].x, (int)v[e].y, (int)v[e].z, (int)v[e].w};
+        int da = 0, db = 0, q = 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          da = __builtin_amdgcn_sdot8(w[x], cav[x], da, false);
+          db = __builtin_amdgcn_sdot8(w[x], cbv[x], db, false);
+          q = __builtin_amdgcn_sdot8(w[x], w[x], q, false);
         }
-        uint4 ca = make_uint4(0, 0, 0, 0), cb = ca;
-        if (on) {
-          ca = *reinterpret_cast<const uint4*>(ch4 + 4 * sub);
-          cb = *reinterpret_cast<const uint4*>(cl4 + 4 * sub);
-        }
-        const int cav[4] = {(int)ca.x, (int)ca.y, (int)ca.z, (int)ca.w};
-        const int cbv[4] = {(int)cb.x, (int)cb.y, (int)cb.z, (int)cb.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int w[4] = {(int)v[e].x, (int)v[e].y, (int)v[e].z, (int)v[e].w};
-          int da = 0, db = 0, q = 0;
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            da = __builtin_amdgcn_sdot8(w[x], cav[x], da, false);
-            db = __builtin_amdgcn_sdot8(w[x], cbv[x], db, false);
-            q = __builtin_amdgcn_sdot8(w[x], w[x], q, false);
-          }
-          dot[e] = 16 * da + db;
-          qn[e] = on ? q : 0;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const size_t i = base + act[min(u0 + e * G + g, m1 - 1)];
-          int da = 0, db = 0, q = 0;
-          for (int ck = sub; ck < chunks; ck += LP) {
-            const uint4 v = *reinterpret_cast<const uint4*>(Q4 + i * words4 + 4 * ck);
-            const int w[4] = {(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              da = __builtin_amdgcn_sdot8(w[x], (int)ch4[4 * ck + x], da, false);
-              db = __builtin_amdgcn_sdot8(w[x], (int)cl4[4 * ck + x], db, false);
-              q = __builtin_amdgcn_sdot8(w[x], w[x], q, false);
-            }
-          }
-          dot[e] = 16 * da + db;
-          qn[e] = q;
-        }
+        dot[e] = 16 * da + db;
+        qn[e] = on ? q : 0;
       }
       auto sum = [](int x) {
         if constexpr (LP >= 2) x += (int)xor_lane<1>((uint32_t)x);
         if constexpr (LP >= 4) x += (int)xor_lane<2>((uint32_t)x);
         if constexpr (LP >= 8) x += (int)xor_lane<4>((uint32_t)x);
-        if constexpr (LP >= 16) x += (int)xor_lane<8>((uint32_t)x);
         return x;
       };
 #pragma unroll
@@ -2150,22 +2137,36 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   const int vec4 = (ldp % 4 == 0 && dim % 4 == 0 && ((uintptr_t)P & 15) == 0) ? 1 : 0;
   hipLaunchKernelGGL(km_pp_round, dim3(nb), dim3(256), 0, s, P, ldp, (int)n, dim, cents, ns.p, 1, ps.p, pe.p, vec4);
   PXG_HIP(hipGetLastError());
-  // rounds after the first over the certified 4-bit and int8 copies (dim >=
-  // 32; for narrower points the copies save little of each row's bytes)
+  // rounds after the first over the certified copies (dim >= 32; for narrower
+  // points they save little of each row's bytes)
   const bool q8 = dim >= 32 && dim <= KW_DMAX && k > 1;
   const int kq = (dim + 3) / 4 * 4, words4 = (dim + 31) / 32 * 4;
   DevBuf<int8_t> Q(q8 ? n * kq : 0);
   DevBuf<float> qscale(q8 ? n : 0), qdelta(q8 ? n : 0);
   DevBuf<int> qnorm(q8 ? n : 0);
-  // four blocks of points per workgroup once that still gives every CU two
-  const bool wide = nb >= 4 * 512;
-  DevBuf<uint32_t> q4(q8 && wide ? n * words4 : 0), qmeta4(q8 ? n : 0);
+  // Step 2 pays where the int8 copies are far larger than the L2s and there
+  // are rounds enough for the 4-bit ones' preparation: 2M x 128, rounds 66 to
+  // 130 / 258 to 514 68 / 53 us with it, 76 / 69 without, in all 258 rounds
+  // 23.6 and 26.4 ms. Smaller stores and wider rows lose by it (their rounds
+  // are chains of dependent loads, and the coarser copy settles few points in
+  // many dimensions): 530k x 100, 130 rounds 9.1 against 8.1 ms, 530k x 300
+  // 20.6 against 15.3, 600k x 1000 50.8 against 33.4.
+  // (PXG_PP_FOUR=size takes it from that many components and any k on, so that
+  // small inputs can: a test hook, the results are the same either way.)
+  const char* four_env = std::getenv("PXG_PP_FOUR");
+  const size_t four_from = four_env ? (size_t)std::strtoull(four_env, nullptr, 10) : (size_t)1 << 27;
+  const bool four = q8 && dim <= 256 && n * (size_t)dim >= four_from && (k > 64 || four_env);
+  DevBuf<uint32_t> q4(four ? n * words4 : 0), qmeta4(four ? n : 0);
   DevBuf<uint32_t> near(q8 ? n : 0);  // every distance is to centre 0 so far
   DevBuf<float> tnear(q8 ? k : 0);
   if (q8) {
     PXG_HIP(hipMemsetAsync(near.p, 0, n * 4, s));
-    hipLaunchKernelGGL(km_q8_prep, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, P, ldp, (int)n, dim, kq, Q.p,
-                       qscale.p, qdelta.p, qnorm.p, words4, wide ? q4.p : nullptr, qmeta4.p);
+    if (four)
+      hipLaunchKernelGGL(km_q8_prep<true>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, P, ldp, (int)n, dim, kq,
+                         Q.p, qscale.p, qdelta.p, qnorm.p, words4, q4.p, qmeta4.p);
+    else
+      hipLaunchKernelGGL(km_q8_prep<false>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, P, ldp, (int)n, dim, kq,
+                         Q.p, qscale.p, qdelta.p, qnorm.p, 0, (uint32_t*)nullptr, (uint32_t*)nullptr);
     PXG_HIP(hipGetLastError());
   }
   const double gamma = (double)(dim + 4) * 0x1p-24 * 1.01;
@@ -2182,7 +2183,7 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
                      (const int8_t*)Q.p, kq, (const float*)qscale.p, (const float*)qdelta.p, (const int*)qnorm.p,    \
                      (const uint32_t*)q4.p, (const uint32_t*)qmeta4.p, words4, (const int*)picked, ns.p, ps.p,       \
                      pe.p, gamma, near.p, (const float*)tnear.p, (int)chosen)
-        if (!wide) {
+        if (!four) {
           if (dim <= 256) PXG_PP(8, 1); else PXG_PP(16, 1);
         } else if (dim <= 32) {
           PXG_PP(1, 4);
@@ -2190,10 +2191,8 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
           PXG_PP(2, 4);
         } else if (dim <= 128) {
           PXG_PP(4, 4);
-        } else if (dim <= 256) {
-          PXG_PP(8, 4);
         } else {
-          PXG_PP(16, 4);
+          PXG_PP(8, 4);
         }
 #undef PXG_PP
       } else

@@ -459,11 +459,15 @@ def test_lloyd_split_any_alignment(gpu, dim):
     assert np.array_equal(want[1], assign) and want[2] == inertia and want[3] == its
 
 
+@pytest.mark.parametrize("four", [True, False])
 @pytest.mark.parametrize("dim,k", [(32, 24), (60, 24), (100, 20), (200, 10), (270, 8)])
-def test_kmeans_pp_four_bit_rounds(gpu, dim, k):
-    """Enough points (2048 blocks of 256) for the rounds over the 4-bit copy, at
-    each of its lane counts: tight clusters, coarse copies (one large
+def test_kmeans_pp_four_bit_rounds(gpu, monkeypatch, dim, k, four):
+    """2048 blocks of 256 points and one more through the rounds over the 4-bit
+    copy, at each of its lane counts (up to 256 dimensions), and over the int8
+    copy alone: tight clusters, coarse copies (one large
     coordinate), duplicates and far outliers; the seeds are the oracle's bits."""
+    if four:
+        monkeypatch.setenv("PXG_PP_FOUR", "0")
     rng = np.random.default_rng(dim)
     n = 524_288 + 77
     pts = rng.standard_normal((15, dim)).astype(np.float32)[rng.integers(0, 15, n)]
