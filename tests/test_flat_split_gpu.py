@@ -109,3 +109,40 @@ def test_mixed_norms_and_ties(gpu, metric):
     data[3000] = 0.0
     q[:5] = data[7]
     _check(gpu, _index(gpu, data, metric), data, metric, q, 30)
+
+
+@pytest.mark.parametrize("metric", [0, 1, 2])
+@pytest.mark.parametrize("n,dim,nq", [(5003, 95, 20), (9001, 130, 50), (12_001, 64, 70), (8000, 768, 200)])
+def test_the_split_pass_answers(gpu, metric, n, dim, nq):
+    """Well separated rows of ordinary norms are answered from the candidates:
+    no query goes to the exact scan, whose results would hide a pass or a
+    certificate that always fails."""
+    rng = np.random.default_rng(dim + metric)
+    data, q = _clustered(rng, n, dim, nq)
+    idx = _index(gpu, data, metric)
+    _check(gpu, idx, data, metric, q, 10)
+    assert gpu.FlatIndex.last_fallbacks() == 0
+
+
+@pytest.mark.parametrize("nq,k,near", [(8, 10, 100), (300, 64, 100), (300, 100, 300), (800, 10, 100), (800, 256, 200),
+                                       (2000, 10, 100), (2000, 100, 300)])
+def test_merge_gathers_more_than_its_lds_holds(gpu, nq, k, near):
+    """20,000 rows are 32 splits of 640 (5 tiles) at every batch here. The first
+    tile of each, which seeds the threshold, is far off and `near` rows of the
+    rest are close, few enough that no list is compacted: every one of them is
+    at or below the seed threshold, 3200 to 9600 keys a query for merges that
+    hold 512 to 4096, so the merge gathers again, more than once for some."""
+    rng = np.random.default_rng(nq + k)
+    n, dim, split = 20_000, 64, 640
+    data = rng.standard_normal((n, dim))
+    data /= np.linalg.norm(data, axis=1, keepdims=True)
+    at = np.arange(n) % split
+    norm = np.where(at < 128, 2.0, 3.0) + rng.uniform(0.0, 0.2, n)
+    for a in range(0, n, split):
+        rows = a + 128 + rng.permutation(min(split, n - a) - 128)[:near] if n - a > 128 else []
+        norm[rows] = rng.uniform(0.9, 1.1, len(rows))
+    data = (data * norm[:, None]).astype(np.float32)
+    q = (0.01 * rng.standard_normal((nq, dim)) / 8.0).astype(np.float32)
+    idx = _index(gpu, data, 0)
+    _check(gpu, idx, data, 0, q, k)
+    assert gpu.FlatIndex.last_fallbacks() <= nq // 20

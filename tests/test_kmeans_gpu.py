@@ -507,3 +507,18 @@ def test_lloyd_far_group_larger_than_the_first_pool(gpu):
     assert stats["reseeds"] >= 2 and stats["pool"] == stats["reseeds"] and stats["pool_fallbacks"] == 0, stats
     wc, wa, wi, wit = orc.kmeans_lloyd(pts, init, 3)
     assert np.array_equal(bits(c), bits(wc)) and np.array_equal(a, wa) and inertia == wi and its == wit
+
+
+@pytest.mark.parametrize("dim,k", [(64, 64), (95, 97), (128, 200), (200, 100), (256, 64), (300, 64)])
+def test_assignment_passes_certify_what_they_can(gpu, dim, k):
+    """Well separated clusters: the matrix pass settles all but a few points,
+    which the exact scan of the rest would hide if it settled none."""
+    rng = np.random.default_rng(dim)
+    n = 6001
+    pts = clustered(rng, n, dim, k, 0.1)
+    init = (pts[:k] + np.float32(0.01)).astype(np.float32)
+    got = gpu.kmeans_lloyd(pts, init, 1)
+    stats = gpu.kmeans_last_stats()
+    assert stats["mfma_passes"] >= 1 and stats["rescanned"] <= n // 100, stats
+    want = orc.kmeans_lloyd(pts, init, 1)
+    assert np.array_equal(bits(got[0]), bits(want[0])) and np.array_equal(got[1], want[1]) and got[2] == want[2]
