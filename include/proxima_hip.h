@@ -166,8 +166,8 @@ int pxg_flat_search_device_noalloc(const pxg_flat* index, const float* d_queries
 uint64_t pxg_flat_last_fallbacks(void);
 /* Search path selection (no reference counterpart; for tests and tuning):
  * 0 = automatic (the exact scan for stores under 4096 rows and for batches
- * it is estimated to finish sooner, e.g. up to 2 queries over 100k x 128
- * or 12 over 20k x 128; otherwise the MFMA path), 1 = MFMA
+ * it is estimated to finish sooner, e.g. with k = 10 up to 2 queries over
+ * 100k x 128 or 15 over 20k x 128; otherwise the MFMA path), 1 = MFMA
  * candidates + exact rescoring whenever the metric and k allow it, 2 = exact
  * VALU scan only. Results are identical. */
 int pxg_flat_set_search_mode(pxg_flat* index, int mode);

@@ -565,43 +565,36 @@ __global__ __launch_bounds__(256, 2) void km_mfma_small(const float* __restrict_
                          blockIdx.x);
 }
 
-// km_mfma_reg: km_mfma_small's form for rows of 32 floats: each wave holds its 32 points' rows in VGPRs (lane half h
-// the dims [h dim/2, (h+1) dim/2)) for the whole pass, and the centroids
-// stream through LDS 32 rows at a time (a block of the MFMA), copied
+// km_mfma_reg: km_mfma_small's form for rows of 32 floats: each wave holds its
+// 32 points' rows in VGPRs (lane half h the dims [16 h, 16 h + 16)) for the
+// whole pass, and the centroids stream through LDS 32 rows at a time (a block
+// of the MFMA), copied
 // straight from memory (km_lds_copy16), double-buffered, one barrier per
 // block. Rows are stored unpadded with 16-byte chunk c of row r at position
 // c ^ (r & 7), so the lanes' float4 operand reads of 32 rows spread over the
 // banks. The top-2 scan is km_mfma_small's; no dot-product tile goes
 // through LDS. 128 points per 256-thread workgroup.
-template <int HD>  // dim / 2
 __global__ __launch_bounds__(256, 3) void km_mfma_reg(const float* __restrict__ P, int ldp,
                                                    const uint32_t* __restrict__ rows, int n,
                                                    const float* __restrict__ C, int ldc, int k,
                                                    const float* __restrict__ cn, uint32_t* __restrict__ best_idx,
                                                    float* __restrict__ best, float* __restrict__ second) {
-  constexpr int D = 2 * HD, CPR = D / 4;  // 16-byte chunks per row
-  static_assert(D % 32 == 0 && D <= 128, "whole groups of eight chunks per row");
-  constexpr int TILE = 32 * D;             // floats per centroid block
-  constexpr int NI = CPR / 8;              // copy instructions per wave per block (4 waves, 64 lanes)
+  constexpr int D = 32, HD = D / 2, CPR = D / 4;  // 16-byte chunks per row
+  constexpr int TILE = 32 * D;                    // floats per centroid block, one copy per lane
   __shared__ __align__(16) float sc[2 * TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, r = lane & 31;
   const int wid_s = __builtin_amdgcn_readfirstlane(w);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) float*)sc;
-  // the copy of block b into buffer buf: instruction u of wave w covers
-  // chunk positions 64 (w NI + u) + lane of the block
-  // (a full block's rows are the lane's fixed offsets plus the block's
-  // uniform first row; the last block clamps its rows to k - 1)
+  // the copy of block b into buffer buf: wave w covers chunk positions 64 w +
+  // lane of the block (a full block's rows are the lane's fixed offsets plus
+  // the block's uniform first row; the last block clamps its rows to k - 1)
   auto gload = [&](int b, int buf) __attribute__((always_inline)) {
     const bool full = b * 32 + 32 <= k;
     const float* cb = C + (size_t)(b * 32) * ldc;
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int g = wid_s * NI + u;
-      const int idx = 64 * g + lane, row = idx / CPR, pos = idx - row * CPR;
-      const int c = pos ^ (row & 7);
-      const float* src = full ? cb + (row * ldc + 4 * c) : C + (size_t)min(b * 32 + row, k - 1) * ldc + 4 * c;
-      km_lds_copy16(src, lds0 + (uint32_t)((buf * TILE + 64 * 4 * g) * 4));
-    }
+    const int idx = 64 * wid_s + lane, row = idx / CPR, pos = idx - row * CPR;
+    const int c = pos ^ (row & 7);
+    const float* src = full ? cb + (row * ldc + 4 * c) : C + (size_t)min(b * 32 + row, k - 1) * ldc + 4 * c;
+    km_lds_copy16(src, lds0 + (uint32_t)((buf * TILE + 64 * 4 * wid_s) * 4));
   };
   const int p0 = (blockIdx.x * 4 + w) * 32;
   const int pi = min(p0 + r, n - 1);
@@ -1118,9 +1111,8 @@ __global__ void km_compose_rows(const uint32_t* __restrict__ redo, int m, const 
   if (t < m) out[t] = rows ? rows[redo[t]] : redo[t];
 }
 
-// Points with enough work for the matrix cores
-// take the MFMA pass; the exact VALU scan serves the rest and the points the
-// MFMA pass cannot certify.
+// Points with enough work for the matrix cores take the MFMA pass; the exact
+// VALU scan serves the rest and the points the MFMA pass cannot certify.
 void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int dim, const float* C, int ldc,
                     size_t k, bool unrolled, uint32_t* assign, float* dist, hipStream_t s) {
   nearest_device(P, ldp, rows, n, dim, C, ldc, k, unrolled, assign, dist, s, nullptr);
@@ -1212,7 +1204,7 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
 #undef PXG_KM_SPLIT
     }
     else if (dim == 32)
-      hipLaunchKernelGGL(km_mfma_reg<16>, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
+      hipLaunchKernelGGL(km_mfma_reg, g128, dim3(256), 0, s, P, ldp, rows, (int)n, C, ldc, (int)k,
                          (const float*)cn, bidx, best, second);
     else
       hipLaunchKernelGGL(km_mfma_top, dim3((unsigned)((n + KA_M - 1) / KA_M)), dim3(256), 0, s, P, ldp, rows,
@@ -1233,7 +1225,7 @@ void nearest_device(const float* P, int ldp, const uint32_t* rows, size_t n, int
   int m = 0;
   PXG_HIP(hipMemcpyAsync(&m, nredo, 4, hipMemcpyDeviceToHost, s));
   PXG_HIP(hipStreamSynchronize(s));
-  if (!small) {  // the counters cover km_mfma_top
+  if (!small) {  // the counters cover km_split, km_mfma_reg and km_mfma_top
     float ms = 0.0f;
     PXG_HIP(hipEventElapsedTime(&ms, e0, e1));
     PXG_HIP(hipEventDestroy(e0));
