@@ -339,8 +339,12 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, r = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = qgroup * (WQ * QT * 32) + w % WQ * (QT * 32);
-  const int rb0 = w / WQ * RT;  // this wave's first row block
+  // without row groups the row block's offset is a constant: as a value that
+  // only the launch makes 0 it cost the 128-byte codes' widest scan 8 spilled
+  // registers (1000 queries over 1M codes 115 -> 131 us)
+  const int rg = RS == 1 ? 0 : w / WQ;  // this wave's row group
+  const int q0 = qgroup * (WQ * QT * 32) + (RS == 1 ? w : w % WQ) * (QT * 32);
+  const int rb0 = rg * RT;  // its first row block
   const bool active = q0 < nq;
 
   i4v qa[QT][KB];
@@ -420,7 +424,8 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
   // stage 2: the passing scores x[0..15] of a lane's query in row block rt of
   // tile t, to the workgroup list
   auto collect = [&](const i16v& x, int qt, int rt, int t) __attribute__((always_inline)) {
-    const int q = q0 + qt * 32 + r;
+    int q = q0 + qt * 32 + r;
+    asm volatile("" : "+v"(q));  // what hangs on q is worked out here, not held in registers over the scan
     const int tq = thr[qt];
     const int rowb = t * R + (rb0 + rt) * 32 + 4 * h;
 #pragma unroll
@@ -579,7 +584,7 @@ __global__ __launch_bounds__(SQ_NW * 64) void sq8_mfma_scan(
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const int q = q0 + qt * 32 + r;
-        if (q < nq) tmax[(size_t)q * (nchunks * 2 * RS) + (chunk * RS + w / WQ) * 2 + h] = run[qt];
+        if (q < nq) tmax[(size_t)q * (nchunks * 2 * RS) + (chunk * RS + rg) * 2 + h] = run[qt];
       }
     }
   } else {
