@@ -1894,7 +1894,11 @@ __device__ inline double wave_incl_scan_f64(double v, int lane) {
 // status: 0 ok, 1 non-finite total (the round and all later ones stop).
 // The prefix sums are wave scans joined through the 16 (or 4) wave totals:
 // under the certificate every order gives the exact sums, and otherwise this
-// is the fixed parallel order.
+// is the fixed parallel order. PER: partials per thread, at most (0: any
+// number), a kernel each, since they shape the whole of it: 2 a thread (520k
+// points) take 9.3 us loaded as they are and 11.0 through LDS, 8 (2M) 14.5 and
+// 11.4; one kernel for all forms costs one a thread (200k) 0.6 us of 8.3.
+template <int PER>
 __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int ldp, int n, int dim,
                                                    const float* __restrict__ ns, const double* __restrict__ ps,
                                                    const int* __restrict__ pe, int nb, ChaCha8* __restrict__ grng,
@@ -1915,35 +1919,47 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
   constexpr int RNG_WORDS = sizeof(ChaCha8) / 4;
   static_assert(sizeof(ChaCha8) % 4 == 0, "copied by words");
   if (t < RNG_WORDS) reinterpret_cast<uint32_t*>(rng_mem)[t] = reinterpret_cast<const uint32_t*>(grng)[t];
-  // each thread sums a contiguous run of block partials; up to PB of them
-  // come through LDS (coalesced loads, all in flight together; a run starts
-  // one place further on per thread, so that the threads' reads spread over
-  // the banks) and are held for the search below
-  constexpr int PB = 8;
-  __shared__ double sps[1024 * (PB + 1)];
+  // each thread sums a contiguous run of block partials; up to PER of them are
+  // held for the search below
   const int per = (nb + 1023) / 1024;
   const int b0 = min(nb, t * per), b1 = min(nb, (t + 1) * per);
-  double ls = 0.0, pv[PB];
+  double ls = 0.0;
+  [[maybe_unused]] double pv[PER > 0 ? PER : 1];
   int le = NO_TERMS;
-  if (per == 1) {
-    const int b = min(t, nb - 1);
-    pv[0] = ps[b];
-    const int e = pe[b];
-    if (t < nb) {
-      ls = pv[0];
-      le = e;
+  if constexpr (PER == 0) {
+    for (int b = b0; b < b1; ++b) {
+      ls += ps[b];
+      le = min(le, pe[b]);
     }
-  } else if (per <= PB) {
-    double lv[PB];
-    int ev[PB];
+  } else if constexpr (PER <= 3) {
+    int ev[PER];
 #pragma unroll
-    for (int u = 0; u < PB; ++u) {
+    for (int u = 0; u < PER; ++u) {
+      const int b = min(b0 + u, nb - 1);  // unconditional loads
+      pv[u] = ps[b];
+      ev[u] = pe[b];
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u)
+      if (b0 + u < b1) {
+        ls += pv[u];
+        le = min(le, ev[u]);
+      }
+  } else {
+    // through LDS: coalesced loads, all in flight together; a run starts one
+    // place further on per thread, so that the threads' reads spread over the
+    // banks
+    __shared__ double sps[1024 * (PER + 1)];
+    double lv[PER];
+    int ev[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
       const int b = min(u * 1024 + t, nb - 1);  // unconditional loads
       lv[u] = ps[b];
       ev[u] = pe[b];
     }
 #pragma unroll
-    for (int u = 0; u < PB; ++u)
+    for (int u = 0; u < PER; ++u)
       if (u * 1024 + t < nb) {
         const int b = u * 1024 + t;
         sps[b + b / per] = lv[u];
@@ -1951,16 +1967,11 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
       }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < PB; ++u)
+    for (int u = 0; u < PER; ++u)
       if (b0 + u < b1) {
         pv[u] = sps[b0 + t + u];
         ls += pv[u];
       }
-  } else {
-    for (int b = b0; b < b1; ++b) {
-      ls += ps[b];
-      le = min(le, pe[b]);
-    }
   }
   if (stat != 0) return;
   // inclusive scan over the threads: wave scans, then the earlier waves'
@@ -2028,10 +2039,10 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
     // first block whose inclusive prefix reaches the target, then the first
     // point inside it
     double run = before;
-    if (per <= PB) {
+    if constexpr (PER > 0) {
       bool found = false;
 #pragma unroll
-      for (int u = 0; u < PB; ++u)
+      for (int u = 0; u < PER; ++u)
         if (!found && b0 + u < b1) {
           if (run + pv[u] >= target) {
             atomicMin(&s_block, b0 + u);
@@ -2074,12 +2085,26 @@ __device__ __forceinline__ void km_pp_pick_body(const float* __restrict__ P, int
   if (t == 0 && picked_out) *picked_out = picked;
 }
 
+template <int PER>
 __global__ __launch_bounds__(1024) void km_pp_pick(const float* __restrict__ P, int ldp, int n, int dim,
                                                    const float* __restrict__ ns, const double* __restrict__ ps,
                                                    const int* __restrict__ pe, int nb, ChaCha8* __restrict__ grng,
                                                    float* __restrict__ row_out, int* __restrict__ status,
                                                    int* __restrict__ inexact, int* __restrict__ picked_out) {
-  km_pp_pick_body(P, ldp, n, dim, ns, ps, pe, nb, grng, row_out, status, inexact, picked_out);
+  km_pp_pick_body<PER>(P, ldp, n, dim, ns, ps, pe, nb, grng, row_out, status, inexact, picked_out);
+}
+// launch(PER) for nb blocks of partials
+template <class F>
+static void with_pick(int nb, F launch) {
+  const int per = (nb + 1023) / 1024;
+  if (per == 1)
+    launch(std::integral_constant<int, 1>{});
+  else if (per <= 3)
+    launch(std::integral_constant<int, 3>{});
+  else if (per <= 8)
+    launch(std::integral_constant<int, 8>{});
+  else
+    launch(std::integral_constant<int, 0>{});
 }
 
 __global__ void copy_row(const float* __restrict__ src, int ld_src, size_t row, int dim, float* __restrict__ dst) {
@@ -2164,8 +2189,10 @@ size_t kmeans_pp_device(const float* P, size_t n, int dim, int ldp, size_t k, Ch
   const double gamma = (double)(dim + 4) * 0x1p-24 * 1.01;
   for (size_t chosen = 1; chosen < k; ++chosen) {
     float* c = cents + chosen * dim;
-    hipLaunchKernelGGL(km_pp_pick, dim3(1), dim3(1024), 0, s, P, ldp, (int)n, dim, ns.p, ps.p, pe.p, nb, drng.p, c,
-                       flags.p, flags.p + 1, picked);
+    with_pick(nb, [&](auto per) {
+      hipLaunchKernelGGL(km_pp_pick<decltype(per)::value>, dim3(1), dim3(1024), 0, s, P, ldp, (int)n, dim, ns.p, ps.p,
+                         pe.p, nb, drng.p, c, flags.p, flags.p + 1, picked);
+    });
     if (chosen + 1 < k) {
       if (q8) {
         hipLaunchKernelGGL(km_pp_cdist, dim3((unsigned)((chosen + 15) / 16)), dim3(256), 0, s, (const float*)cents,
@@ -3025,10 +3052,11 @@ __global__ __launch_bounds__(256) void pqb_pp_round_w(const PqSub* __restrict__ 
   }
 }
 
+template <int PER>
 __global__ __launch_bounds__(1024) void pqb_pp_pick(const PqSub* __restrict__ S, int n, int nb, int chosen) {
   const PqSub& q = S[blockIdx.x];
-  km_pp_pick_body(q.P, q.w, n, q.w, q.ns, q.ps, q.pe, nb, q.rng, q.cents + (size_t)chosen * q.w, q.flags,
-                  q.flags + 1, nullptr);
+  km_pp_pick_body<PER>(q.P, q.w, n, q.w, q.ns, q.ps, q.pe, nb, q.rng, q.cents + (size_t)chosen * q.w, q.flags,
+                       q.flags + 1, nullptr);
 }
 
 // The certified matrix-core assignment of every subspace at once: the
@@ -3315,7 +3343,10 @@ static int pq_train_batched(const std::vector<DevBuf<float>>& proj, size_t n, co
   hipLaunchKernelGGL(pqb_first, dim3(M), dim3(64), 0, s, (const PqSub*)dS.p, (const uint64_t*)dfirst.p);
   round(0, 1);
   for (size_t chosen = 1; chosen < k; ++chosen) {
-    hipLaunchKernelGGL(pqb_pp_pick, dim3(M), dim3(1024), 0, s, (const PqSub*)dS.p, (int)n, nb, (int)chosen);
+    with_pick(nb, [&](auto per) {
+      hipLaunchKernelGGL(pqb_pp_pick<decltype(per)::value>, dim3(M), dim3(1024), 0, s, (const PqSub*)dS.p, (int)n, nb,
+                         (int)chosen);
+    });
     if (chosen + 1 < k) round((int)chosen, 0);
   }
   PXG_HIP(hipGetLastError());

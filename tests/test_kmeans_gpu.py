@@ -183,6 +183,16 @@ def test_kmeans_pp_parallel_sums_above_2_17_points(gpu):
     assert np.array_equal(bits(px.kmeans_pp(pts, 24, 77)), bits(orc.kmeans_pp(pts, 24, 77)))
 
 
+@pytest.mark.parametrize("blocks", [1024, 1025, 3072, 3073, 8192, 8193])
+def test_kmeans_pp_pick_partials_per_thread(gpu, blocks):
+    """One, up to three, up to eight and more block partials for each of the
+    pick's 1024 threads, at both ends of each form: the last block holds one
+    point. The grid makes the parallel sums exact."""
+    rng = np.random.default_rng(blocks)
+    pts = (rng.integers(0, 16, ((blocks - 1) * 256 + 1, 4)) / 4).astype(np.float32)
+    assert np.array_equal(bits(gpu.kmeans_pp(pts, 16, 9)), bits(orc.kmeans_pp(pts, 16, 9)))
+
+
 def test_kmeans_pp_sequential_sums_when_not_provably_exact(gpu):
     """Near-duplicate points at scale 1000: distances from ~1e-5 to ~1e7, so
     an f64 sum of them rounds and only the sequential order reproduces it."""
