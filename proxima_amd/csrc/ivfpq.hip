@@ -244,6 +244,12 @@ __device__ __attribute__((noinline)) void ivf_table(lds_float* lut, lds_float* s
 // code word at a time -> these); 300 L2 queries of 64 one-wide subspaces, 8
 // probes, shortlist 300: 566 us with the residual staged and one workgroup per
 // CU left, 288 before it was staged.
+// Long lists wait for one load after another: an entry's slot is loaded with
+// its codes, and these up to eight words together. 975k x 144, 24 subspaces, 86
+// lists, 8 L2 queries of 8 probes, shortlist 100: 519 us with the slot behind
+// the distance and four code words together, 403 with the slot ahead, 340 with
+// the words too. Ranks loaded ahead as well lose (1000 queries of 16 probes
+// over 512 lists, 8 x 6: 369 -> 483 us): few entries need theirs.
 template <int CAPW, int METRIC>
 __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, int ld, int dim, int M,
                                                 const int* __restrict__ probes, int nprobe, int pg, int groups,
@@ -296,6 +302,7 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
       const uint32_t e = e0 + lane;
       uint64_t key = KEY_MAX;
       if (e < end) {
+        const uint32_t sl = list_slot[e];  // in flight with the codes
         const uint8_t* code = list_codes + (size_t)e * M;
         float sum = 0.0f;  // DistanceTable::squared_l2 / inner_product, product.rs:580-603
         if (M == 16) {
@@ -304,20 +311,38 @@ __global__ __launch_bounds__(256) void ivf_scan(const float* __restrict__ Qp, in
 #pragma unroll
           for (int s = 0; s < 16; ++s) sum += lut[s * 256 + ((wv[s >> 2] >> (8 * (s & 3))) & 255)];
         } else if ((M & 3) == 0) {
-#pragma unroll 4
-          for (int s = 0; s < M; s += 4) {
-            const uint32_t cw = *reinterpret_cast<const uint32_t*>(code + s);
-            sum += lut[s * 256 + (cw & 255)];
-            sum += lut[s * 256 + 256 + ((cw >> 8) & 255)];
-            sum += lut[s * 256 + 512 + ((cw >> 16) & 255)];
-            sum += lut[s * 256 + 768 + (cw >> 24)];
+          // up to eight code words in flight together
+          auto words = [&](int s, auto n) {
+            uint32_t cw[n];
+#pragma unroll
+            for (int u = 0; u < n; ++u) cw[u] = *reinterpret_cast<const uint32_t*>(code + s + 4 * u);
+#pragma unroll
+            for (int u = 0; u < n; ++u) {
+              const float* t = lut + (s + 4 * u) * 256;
+              sum += t[cw[u] & 255];
+              sum += t[256 + ((cw[u] >> 8) & 255)];
+              sum += t[512 + ((cw[u] >> 16) & 255)];
+              sum += t[768 + (cw[u] >> 24)];
+            }
+          };
+          int s = 0;
+          for (; s + 32 <= M; s += 32) words(s, std::integral_constant<int, 8>{});
+          switch ((M - s) >> 2) {
+            case 1: words(s, std::integral_constant<int, 1>{}); break;
+            case 2: words(s, std::integral_constant<int, 2>{}); break;
+            case 3: words(s, std::integral_constant<int, 3>{}); break;
+            case 4: words(s, std::integral_constant<int, 4>{}); break;
+            case 5: words(s, std::integral_constant<int, 5>{}); break;
+            case 6: words(s, std::integral_constant<int, 6>{}); break;
+            case 7: words(s, std::integral_constant<int, 7>{}); break;
+            default: break;
           }
         } else {
           for (int s = 0; s < M; ++s) sum += lut[s * 256 + code[s]];
         }
         const uint32_t dk = ord_key(METRIC == 0 ? sum : ivf_cos_score(one_minus_qdc, sum));
+        asm volatile("" ::"v"(sl));  // keeps the load above from sinking into the branch
         if (dk <= (uint32_t)(thr >> 32)) {
-          const uint32_t sl = list_slot[e];
           if (accept == nullptr || accept[sl]) key = ((uint64_t)dk << 32) | slot_rank[sl];
         }
       }

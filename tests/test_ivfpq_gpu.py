@@ -683,3 +683,25 @@ def test_general_scan_tables(gpu, metric, dim, m, shortlist):
     want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), orc.prepare_rows(metric, q), shortlist, 3,
                           m, threads=8)
     assert_same(idx.search_batch(q, shortlist, nprobe=3), want)
+
+
+@pytest.mark.parametrize("metric", [0, 1])
+@pytest.mark.parametrize("m", [4, 8, 12, 20, 24, 28, 32, 36, 40, 64, 68])
+def test_general_scan_code_words(gpu, metric, m):
+    """Every number of code words that the general scan takes together: one to
+    eight, and what is left beyond eight; with a filter and without."""
+    px = gpu
+    n, nlist, dim = 1500, 3, 3 * m
+    data = corpus(n, dim, 12) + np.random.default_rng(m).standard_normal((n, dim)).astype(np.float32) * 0.2
+    prep = orc.prepare_rows(metric, data)
+    cents, books, _ = orc.ivf_train(prep, nlist, m, max_iter=1, seed=1)
+    codes, list_of = orc.ivf_encode(prep, cents, books, m)
+    idx = build(px, data, px.IvfPqConfig(nlist, m).with_train_threshold(1 << 62), metric)
+    idx.load_trained(cents, books, codes, list_of)
+    q = data[::150] + np.float32(0.01)
+    qp = orc.prepare_rows(metric, q)
+    want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), qp, 100, 2, m, threads=8)
+    assert_same(idx.search_batch(q, 100, nprobe=2), want)
+    accept = np.arange(n) % 3 != 1
+    want = orc.ivf_search(metric, cents, books, codes, list_of, np.arange(n), qp, 100, 2, m, threads=8, accept=accept)
+    assert_same(idx.search_batch(q, 100, lambda i, _m: bool(accept[i]), nprobe=2), want)
