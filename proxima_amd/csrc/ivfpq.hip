@@ -2768,9 +2768,23 @@ struct IvfPqIndex {
                                            s, ldo);
         scanned_dev = nullptr;
       } else {
-      // probes per workgroup as on the register path
-      int pg = IVF_PGMAX;
-      while (pg > 1 && (int64_t)nq * ((np + pg - 1) / pg) < 512) pg >>= 1;
+      // Probes per workgroup: the fewest rounds of one workgroup per CU, a
+      // workgroup's own cost (its lists' sorts and its share of the merge)
+      // counted as one probe more, among those that leave 512 workgroups (or
+      // one probe each). 300 queries of 16 probes over 128 lists of 4700, 12 x 6
+      // dimensions: groups of 8 (600 workgroups, 3 on some CUs and 2 on others)
+      // 566 us, of 4 407; 1000 queries over 512 lists, 8 x 6: of 16 351, of 8
+      // 419; 100 queries over 1024 lists, 12 x 8: of 2 111, of 1 115.
+      int pg = 1;
+      int64_t least = INT64_MAX;
+      for (int g = IVF_PGMAX; g >= 1; g >>= 1) {
+        const int64_t wgs = (int64_t)nq * ((np + g - 1) / g);
+        const int64_t cost = (wgs + 255) / 256 * (g + 1);
+        if ((wgs >= 512 || g == 1) && cost < least) {
+          least = cost;
+          pg = g;
+        }
+      }
       const int groups = (np + pg - 1) / pg;
       const size_t table = (size_t)M() * 256 * 4;
       // the query (or residual) is staged beside the table where that takes at
